@@ -139,7 +139,7 @@ def test_bench_refuses_more_than_one_gpu():
 REF_ROOT = "/root/reference"
 
 
-@pytest.mark.skipif(not os.path.isdir(REF_ROOT), reason="reference sources not present")
+@pytest.mark.skipif(not os.path.isfile(os.path.join(REF_ROOT, "qwen_tts.h")), reason="reference sources not present")
 def test_glue_compiles_against_reference_header():
     """The reference-side glue (qwen3-tts_amd/glue) is real C against the reference's own
     qwen_tts.h: it compiles warning-free with the reference's flags."""
