@@ -496,7 +496,6 @@ static int ps_setup(talker_t *t) {
     HCK(hipMalloc((void **)&t->ps_epoch, 64));
     HCK(hipMalloc((void **)&t->ps_err, 64));
     HCK(hipMalloc((void **)&t->ps_xin, (size_t)s->H * sizeof(float)));
-    HCK(hipHostMalloc((void **)&t->h_err, 64, hipHostMallocDefault));
     HCK(hipMemsetAsync(t->ps_ring, 0, (t->rs_on ? 1 : words) * sizeof(unsigned long long), t->st));
     HCK(hipMemsetAsync(t->ps_err, 0, 64, t->st));
     HCK(hipMemcpyAsync(t->ps_epoch, &one, sizeof one, hipMemcpyHostToDevice, t->st));
@@ -652,6 +651,8 @@ void *qwen_hip_talker_init(const qwen_hip_talker_desc_t *desc) {
     HCK(hipHostMalloc((void **)&t->h_in, (size_t)H * sizeof(float), hipHostMallocDefault));
     HCK(hipHostMalloc((void **)&t->h_out, (size_t)2 * H * sizeof(float), hipHostMallocDefault));
     HCK(hipHostMalloc((void **)&t->h_pos, 4 * sizeof(int), hipHostMallocDefault));
+    /* [0] the fused step's error flag, [1] the fused CP frame's (a frame loop may use only the latter) */
+    HCK(hipHostMalloc((void **)&t->h_err, 64, hipHostMallocDefault));
     HCK(hipMemsetAsync(t->io, 0, (size_t)2 * H * sizeof(float), t->st));
     HCK(hipStreamSynchronize(t->st));
     t->dev_pos = -1;
