@@ -5,9 +5,9 @@
 // a convolutional upsampler (ConvNeXt x2, then four blocks of transposed conv + dilated
 // residual units) to 1920 samples per frame.  All of it is f32.  Here every activation is
 // kept time-major ([T][C], channels contiguous), and every projection, convolution and
-// transposed convolution is one implicit GEMM on the f32 matrix cores:
+// transposed convolution is one implicit GEMM:
 //
-//   Y[t*os + z][n] = epi( sum over taps p, channels k of X[t + off_p][k] * W[z][p][k][n] )
+//   Y[t*os + z][n] = epi( sum over channels k, taps p of X[t + off_p][k] * W[z][p][k][n] )
 //
 // (rows of X outside [xlo, Tx) read as zero: the causal left padding; the streaming decode
 // keeps the previous chunk's last rows at negative indices, xlo < 0).  A causal conv of
@@ -17,23 +17,93 @@
 // applies GELU, scales per column (layer scale, ConvNeXt gamma), adds a residual and
 // applies the snake activation that the next layer needs on its input (so no separate
 // pass over the activation: the upsampler's snakes all live in the producing GEMM).
-// Products accumulate in f32 in MFMA order (the reference sums in loop order): the
-// results agree to f32 rounding, not bitwise.
-#include "qt_device.h"
-
-typedef float qt_sd_f4 __attribute__((ext_vector_type(4)));
+//
+// The products run on the bf16 matrix cores, sixteen times as fast as the f32 ones: each f32
+// operand is the exact sum of three bf16 planes, a product of two planes is exact in f32,
+// and the six largest of the nine plane products of an f32 product are accumulated in f32
+// (the rest are under 2^-25 of it, below its own rounding).  The weights' planes are made
+// once, when the decoder is loaded; an input's on its way into LDS.
+#include "qt_attn_mf.h"
 
 #define SD_WG 256
-#define SD_KC 16                 // K chunk staged per step (the 16- and 32-row tiles stage 64 where K allows)
 #define SD_MAXTAP 8
+#define SD_HALO 54               // staged rows before a tile's own: a 7-tap conv of dilation 9
 
 enum { SD_EPI_BIAS = 1, SD_EPI_GELU = 2, SD_EPI_CSCALE = 4, SD_EPI_RESID = 8, SD_EPI_SNAKE = 16, SD_EPI_SNAKE2 = 32 };
 
+// ---- the GEMM's weights: three bf16 planes in the matrix core's order ----------------------
+// v_mfma_f32_16x16x32_bf16 takes A = 16 output channels x 32 k and B = 32 k x 16 output rows;
+// lane l supplies 8 consecutive k (group l / 16) of channel (row) l % 16 and receives
+// D[channel 4 (l / 16) + r][row l % 16], r < 4.  A weight tile of 16 channels x 32 k is
+// stored as its three planes, 64 lanes x 16 bytes each (3 KiB), in the order that a
+// workgroup walks: [K slice][tap][phase][channel tile].  K and the channels of a phase are
+// padded with zeros to 32 and 16.
+// An f32 value v is the sum of its planes exactly: v rounded to bf16, the rest rounded to
+// bf16, and what then remains (at most 8 significant bits).
+__device__ __forceinline__ uint32_t sd_bf16x2(float a, float b) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{a, b}), b2));
+}
+__device__ __forceinline__ float sd_lo(uint32_t u) { return __uint_as_float(u << 16); }
+__device__ __forceinline__ float sd_hi(uint32_t u) { return __uint_as_float(u & 0xFFFF0000u); }
+
+// the planes of 8 values; chk becomes NaN when a value has none (infinite, NaN, or past
+// bf16's range after rounding) and stays as it is otherwise
+__device__ __forceinline__ void sd_planes8(const float (&v)[8], qt_u32x4 (&p)[3], float &chk) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float a = v[2 * i], b = v[2 * i + 1];
+        const uint32_t h = sd_bf16x2(a, b);
+        const float ra = a - sd_lo(h), rb = b - sd_hi(h);
+        const uint32_t m = sd_bf16x2(ra, rb);
+        chk = fmaf(ra, 0.f, fmaf(rb, 0.f, chk));
+        p[0][i] = h;
+        p[1][i] = m;
+        p[2][i] = sd_bf16x2(ra - sd_lo(m), rb - sd_hi(m));
+    }
+}
+
+// One tensor of the reference's layout (element [n][k][column] at n * sn + k * sk + column * sc)
+// into channels [n0, n0 + nn) and k [k0, k0 + kk) of the packed weights (n0, k0: whole tiles).
+// Tap p of phase z is column p (stride 0: a conv or linear layer) or z + p * stride (zero past the
+// kernel's columns).  A value without planes (infinite, NaN or too large) sets *bad.
+struct SdPackArgs {
+    const float *src;
+    long long sn, sk, sc;
+    int cols, stride, ntap, phases, tiles;         // tiles: channel tiles of a phase
+    int n0, nn, k0, kk;
+    uint16_t *dst;
+    int *bad;
+};
+__global__ __launch_bounds__(SD_WG) void k_sd_pack(SdPackArgs a) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nt = (a.nn + 15) / 16;
+    const int t = blockIdx.x * QT_WAVES + wave, z = blockIdx.z;
+    const int kc = t / (a.ntap * nt), r = t - kc * a.ntap * nt, p = r / nt, j = r - p * nt;
+    if (kc >= (a.kk + 31) / 32) return;
+    const int n = 16 * j + (lane & 15), k = 32 * kc + 8 * (lane >> 4), col = a.stride ? z + p * a.stride : p;
+    float v[8], chk = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        v[i] = (n < a.nn && k + i < a.kk && col < a.cols) ? a.src[n * a.sn + (k + i) * a.sk + col * a.sc] : 0.f;
+    qt_u32x4 pl[3];
+    sd_planes8(v, pl, chk);
+    if (chk != chk) *a.bad = 1;
+    uint16_t *d = a.dst + ((((size_t)(a.k0 / 32 + kc) * a.ntap + p) * a.phases + z) * a.tiles + a.n0 / 16 + j) * 1536 + 8 * lane;
+#pragma unroll
+    for (int q = 0; q < 3; q++) *reinterpret_cast<qt_u32x4 *>(d + 512 * q) = pl[q];
+}
+
 struct SdGemmArgs {
     const float *X; int ldx, Tx, xlo;     // input rows [xlo, Tx) of a [.][ldx] buffer (xlo <= 0: history rows)
-    const float *W;                       // [phases][ntap][K][N]
+    const uint16_t *W;                    // packed planes
     int K, N, ntap;
+    int slices, tiles, phases;            // K slices of 32; channel tiles of a phase
     int off[SD_MAXTAP];
+    int omin, span;                       // smallest offset; largest minus smallest
+    int tps;                              // taps that share a staged slice (ntap, or 1 where span is too long)
+    int serial;                           // weights without planes: every output by sd_serial
     int T;                                // output rows per phase (t < T)
     float *Y; int ldy, os;                // output row t*os + phase
     const float *bias, *cscale;
@@ -53,155 +123,276 @@ __device__ __forceinline__ float sd_snake(float x, float a, float ib) {
     return fmaf(ib, s * s, x);
 }
 
-// TM x TN output tile (16, 32 or 64 x 64, or 128 x 128), four waves of a 2 x 2 grid (a
-// 1 x 4 grid for TM = 16), each a grid of 16 x 16 MFMA tiles; K in chunks of KC (16, or
-// 64 for the small tiles where K allows) staged through LDS (two buffers).  The global
-// loads of the next P chunks sit in a ring of P register slots: a chunk's loads are
-// issued P - 1 chunks before it is staged, which hides HBM latency when only a few
-// workgroups share a CU (a streaming chunk of a few frames gives the long-K convolutions
-// a few dozen tiles).  The fetch index is clamped to the last chunk rather than guarded,
-// so the loads are straight-line code and the compiler counts them exactly.  Every
-// output element sums its products four k at a time in ascending k, one MFMA after
-// another, whatever TM, TN, P and KC are, so every tile gives the same bits.
-// The 128 x 128 tile reads each A and B value from LDS once per four MFMAs (twice as
-// many as the 64 x 64 tile's two).
-// v_mfma_f32_16x16x4_f32: lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16] and
-// receives D[4 (l / 16) + r][l % 16], r < 4.
-template <int TM, int TN, int P, int KC>
-__global__ __launch_bounds__(SD_WG) void k_sd_gemm(SdGemmArgs a) {
-    static_assert(P >= 2 && P % 2 == 0, "chunk c sits in LDS buffer c & 1 == slot & 1");
-    static_assert(KC == 16 || KC == 64, "K chunk");
-    // A chunk is TM x KC floats = TM * KC / 4 float4s; where that is fewer than the 256
-    // threads (16 or 32 rows at KC = 16) the spare waves load a copy of the same rows
-    // (same addresses, nothing staged)
-    constexpr int AF4 = TM * KC / 4, AQ = AF4 >= SD_WG ? AF4 / SD_WG : 1;   // A float4 loads per thread
-    constexpr int BQ = KC * TN / (4 * SD_WG);                               // B float4 loads per thread
-    constexpr int AS = KC + (KC == 16 ? 1 : 17);   // A row stride = 17 mod 32 floats: 16 rows spread over banks
-    constexpr int WMW = TM >= 32 ? 2 : 1, WNW = 4 / WMW;     // wave grid: WMW along M, WNW along N
-    constexpr int BS = TN + 16;                        // B row stride: rows k, k+1 on opposite bank halves
-    constexpr int MI = TM / (16 * WMW), NJ = TN / (16 * WNW);   // 16 x 16 MFMA tiles per wave
-    static_assert(MI >= 1 && NJ >= 1 && TN % 64 == 0 && BQ >= 1, "tile shape");
-    __shared__ float As[2][TM * AS];
-    __shared__ float Bs[2][KC * BS];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int t0 = blockIdx.x * TM, n0 = blockIdx.y * TN, z = blockIdx.z;
-    const float *W = a.W + (size_t)z * a.ntap * a.K * a.N;
-    const int kpt = a.K / KC, nch = a.ntap * kpt;
-    // ring slots hold the loads as issued (clamped rows and columns); which of them are
-    // real (am: bit q of the slot's A loads, bok: B columns inside N) is applied when a
-    // slot is staged, so the loads have no use before then and nothing branches around them
-    float4 av[P][AQ], bv[P][BQ];
-    unsigned amk[P];
-    unsigned bok = 0;
-#pragma unroll
-    for (int q = 0; q < BQ; q++) bok |= (n0 + ((tid + q * SD_WG) % (TN / 4)) * 4 < a.N) ? 1u << q : 0u;
-    auto fetch = [&](int c, float4 (&ra)[AQ], float4 (&rb)[BQ], unsigned &am) {
-        const int p = c / kpt, k0 = (c - p * kpt) * KC;
-#pragma unroll
-        for (int q = 0; q < AQ; q++) {
-            const int f = tid + q * SD_WG, ar = (f / (KC / 4)) % TM, ac = (f % (KC / 4)) * 4;
-            const int xr = t0 + ar + a.off[p];
-            const bool ok = t0 + ar < a.T && xr >= a.xlo && xr < a.Tx;
-            const int xc = min(max(xr, a.xlo), a.Tx - 1);   // in bounds; the value is dropped when !ok
-            ra[q] = *reinterpret_cast<const float4 *>(a.X + (ptrdiff_t)xc * a.ldx + k0 + ac);
-            am = ok ? am | (1u << q) : am & ~(1u << q);
-        }
-#pragma unroll
-        for (int q = 0; q < BQ; q++) {
-            const int f = tid + q * SD_WG, br = f / (TN / 4), bc = (f % (TN / 4)) * 4;
-            const int nc = min(n0 + bc, a.N - 4);
-            rb[q] = *reinterpret_cast<const float4 *>(W + ((size_t)p * a.K + k0 + br) * a.N + nc);
-        }
-    };
-    auto stage = [&](int buf, const float4 (&ra)[AQ], const float4 (&rb)[BQ], unsigned am) {
-        // masks on the bits, value by value (a select of whole float4s becomes a select of
-        // their addresses, which moves the ring to scratch)
-#pragma unroll
-        for (int q = 0; q < AQ; q++) {
-            const int f = tid + q * SD_WG, ar = f / (KC / 4), ac = (f % (KC / 4)) * 4;
-            if (AF4 < SD_WG && f >= AF4) continue;    // the copies (whole waves)
-            const unsigned m = 0u - ((am >> q) & 1u);
-            float *as = As[buf] + ar * AS + ac;
-            as[0] = __uint_as_float(__float_as_uint(ra[q].x) & m);
-            as[1] = __uint_as_float(__float_as_uint(ra[q].y) & m);
-            as[2] = __uint_as_float(__float_as_uint(ra[q].z) & m);
-            as[3] = __uint_as_float(__float_as_uint(ra[q].w) & m);
-        }
-#pragma unroll
-        for (int q = 0; q < BQ; q++) {
-            const int f = tid + q * SD_WG, br = f / (TN / 4), bc = (f % (TN / 4)) * 4;
-            const unsigned m = 0u - ((bok >> q) & 1u);
-            *reinterpret_cast<float4 *>(Bs[buf] + br * BS + bc) =
-                make_float4(__uint_as_float(__float_as_uint(rb[q].x) & m), __uint_as_float(__float_as_uint(rb[q].y) & m),
-                            __uint_as_float(__float_as_uint(rb[q].z) & m), __uint_as_float(__float_as_uint(rb[q].w) & m));
-        }
-    };
-    const int wm = (wave / WNW) * (TM / WMW), wn = (wave % WNW) * (TN / WNW);
-    const int li = lane & 15, lk = lane >> 4;
-    qt_sd_f4 acc[MI][NJ];
-#pragma unroll
-    for (int i = 0; i < MI; i++)
-#pragma unroll
-        for (int j = 0; j < NJ; j++) acc[i][j] = qt_sd_f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < P; s++) fetch(min(s, nch - 1), av[s], bv[s], amk[s]);
-    stage(0, av[0], bv[0], amk[0]);
-    __syncthreads();
-    for (int c0 = 0; c0 < nch; c0 += P) {
-#pragma unroll
-        for (int s = 0; s < P; s++) {
-            const int c = c0 + s;
-            // slot s held chunk c, staged one step ago: refill it with chunk c + P (loads
-            // issued on every path, so the waits before each stage count them exactly)
-            fetch(min(c + P, nch - 1), av[s], bv[s], amk[s]);
-            if (c < nch) {
-                const float *as = As[s & 1], *bs = Bs[s & 1];
-#pragma unroll
-                for (int kk = 0; kk < KC; kk += 4) {
-                    float fa[MI], fb[NJ];
-#pragma unroll
-                    for (int i = 0; i < MI; i++) fa[i] = as[(wm + 16 * i + li) * AS + kk + lk];
-#pragma unroll
-                    for (int j = 0; j < NJ; j++) fb[j] = bs[(kk + lk) * BS + wn + 16 * j + li];
-#pragma unroll
-                    for (int i = 0; i < MI; i++)
-#pragma unroll
-                        for (int j = 0; j < NJ; j++)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i], fb[j], acc[i][j], 0, 0, 0);
-                }
-                if (c + 1 < nch) stage((s & 1) ^ 1, av[(s + 1) % P], bv[(s + 1) % P], amk[(s + 1) % P]);
-                __syncthreads();
+// Channels n..n+3 of output row t, phase z, one product after the other in f32: what a tile
+// falls back to when an operand has no planes (an infinite or NaN input must reach the
+// outputs that it reaches in plain arithmetic, and only those).
+__device__ __forceinline__ qt_f32x4 sd_serial(const SdGemmArgs &a, int t, int tile, int n) {
+    qt_f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < a.ntap; p++) {
+        const int xr = t + a.off[p];
+        const bool ok = t < a.T && xr >= a.xlo && xr < a.Tx;
+        for (int k = 0; k < a.K; k++) {
+            const float x = ok ? a.X[(ptrdiff_t)xr * a.ldx + k] : 0.f;
+            const uint16_t *w = a.W + (((size_t)(k / 32) * a.ntap + p) * a.phases * a.tiles + tile) * 1536 +
+                                8 * ((n & 15) + 16 * ((k % 32) / 8)) + k % 8;
+            for (int r = 0; r < 4; r++) {
+                const float w0 = __uint_as_float((uint32_t)w[8 * r] << 16), w1 = __uint_as_float((uint32_t)w[8 * r + 512] << 16),
+                            w2 = __uint_as_float((uint32_t)w[8 * r + 1024] << 16);
+                s[r] = fmaf(x, (w0 - w0 == 0.f) ? w0 + (w1 + w2) : w0, s[r]);
             }
         }
     }
+    return s;
+}
+
+// The four channels n..n+3 (n: channel of the phase) of output row t: bias, GELU, column
+// scale, residual, snake.
+__device__ __forceinline__ void sd_epilogue(const SdGemmArgs &a, int t, int z, int n, qt_f32x4 v) {
+    if (t >= a.T || n >= a.N) return;
+    const size_t o = (size_t)(t * a.os + z) * a.ldy + n;
+    const auto ld = [](const float *p) { return *reinterpret_cast<const qt_f32x4 *>(p); };
+    if (a.epi & SD_EPI_BIAS) v += ld(a.bias + n);
+    if (a.epi & SD_EPI_GELU)
 #pragma unroll
-    for (int i = 0; i < MI; i++)
+        for (int r = 0; r < 4; r++) v[r] = sd_gelu(v[r]);
+    if (a.epi & SD_EPI_CSCALE) v *= ld(a.cscale + n);
+    if (a.epi & SD_EPI_RESID) v = ld(a.R + o) + v;
+    if (a.epi & (SD_EPI_SNAKE | SD_EPI_SNAKE2)) {
+        const qt_f32x4 pa = ld(a.sa + n), pb = ld(a.sib + n);
+        qt_f32x4 s;
 #pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            const int n = n0 + wn + 16 * j + li;
-            if (n >= a.N) continue;
-            const float bn = (a.epi & SD_EPI_BIAS) ? a.bias[n] : 0.f;
-            const float sn = (a.epi & SD_EPI_CSCALE) ? a.cscale[n] : 1.f;
-            const float pa = (a.epi & (SD_EPI_SNAKE | SD_EPI_SNAKE2)) ? a.sa[n] : 0.f;
-            const float pb = (a.epi & (SD_EPI_SNAKE | SD_EPI_SNAKE2)) ? a.sib[n] : 0.f;
+        for (int r = 0; r < 4; r++) s[r] = sd_snake(v[r], pa[r], pb[r]);
+        if (a.epi & SD_EPI_SNAKE2) *reinterpret_cast<qt_f32x4 *>(a.Y2 + o) = s;
+        else v = s;
+    }
+    *reinterpret_cast<qt_f32x4 *>(a.Y + o) = v;
+}
+
+// The six plane products that an f32 product needs (the other three are below 2^-25 of it),
+// the smallest first.
+__device__ __forceinline__ qt_f32x4 sd_mma6(const qt_u32x4 (&w)[3], const qt_u32x4 (&x)[3], qt_f32x4 c) {
+    c = qt_mfma_bf16(w[0], x[2], c);
+    c = qt_mfma_bf16(w[2], x[0], c);
+    c = qt_mfma_bf16(w[1], x[1], c);
+    c = qt_mfma_bf16(w[0], x[1], c);
+    c = qt_mfma_bf16(w[1], x[0], c);
+    return qt_mfma_bf16(w[0], x[0], c);
+}
+
+// Where a layer has at least SD_GROUP_SLICES slices of 32 k (512), its slices are SD_GROUPS
+// equal runs whose sums are added in order.  That is a property of the layer alone, so a
+// small call can give the runs to different waves and still return the bits of a large one.
+#define SD_GROUPS 8
+#define SD_GROUP_SLICES 16
+
+// swizzle of the 16-byte unit kg of an LDS row of 32 k: 8 (and 16) consecutive rows read one
+// unit each from different banks
+__device__ __forceinline__ int sd_unit(int row, int kg) { return 16 * (kg ^ (((row >> 2) & 3) ^ (row & 2))); }
+
+// ---- tiles for many rows ---------------------------------------------------------------------
+// A workgroup of WN x WT waves computes 16 NT WN channels x 16 MT WT rows.  A slice of 32 k of
+// the rows that all its taps read (the tile's rows and the taps' span before them) is
+// loaded once, split into planes on the way into LDS, and every tap runs from there, so a
+// 7-tap conv stages each input once; the weights' planes come straight from L2 in operand
+// order, one (slice, tap) ahead.  Two LDS buffers, one barrier per slice.
+template <int WN, int NT, int WT, int MT, bool GRP>
+__global__ __launch_bounds__(SD_WG) __attribute__((amdgpu_waves_per_eu(2))) void k_sd_tile(SdGemmArgs a) {
+    static_assert(WN * WT == QT_WAVES, "four waves");
+    constexpr int TT = 16 * MT * WT, RM = TT + SD_HALO, PS = RM * 64, BUF = 3 * PS, NU = (RM * 4 + SD_WG - 1) / SD_WG;
+    __shared__ __align__(16) uint8_t xs[2 * BUF];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, kg = lane >> 4;
+    const int t0 = blockIdx.x * TT, all = a.phases * a.tiles;
+    const int j0 = (blockIdx.y * WN + wave % WN) * NT, tw = 16 * MT * (wave / WN);
+    const int rows = TT + (a.tps > 1 ? a.span : 0), ns = a.slices * (a.ntap / a.tps);
+    float chk = 0.f;
+    float st[NU][8];
+    unsigned ok = 0;
+    auto fetch = [&](int s) {
+        const int per = a.ntap / a.tps, kc = s / per, o = a.tps > 1 ? a.omin : a.off[s - kc * per];
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int t = t0 + wm + 16 * i + 4 * lk + r;
-                if (t >= a.T) continue;
-                const size_t o = (size_t)(t * a.os + z) * a.ldy + n;
-                float v = acc[i][j][r];
-                if (a.epi & SD_EPI_BIAS) v += bn;
-                if (a.epi & SD_EPI_GELU) v = sd_gelu(v);
-                if (a.epi & SD_EPI_CSCALE) v *= sn;
-                if (a.epi & SD_EPI_RESID) v = a.R[o] + v;
-                if (a.epi & SD_EPI_SNAKE2) {
-                    a.Y[o] = v;
-                    a.Y2[o] = sd_snake(v, pa, pb);
-                } else {
-                    a.Y[o] = (a.epi & SD_EPI_SNAKE) ? sd_snake(v, pa, pb) : v;
-                }
+        for (int i = 0; i < NU; i++) {
+            const int u = tid + i * SD_WG, row = u >> 2, k = 32 * kc + 8 * (u & 3), xr = t0 + row + o;
+            const bool in = row < rows && xr >= a.xlo && xr < a.Tx && k < a.K;
+            ok = in ? ok | (1u << i) : ok & ~(1u << i);
+            // in bounds either way; the value is dropped when !in
+            const float *src = a.X + (ptrdiff_t)min(max(xr, a.xlo), a.Tx - 1) * a.ldx + min(k, a.K - 8);
+            const float4 p = *reinterpret_cast<const float4 *>(src), q = *reinterpret_cast<const float4 *>(src + 4);
+            st[i][0] = p.x; st[i][1] = p.y; st[i][2] = p.z; st[i][3] = p.w;
+            st[i][4] = q.x; st[i][5] = q.y; st[i][6] = q.z; st[i][7] = q.w;
+        }
+    };
+    auto put = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < NU; i++) {
+            const int u = tid + i * SD_WG, row = u >> 2;
+            if ((i + 1) * SD_WG > RM * 4 && row >= RM) continue;
+            const unsigned m = 0u - ((ok >> i) & 1u);
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] = __uint_as_float(__float_as_uint(st[i][e]) & m);
+            qt_u32x4 pl[3];
+            sd_planes8(v, pl, chk);
+            uint8_t *d = xs + buf * BUF + row * 64 + sd_unit(row, u & 3);
+#pragma unroll
+            for (int p = 0; p < 3; p++) *reinterpret_cast<qt_u32x4 *>(d + p * PS) = pl[p];
+        }
+    };
+    const uint16_t *wp[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) wp[j] = a.W + (size_t)min(j0 + j, all - 1) * 1536 + 8 * lane;
+    const size_t step = (size_t)all * 1536;
+    const int items = a.slices * a.ntap;
+    qt_u32x4 w[NT][3], wn[NT][3];
+    auto weights = [&](int it, qt_u32x4 (&d)[NT][3]) {
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int p = 0; p < 3; p++) d[j][p] = *reinterpret_cast<const qt_u32x4 *>(wp[j] + it * step + 512 * p);
+    };
+    qt_f32x4 acc[NT][MT], tot[GRP ? NT : 1][GRP ? MT : 1];
+    const qt_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++) acc[j][i] = zero;
+    fetch(0);
+    weights(0, w);
+    put(0);
+    __syncthreads();
+    int g = 0;
+    for (int s = 0, it = 0; s < ns; s++) {
+        if (s + 1 < ns) fetch(s + 1);
+        const uint8_t *b = xs + (s & 1) * BUF;
+        for (int p = 0; p < a.tps; p++, it++) {
+            weights(min(it + 1, items - 1), wn);
+            const int row = tw + li + (a.tps > 1 ? a.off[p] - a.omin : 0);
+            const uint8_t *x0 = b + row * 64 + sd_unit(row, kg);
+#pragma unroll
+            for (int i = 0; i < MT; i++) {
+                qt_u32x4 x[3];
+#pragma unroll
+                for (int q = 0; q < 3; q++) x[q] = qt_lds16(x0 + i * 1024 + q * PS);
+#pragma unroll
+                for (int j = 0; j < NT; j++) acc[j][i] = sd_mma6(w[j], x, acc[j][i]);
+            }
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+#pragma unroll
+                for (int q = 0; q < 3; q++) w[j][q] = wn[j][q];
+        }
+        if constexpr (GRP) {
+            if (it == (a.slices * (g + 1) / SD_GROUPS) * a.ntap) {   // a run ends here
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int i = 0; i < MT; i++) {
+                        tot[j][i] = g ? tot[j][i] + acc[j][i] : acc[j][i];
+                        acc[j][i] = zero;
+                    }
+                g++;
             }
         }
+        if (s + 1 < ns) put((s + 1) & 1);
+        __syncthreads();
+    }
+    const bool serial = __syncthreads_or(chk != chk || a.serial);
+    // the sums through LDS, so that a row's channels go out (and its residual comes in) together
+    constexpr int TN = 16 * WN * NT, LD = TN + 4;
+    static_assert(TT * LD * 4 <= 2 * BUF, "the tile's sums fit in the staging buffers");
+    float *ys = reinterpret_cast<float *>(xs);
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+            *reinterpret_cast<qt_f32x4 *>(ys + (tw + 16 * i + li) * LD + 16 * (wave % WN * NT + j) + 4 * kg) =
+                GRP ? tot[GRP ? j : 0][GRP ? i : 0] : acc[j][i];
+    __syncthreads();
+    for (int e = tid; e < TT * TN / 4; e += SD_WG) {
+        const int row = e / (TN / 4), c = 4 * (e % (TN / 4)), t = t0 + row, tile = blockIdx.y * (WN * NT) + c / 16;
+        if (tile >= all || t >= a.T) continue;
+        const int z = tile / a.tiles, n = 16 * (tile - z * a.tiles) + c % 16;
+        sd_epilogue(a, t, z, n, serial ? sd_serial(a, t, tile, n) : *reinterpret_cast<qt_f32x4 *>(ys + row * LD + c));
+    }
+}
+
+// ---- few rows ---------------------------------------------------------------------------------
+// A workgroup of eight waves computes 16 NT channels x 16 MT rows; wave g takes the layer's g-th
+// run of slices, with its operands straight from memory (no staging, no barrier until the
+// runs' sums meet in LDS), D (slice, tap) pairs in flight.  A call of a few frames leaves the
+// long-K layers with a few dozen such tiles: the time is the latency of one run.
+template <int NT, int MT, int D>
+__global__ __launch_bounds__(64 * SD_GROUPS) void k_sd_split(SdGemmArgs a) {
+    __shared__ __align__(16) qt_f32x4 part[SD_GROUPS][NT * MT][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, kg = lane >> 4;
+    const int t0 = blockIdx.x * 16 * MT, all = a.phases * a.tiles, j0 = blockIdx.y * NT;
+    const int i0 = (a.slices * wave / SD_GROUPS) * a.ntap, i1 = (a.slices * (wave + 1) / SD_GROUPS) * a.ntap;
+    const size_t step = (size_t)all * 1536;
+    const uint16_t *wp[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) wp[j] = a.W + (size_t)min(j0 + j, all - 1) * 1536 + 8 * lane;
+    qt_u32x4 w[D][NT][3];
+    float4 xa[D][MT], xb[D][MT];
+    unsigned ok[D];
+    float chk = 0.f;
+    auto fetch = [&](int it, int d) {
+        const int kc = it / a.ntap, p = it - kc * a.ntap, k = 32 * kc + 8 * kg, o = a.off[p];
+        unsigned m = 0;
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            const int xr = t0 + 16 * i + li + o;
+            if (xr >= a.xlo && xr < a.Tx && k < a.K) m |= 1u << i;
+            const float *src = a.X + (ptrdiff_t)min(max(xr, a.xlo), a.Tx - 1) * a.ldx + min(k, a.K - 8);
+            xa[d][i] = *reinterpret_cast<const float4 *>(src);
+            xb[d][i] = *reinterpret_cast<const float4 *>(src + 4);
+        }
+        ok[d] = m;
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int q = 0; q < 3; q++) w[d][j][q] = *reinterpret_cast<const qt_u32x4 *>(wp[j] + it * step + 512 * q);
+    };
+    qt_f32x4 acc[NT][MT];
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++) acc[j][i] = qt_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < D; d++) fetch(min(i0 + d, i1 - 1), d);
+    for (int it = i0; it < i1; it += D) {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            if (it + d < i1) {
+#pragma unroll
+                for (int i = 0; i < MT; i++) {
+                    const unsigned m = 0u - ((ok[d] >> i) & 1u);
+                    const float4 p = xa[d][i], q = xb[d][i];
+                    float v[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
+#pragma unroll
+                    for (int e = 0; e < 8; e++) v[e] = __uint_as_float(__float_as_uint(v[e]) & m);
+                    qt_u32x4 pl[3];
+                    sd_planes8(v, pl, chk);
+#pragma unroll
+                    for (int j = 0; j < NT; j++) acc[j][i] = sd_mma6(w[d][j], pl, acc[j][i]);
+                }
+            }
+            fetch(min(it + d + D, i1 - 1), d);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++) part[wave][j * MT + i][lane] = acc[j][i];
+    const bool serial = __syncthreads_or(chk != chk || a.serial);
+    for (int c = wave; c < NT * MT; c += SD_GROUPS) {
+        const int j = c / MT, i = c - j * MT;
+        if (j0 + j >= all) continue;
+        const int z = (j0 + j) / a.tiles, n = 16 * (j0 + j - z * a.tiles) + 4 * kg, t = t0 + 16 * i + li;
+        qt_f32x4 v = part[0][c][lane];
+#pragma unroll
+        for (int g = 1; g < SD_GROUPS; g++) v += part[g][c][lane];
+        if (serial) v = sd_serial(a, t, j0 + j, n);
+        sd_epilogue(a, t, z, n, v);
+    }
 }
 
 // ---- elementwise / small kernels ---------------------------------------------------------
@@ -416,57 +607,77 @@ __global__ __launch_bounds__(SD_WG) void k_sd_shift(float *buf, int H, int T, in
 
 // ---- launchers ----------------------------------------------------------------------------
 
-// tile: 0 = by size (128 x 128 where that still gives two workgroups per CU, else the
-// largest of 64, 32, 16 rows x 64 columns that fills the CUs), 16, 32, 64 or 128 = forced.
-// Every tile sums each output's products in the same order, so the choice never changes
-// a result bit.
-extern "C" hipError_t qt_launch_sd_gemm(const float *X, int ldx, int Tx, int xlo, const float *W, int K, int N, int ntap,
-                                        const int *off, int phases, int T, float *Y, int ldy, const float *bias,
+// bf16 values of a layer's packed weights
+extern "C" size_t qt_sd_pack_elems(int K, int N, int ntap, int phases) {
+    return (size_t)((K + 31) / 32) * ntap * phases * ((N + 15) / 16) * 1536;
+}
+extern "C" hipError_t qt_launch_sd_pack(const float *src, long long sn, long long sk, long long sc, int cols, int stride,
+                                        int ntap, int phases, int N, int n0, int nn, int k0, int kk, uint16_t *dst,
+                                        int *bad, hipStream_t st) {
+    if (!src || !dst || !bad || n0 % 16 || k0 % 32 || nn <= 0 || kk <= 0 || n0 + nn > N) return hipErrorInvalidValue;
+    const SdPackArgs a = {src, sn, sk, sc, cols, stride, ntap, phases, (N + 15) / 16, n0, nn, k0, kk, dst, bad};
+    const int t = (kk + 31) / 32 * ntap * ((nn + 15) / 16);
+    hipLaunchKernelGGL(k_sd_pack, dim3((t + QT_WAVES - 1) / QT_WAVES, 1, phases), dim3(SD_WG), 0, st, a);
+    return hipGetLastError();
+}
+
+// tile: 0 = by size, 16, 32, 64 or 128 = rows per workgroup.  Every tile sums each output's
+// products in the same order, so the choice never changes a result bit.
+extern "C" hipError_t qt_launch_sd_gemm(const float *X, int ldx, int Tx, int xlo, const uint16_t *W, int serial, int K, int N,
+                                        int ntap, const int *off, int phases, int T, float *Y, int ldy, const float *bias,
                                         const float *cscale, const float *R, const float *sa, const float *sib,
                                         float *Y2, int epi, int tile, hipStream_t st) {
-    if (!X || !W || !Y || K <= 0 || K % SD_KC || N <= 0 || N % 4 || ntap < 1 || ntap > SD_MAXTAP || phases < 1 ||
-        T <= 0 || Tx <= 0 || xlo > 0 || ldx % 4 || ldx < K || ldy < N)
+    if (!X || !W || !Y || K <= 0 || K % 16 || N <= 0 || N % 4 || ntap < 1 || ntap > SD_MAXTAP || phases < 1 ||
+        T <= 0 || Tx <= 0 || xlo > 0 || ldx % 4 || ldx < K || ldy < N || ldy % 4)
         return hipErrorInvalidValue;
     if (((epi & 1) && !bias) || ((epi & 4) && !cscale) || ((epi & 8) && !R)) return hipErrorInvalidValue;
     if ((epi & (SD_EPI_SNAKE | SD_EPI_SNAKE2)) && (!sa || !sib)) return hipErrorInvalidValue;
     if ((epi & SD_EPI_SNAKE2) && (!Y2 || (epi & SD_EPI_SNAKE))) return hipErrorInvalidValue;
     SdGemmArgs a;
-    a.X = X; a.ldx = ldx; a.Tx = Tx; a.xlo = xlo; a.W = W; a.K = K; a.N = N; a.ntap = ntap;
-    for (int i = 0; i < SD_MAXTAP; i++) a.off[i] = i < ntap ? off[i] : 0;
+    a.X = X; a.ldx = ldx; a.Tx = Tx; a.xlo = xlo; a.W = W; a.serial = serial; a.K = K; a.N = N; a.ntap = ntap;
+    a.slices = (K + 31) / 32; a.tiles = (N + 15) / 16; a.phases = phases;
+    int omax = off[0];
+    a.omin = off[0];
+    for (int i = 0; i < SD_MAXTAP; i++) {
+        a.off[i] = i < ntap ? off[i] : 0;
+        if (i < ntap && off[i] < a.omin) a.omin = off[i];
+        if (i < ntap && off[i] > omax) omax = off[i];
+    }
+    a.span = omax - a.omin;
+    a.tps = a.span <= SD_HALO ? ntap : 1;
     a.T = T; a.Y = Y; a.ldy = ldy; a.os = phases; a.bias = bias; a.cscale = cscale; a.R = R; a.epi = epi;
     a.sa = sa; a.sib = sib; a.Y2 = Y2;
-    const long long nt = (long long)((N + 63) / 64) * phases;
-    const long long big = (long long)((T + 127) / 128) * ((N + 127) / 128) * phases;
-    if (tile == 0) {
-        // the largest row tile whose grid still gives every CU a workgroup: a streaming
-        // chunk of a few frames leaves T at 10..320 rows, where 64-row tiles would be
-        // mostly padding on a few dozen CUs
-        if (N >= 128 && big >= 512) tile = 128;
-        else if ((T + 63) / 64 * nt >= 256) tile = 64;
-        else if ((T + 31) / 32 * nt >= 256) tile = 32;
-        else tile = 16;
-    }
+    const bool grp = a.slices >= SD_GROUP_SLICES;
+    const int all = phases * a.tiles;
+    const auto wgs = [&](int tt, int nt) { return (long long)((T + tt - 1) / tt) * ((all + nt - 1) / nt); };
+    if (tile == 0) tile = wgs(128, 8) >= 256 ? 128 : wgs(64, 8) >= 256 ? 64 : wgs(32, grp ? 2 : 4) >= 256 ? 32 : 16;
+#define SD_TILE(WN, NT, WT, MT, G)                                                                                          \
+    hipLaunchKernelGGL((k_sd_tile<WN, NT, WT, MT, G>),                                                                      \
+                       dim3((T + 16 * MT * WT - 1) / (16 * MT * WT), (all + WN * NT - 1) / (WN * NT)), dim3(SD_WG), 0, st, a)
+#define SD_SPLIT(NT, MT, D)                                                                                                 \
+    hipLaunchKernelGGL((k_sd_split<NT, MT, D>), dim3((T + 16 * MT - 1) / (16 * MT), (all + NT - 1) / NT),                   \
+                       dim3(64 * SD_GROUPS), 0, st, a)
+    // 96 channels a tile where 128 would be half empty (the decoder's last two blocks: 192 and 96)
+    const bool n96 = !grp && all % 8 && all % 6 == 0;
     if (tile == 128) {
-        dim3 grid((T + 127) / 128, (N + 127) / 128, phases);
-        hipLaunchKernelGGL((k_sd_gemm<128, 128, 2, 16>), grid, dim3(SD_WG), 0, st, a);
+        if (grp) SD_TILE(4, 2, 1, 8, true);
+        else if (n96) SD_TILE(2, 3, 2, 4, false);
+        else SD_TILE(4, 2, 1, 8, false);
     } else if (tile == 64) {
-        dim3 grid((T + 63) / 64, (N + 63) / 64, phases);
-        hipLaunchKernelGGL((k_sd_gemm<64, 64, 2, 16>), grid, dim3(SD_WG), 0, st, a);
-    } else if (tile == 32 || tile == 16) {
-        // the small tiles stage 64-wide K chunks where K allows: a quarter of the barriers
-        // and LDS round trips per MFMA (the per-element order is the same)
-        dim3 grid((T + tile - 1) / tile, (N + 63) / 64, phases);
-        const bool k64 = K % 64 == 0;
-        if (tile == 32) {
-            if (k64) hipLaunchKernelGGL((k_sd_gemm<32, 64, 4, 64>), grid, dim3(SD_WG), 0, st, a);
-            else hipLaunchKernelGGL((k_sd_gemm<32, 64, 8, 16>), grid, dim3(SD_WG), 0, st, a);
-        } else {
-            if (k64) hipLaunchKernelGGL((k_sd_gemm<16, 64, 4, 64>), grid, dim3(SD_WG), 0, st, a);
-            else hipLaunchKernelGGL((k_sd_gemm<16, 64, 8, 16>), grid, dim3(SD_WG), 0, st, a);
-        }
+        if (grp) SD_TILE(4, 2, 1, 4, true);
+        else if (n96) SD_TILE(2, 3, 2, 2, false);
+        else SD_TILE(4, 2, 1, 4, false);
+    } else if (tile == 32) {
+        if (grp) SD_SPLIT(2, 2, 2);
+        else SD_TILE(4, 1, 1, 2, false);
+    } else if (tile == 16) {
+        if (grp) SD_SPLIT(1, 1, 4);
+        else SD_TILE(4, 1, 1, 1, false);
     } else {
         return hipErrorInvalidValue;
     }
+#undef SD_TILE
+#undef SD_SPLIT
     return hipGetLastError();
 }
 

@@ -3,9 +3,10 @@
  * into the implicit-GEMM layouts, and the one-shot decode sequence of
  * qwen_speech_decoder_decode (sd.c:579-1290) as kernel launches on one stream.
  *
- * Layouts on the device (all f32): activations [T][C]; a conv or linear layer is
- * W[phase][tap][K = in][N = out] with per-tap input row offsets:
- *   linear   [out][in]              -> one tap, offset 0 (W transposed);
+ * Layouts on the device: activations f32 [T][C]; a conv or linear layer's weights as the
+ * GEMM's packed planes (k_sd_pack, straight from the file's layout) with per-tap input row
+ * offsets:
+ *   linear   [out][in]              -> one tap, offset 0;
  *   conv1d   [out][in][k], dil d    -> k taps, offsets (p - k + 1) d;
  *   convT    [in][out][2s], stride s-> s phases (output rows t*s + z), taps: column z at
  *            offset 0 and column z + s at offset -1 (when z + s < kernel).
@@ -27,10 +28,13 @@
 
 enum { SD_BIAS = 1, SD_GELU = 2, SD_CSCALE = 4, SD_RESID = 8, SD_SNAKE = 16, SD_SNAKE2 = 32 };
 
+#define SD_MAXCONV 80
+
 typedef struct {
-    float *w, *b;
+    uint16_t *w; float *b;
     int K, N, ntap, phases;
     int off[8];
+    int id;                       /* index into the state's serial[] */
 } sd_conv_t;
 
 typedef struct { float *a, *ib; } sd_snake_t;
@@ -55,6 +59,7 @@ typedef struct {
     int cap;
     float *E, *V, *P, *H, *XN, *QKV, *A, *GU, *M, *LAT, *big[3];
     int *dcodes; float *daudio;
+    int n_convs, serial[SD_MAXCONV];  /* layers with a weight that has no planes (infinite or NaN) */
     void **allocs; int n_allocs, cap_allocs;
 } sd_t;
 
@@ -93,7 +98,8 @@ typedef struct {
     qwen_hip_sd_get_fn get;
     void *user;
     sd_t *s;
-    float *tmp; size_t tmp_n;
+    float *tmp; size_t tmp_n;     /* device: the tensor being packed */
+    int *serial;                  /* device: [SD_MAXCONV] */
     int bad;
 } sd_ld_t;
 
@@ -108,12 +114,21 @@ static const float *sd_get(sd_ld_t *L, const char *name, long long n) {
     return p;
 }
 
-static float *sd_tmp(sd_ld_t *L, size_t n) {
-    if (n > L->tmp_n) {
-        free(L->tmp);
-        L->tmp = (float *)malloc(n * sizeof(float));
-        L->tmp_n = L->tmp ? n : 0;
-        if (!L->tmp) { qt_seterr("sd_init: out of host memory"); L->bad = 1; }
+/* a tensor in the loader's device buffer (until the next one): the kernels that read the
+ * previous one are ahead of the copy on the stream, and the host source may be reused */
+static const float *sd_stage(sd_ld_t *L, const char *name, long long n) {
+    const float *w = sd_get(L, name, n);
+    if (L->bad) return NULL;
+    if ((size_t)n > L->tmp_n) {
+        if (L->tmp) (void)hipFree(L->tmp);
+        L->tmp = NULL; L->tmp_n = 0;
+        if (hipMalloc((void **)&L->tmp, (size_t)n * sizeof(float)) == hipSuccess) L->tmp_n = (size_t)n;
+    }
+    if (!L->tmp_n || hipMemcpyAsync(L->tmp, w, (size_t)n * sizeof(float), hipMemcpyHostToDevice, L->s->st) != hipSuccess ||
+        hipStreamSynchronize(L->s->st) != hipSuccess) {
+        qt_seterr("sd_init: device allocation or upload failed");
+        L->bad = 1;
+        return NULL;
     }
     return L->tmp;
 }
@@ -142,31 +157,57 @@ static sd_snake_t sd_snake(sd_ld_t *L, const char *pa, const char *pb, int n) {
     return r;
 }
 
-/* linear [out][in] (+ bias) -> one tap [in][out] */
-static sd_conv_t sd_linear(sd_ld_t *L, const char *wn, const char *bn, int out, int in) {
+/* a layer's shape and its (unfilled) packed weights */
+static sd_conv_t sd_layer(sd_ld_t *L, int K, int N, int ntap, int phases) {
     sd_conv_t c; memset(&c, 0, sizeof c);
-    c.K = in; c.N = out; c.ntap = 1; c.phases = 1;
-    const float *w = sd_get(L, wn, (long long)out * in);
-    float *t = sd_tmp(L, (size_t)out * in);
+    c.K = K; c.N = N; c.ntap = ntap; c.phases = phases;
     if (L->bad) return c;
-    for (int o = 0; o < out; o++) for (int i = 0; i < in; i++) t[(size_t)i * out + o] = w[(size_t)o * in + i];
-    c.w = sd_put(L, t, (size_t)out * in);
+    c.id = L->s->n_convs++;
+    if (!L->serial && (hipMalloc((void **)&L->serial, SD_MAXCONV * sizeof(int)) != hipSuccess ||
+                       hipMemsetAsync(L->serial, 0, SD_MAXCONV * sizeof(int), L->s->st) != hipSuccess)) L->bad = 1;
+    if (c.id >= SD_MAXCONV || !(c.w = (uint16_t *)sd_dalloc(L->s, qt_sd_pack_elems(K, N, ntap, phases) * sizeof(uint16_t))))
+        L->bad = 1;
+    if (L->bad) qt_seterr("sd_init: device allocation failed");
+    return c;
+}
+
+/* the tensor wn, element [n][k][column] at n sn + k sk + column sc, into channels [n0, n0 + nn) and
+ * k [k0, k0 + kk) of c (stride: a transposed conv's, else 0) */
+static void sd_pack(sd_ld_t *L, sd_conv_t *c, const char *wn, long long sn, long long sk, long long sc, int cols, int stride,
+                    int n0, int nn, int k0, int kk) {
+    const float *w = sd_stage(L, wn, (long long)nn * kk * cols);
+    if (L->bad) return;
+    if (qt_launch_sd_pack(w, sn, sk, sc, cols, stride, c->ntap, c->phases, c->N, n0, nn, k0, kk, c->w, L->serial + c->id,
+                          L->s->st) != hipSuccess) {
+        qt_seterr("sd_init: packing %s failed", wn);
+        L->bad = 1;
+    }
+}
+
+/* which layers' weights have no planes, once every layer is packed; frees the loader's buffers */
+static int sd_loaded(sd_ld_t *L) {
+    if (!L->bad && L->serial &&
+        (hipMemcpyAsync(L->s->serial, L->serial, SD_MAXCONV * sizeof(int), hipMemcpyDeviceToHost, L->s->st) != hipSuccess ||
+         hipStreamSynchronize(L->s->st) != hipSuccess)) L->bad = 1;
+    if (L->tmp) (void)hipFree(L->tmp);
+    if (L->serial) (void)hipFree(L->serial);
+    L->tmp = NULL; L->serial = NULL;
+    return L->bad;
+}
+
+/* linear [out][in] (+ bias) -> one tap */
+static sd_conv_t sd_linear(sd_ld_t *L, const char *wn, const char *bn, int out, int in) {
+    sd_conv_t c = sd_layer(L, in, out, 1, 1);
+    sd_pack(L, &c, wn, in, 1, 0, 1, 0, 0, out, 0, in);
     if (bn) c.b = sd_vec(L, bn, out);
     return c;
 }
 
-/* causal conv [out][in][k], dilation d -> k taps [p][in][out] at offsets (p - k + 1) d */
+/* causal conv [out][in][k], dilation d -> k taps at offsets (p - k + 1) d */
 static sd_conv_t sd_conv(sd_ld_t *L, const char *wn, const char *bn, int out, int in, int k, int d) {
-    sd_conv_t c; memset(&c, 0, sizeof c);
-    c.K = in; c.N = out; c.ntap = k; c.phases = 1;
+    sd_conv_t c = sd_layer(L, in, out, k, 1);
     for (int p = 0; p < k; p++) c.off[p] = (p - k + 1) * d;
-    const float *w = sd_get(L, wn, (long long)out * in * k);
-    float *t = sd_tmp(L, (size_t)out * in * k);
-    if (L->bad) return c;
-    for (int o = 0; o < out; o++)
-        for (int i = 0; i < in; i++)
-            for (int p = 0; p < k; p++) t[((size_t)p * in + i) * out + o] = w[((size_t)o * in + i) * k + p];
-    c.w = sd_put(L, t, (size_t)out * in * k);
+    sd_pack(L, &c, wn, (long long)in * k, k, 1, k, 0, 0, out, 0, in);
     if (bn) c.b = sd_vec(L, bn, out);
     return c;
 }
@@ -174,21 +215,9 @@ static sd_conv_t sd_conv(sd_ld_t *L, const char *wn, const char *bn, int out, in
 /* causal transposed conv [in][out][k], stride s (k <= 2s) -> s phases of taps at offsets
  * 0 (column z) and -1 (column z + s; zero where z + s >= k) */
 static sd_conv_t sd_convt(sd_ld_t *L, const char *wn, const char *bn, int in, int out, int k, int s) {
-    sd_conv_t c; memset(&c, 0, sizeof c);
-    c.K = in; c.N = out; c.phases = s; c.ntap = k > s ? 2 : 1;
+    sd_conv_t c = sd_layer(L, in, out, k > s ? 2 : 1, s);
     c.off[0] = 0; c.off[1] = -1;
-    const float *w = sd_get(L, wn, (long long)in * out * k);
-    const size_t per = (size_t)in * out;
-    float *t = sd_tmp(L, (size_t)s * c.ntap * per);
-    if (L->bad) return c;
-    for (int z = 0; z < s; z++)
-        for (int p = 0; p < c.ntap; p++) {
-            const int col = z + p * s;
-            float *dst = t + ((size_t)z * c.ntap + p) * per;
-            for (int i = 0; i < in; i++)
-                for (int o = 0; o < out; o++) dst[(size_t)i * out + o] = col < k ? w[((size_t)i * out + o) * k + col] : 0.f;
-        }
-    c.w = sd_put(L, t, (size_t)s * c.ntap * per);
+    sd_pack(L, &c, wn, k, (long long)out * k, 1, k, s, 0, out, 0, in);
     if (bn) c.b = sd_vec(L, bn, out);
     return c;
 }
@@ -199,7 +228,7 @@ void *qwen_hip_sd_init(qwen_hip_sd_get_fn get, void *user) {
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) { qt_seterr("sd_init: no HIP device"); return NULL; }
     sd_t *s = (sd_t *)calloc(1, sizeof *s);
     if (!s) { qt_seterr("sd_init: out of host memory"); return NULL; }
-    sd_ld_t L = {get, user, s, NULL, 0, 0};
+    sd_ld_t L = {get, user, s, NULL, 0, NULL, 0};
     char nm[160], nb[160];
     if (hipStreamCreateWithFlags(&s->st, hipStreamNonBlocking) != hipSuccess) { qt_seterr("sd_init: stream"); goto fail; }
     /* codebooks: EMA sums over usage, on the device */
@@ -218,13 +247,9 @@ void *qwen_hip_sd_init(qwen_hip_sd_get_fn get, void *user) {
     }
     /* VQ projections as one K = 512 product of [codebook 0 | sum of 1..15] rows */
     {
-        s->vq.K = 2 * SD_CB; s->vq.N = 512; s->vq.ntap = 1; s->vq.phases = 1;
-        const float *w1 = sd_get(&L, "decoder.quantizer.rvq_first.output_proj.weight", 512LL * SD_CB);
-        float *t = sd_tmp(&L, (size_t)2 * SD_CB * 512);
-        if (!L.bad) for (int o = 0; o < 512; o++) for (int i = 0; i < SD_CB; i++) t[(size_t)i * 512 + o] = w1[(size_t)o * SD_CB + i];
-        const float *w2 = sd_get(&L, "decoder.quantizer.rvq_rest.output_proj.weight", 512LL * SD_CB);
-        if (!L.bad) for (int o = 0; o < 512; o++) for (int i = 0; i < SD_CB; i++) t[(size_t)(SD_CB + i) * 512 + o] = w2[(size_t)o * SD_CB + i];
-        s->vq.w = sd_put(&L, t, (size_t)2 * SD_CB * 512);
+        s->vq = sd_layer(&L, 2 * SD_CB, 512, 1, 1);
+        sd_pack(&L, &s->vq, "decoder.quantizer.rvq_first.output_proj.weight", SD_CB, 1, 0, 1, 0, 0, 512, 0, SD_CB);
+        sd_pack(&L, &s->vq, "decoder.quantizer.rvq_rest.output_proj.weight", SD_CB, 1, 0, 1, 0, 0, 512, SD_CB, SD_CB);
     }
     s->pre = sd_conv(&L, "decoder.pre_conv.conv.weight", "decoder.pre_conv.conv.bias", 1024, 512, 3, 1);
     s->inp = sd_linear(&L, "decoder.pre_transformer.input_proj.weight", "decoder.pre_transformer.input_proj.bias", 512, 1024);
@@ -235,29 +260,17 @@ void *qwen_hip_sd_init(qwen_hip_sd_get_fn get, void *user) {
         y->n2 = sd_vec(&L, LN("post_attention_layernorm.weight"), 512);
         y->ls1 = sd_vec(&L, LN("self_attn_layer_scale.scale"), 512);
         y->ls2 = sd_vec(&L, LN("mlp_layer_scale.scale"), 512);
-        /* q | k | v as one [512][3072] tap, gate | up as one [512][2048] tap */
+        /* q | k | v as one layer of 3072 channels, gate | up as one of 2048 */
         {
-            y->qkv.K = 512; y->qkv.N = 3072; y->qkv.ntap = 1; y->qkv.phases = 1;
-            float *t = sd_tmp(&L, (size_t)512 * 3072);
             const char *nmq[3] = {"self_attn.q_proj.weight", "self_attn.k_proj.weight", "self_attn.v_proj.weight"};
-            for (int q = 0; q < 3 && !L.bad; q++) {
-                const float *w = sd_get(&L, LN(nmq[q]), 1024LL * 512);
-                if (L.bad) break;
-                for (int o = 0; o < 1024; o++) for (int i = 0; i < 512; i++) t[(size_t)i * 3072 + q * 1024 + o] = w[(size_t)o * 512 + i];
-            }
-            y->qkv.w = sd_put(&L, t, (size_t)512 * 3072);
+            y->qkv = sd_layer(&L, 512, 3072, 1, 1);
+            for (int q = 0; q < 3; q++) sd_pack(&L, &y->qkv, LN(nmq[q]), 512, 1, 0, 1, 0, q * 1024, 1024, 0, 512);
         }
         y->o = sd_linear(&L, LN("self_attn.o_proj.weight"), NULL, 512, 1024);
         {
-            y->gu.K = 512; y->gu.N = 2048; y->gu.ntap = 1; y->gu.phases = 1;
-            float *t = sd_tmp(&L, (size_t)512 * 2048);
             const char *nmg[2] = {"mlp.gate_proj.weight", "mlp.up_proj.weight"};
-            for (int q = 0; q < 2 && !L.bad; q++) {
-                const float *w = sd_get(&L, LN(nmg[q]), 1024LL * 512);
-                if (L.bad) break;
-                for (int o = 0; o < 1024; o++) for (int i = 0; i < 512; i++) t[(size_t)i * 2048 + q * 1024 + o] = w[(size_t)o * 512 + i];
-            }
-            y->gu.w = sd_put(&L, t, (size_t)512 * 2048);
+            y->gu = sd_layer(&L, 512, 2048, 1, 1);
+            for (int q = 0; q < 2; q++) sd_pack(&L, &y->gu, LN(nmg[q]), 512, 1, 0, 1, 0, q * 1024, 1024, 0, 512);
         }
         y->dn = sd_linear(&L, LN("mlp.down_proj.weight"), NULL, 512, 1024);
 #undef LN
@@ -309,8 +322,8 @@ void *qwen_hip_sd_init(qwen_hip_sd_get_fn get, void *user) {
     if (L.bad) goto fail;
     /* RoPE tables of the pre-transformer: angle = pos / theta^(2i/64) (sd.c:455-463) */
     {
-        float *c = sd_tmp(&L, (size_t)2 * SD_ROPE_POS * 32);
-        if (L.bad) goto fail;
+        float *c = (float *)malloc((size_t)2 * SD_ROPE_POS * 32 * sizeof(float));
+        if (!c) { qt_seterr("sd_init: out of host memory"); goto fail; }
         for (int p = 0; p < SD_ROPE_POS; p++)
             for (int i = 0; i < 32; i++) {
                 const float ang = (float)p / powf(10000.0f, (float)(2 * i) / 64.0f);
@@ -319,12 +332,13 @@ void *qwen_hip_sd_init(qwen_hip_sd_get_fn get, void *user) {
             }
         s->rope_c = sd_put(&L, c, (size_t)SD_ROPE_POS * 32);
         s->rope_s = sd_put(&L, c + SD_ROPE_POS * 32, (size_t)SD_ROPE_POS * 32);
+        free(c);
     }
-    if (L.bad || hipStreamSynchronize(s->st) != hipSuccess) goto fail;
-    free(L.tmp);
+    if (sd_loaded(&L) || hipStreamSynchronize(s->st) != hipSuccess) goto fail;
     return s;
 fail:
-    free(L.tmp);
+    L.bad = 1;
+    (void)sd_loaded(&L);
     if (!qwen_hip_last_error()[0]) qt_seterr("sd_init failed");
     qwen_hip_sd_free(s);
     return NULL;
@@ -358,14 +372,14 @@ static int sd_reserve(sd_t *s, int n) {
 
 static hipError_t sd_run(const sd_t *s, const sd_conv_t *c, const float *X, int Tx, int T, float *Y, int epi,
                          const float *cscale, const float *R) {
-    return qt_launch_sd_gemm(X, c->K, Tx, 0, c->w, c->K, c->N, c->ntap, c->off, c->phases, T, Y, c->N,
+    return qt_launch_sd_gemm(X, c->K, Tx, 0, c->w, s->serial[c->id], c->K, c->N, c->ntap, c->off, c->phases, T, Y, c->N,
                              c->b, cscale, R, NULL, NULL, NULL, epi | (c->b ? SD_BIAS : 0), 0, s->st);
 }
 
 /* the same with a snake on the output: in place (Y2 == NULL) or into Y2 beside Y */
 static hipError_t sd_run_snake(const sd_t *s, const sd_conv_t *c, const float *X, int Tx, int T, float *Y, int epi,
                                const float *R, const sd_snake_t *sn, float *Y2) {
-    return qt_launch_sd_gemm(X, c->K, Tx, 0, c->w, c->K, c->N, c->ntap, c->off, c->phases, T, Y, c->N, c->b, NULL, R,
+    return qt_launch_sd_gemm(X, c->K, Tx, 0, c->w, s->serial[c->id], c->K, c->N, c->ntap, c->off, c->phases, T, Y, c->N, c->b, NULL, R,
                              sn->a, sn->ib, Y2, epi | (c->b ? SD_BIAS : 0) | (Y2 ? SD_SNAKE2 : SD_SNAKE), 0, s->st);
 }
 
@@ -495,17 +509,17 @@ static int sd_op(float *Y, const float *X, const float *W, const float *bias, in
         return -1;
     }
     sd_one_t one = {W, (long long)Cout * Cin * k};
-    sd_ld_t L = {sd_one_get, &one, &tmp, NULL, 0, 0};
+    sd_ld_t L = {sd_one_get, &one, &tmp, NULL, 0, NULL, 0};
     if (hipStreamCreateWithFlags(&tmp.st, hipStreamNonBlocking) != hipSuccess) { qt_seterr("op_sd_conv: stream"); return -1; }
     sd_conv_t c = stride ? sd_convt(&L, "w", NULL, Cin, Cout, k, stride) : sd_conv(&L, "w", NULL, Cout, Cin, k, d);
     if (!L.bad && bias) c.b = sd_put(&L, bias, (size_t)Cout);
-    free(L.tmp);
+    (void)sd_loaded(&L);
     const int Tout = stride ? Tin * stride : Tin;
     if (L.bad) goto done;
     if (hipMalloc((void **)&dx, (size_t)Tin * Cin * sizeof(float)) != hipSuccess ||
         hipMalloc((void **)&dy, (size_t)Tout * Cout * sizeof(float)) != hipSuccess) { qt_seterr("op_sd_conv: alloc"); goto done; }
     if (hipMemcpy(dx, X, (size_t)Tin * Cin * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) goto done;
-    if (qt_launch_sd_gemm(dx, Cin, Tin, 0, c.w, Cin, Cout, c.ntap, c.off, c.phases, Tin, dy, Cout, c.b, NULL, NULL, NULL,
+    if (qt_launch_sd_gemm(dx, Cin, Tin, 0, c.w, tmp.serial[c.id], Cin, Cout, c.ntap, c.off, c.phases, Tin, dy, Cout, c.b, NULL, NULL, NULL,
                           NULL, NULL, c.b ? SD_BIAS : 0, tile, tmp.st) != hipSuccess ||
         hipMemcpyAsync(Y, dy, (size_t)Tout * Cout * sizeof(float), hipMemcpyDeviceToHost, tmp.st) != hipSuccess ||
         hipStreamSynchronize(tmp.st) != hipSuccess) { qt_seterr("op_sd_conv: launch failed"); goto done; }
@@ -643,7 +657,7 @@ static hipError_t sds_gemm(const sd_t *s, const sd_conv_t *c, const float *X, in
                            const float *cscale, const float *R, const sd_snake_t *sn, float *Y2) {
     int e = epi | (c->b ? SD_BIAS : 0);
     if (sn) e |= Y2 ? SD_SNAKE2 : SD_SNAKE;
-    return qt_launch_sd_gemm(X, c->K, T, xlo, c->w, c->K, c->N, c->ntap, c->off, c->phases, T, Y, c->N, c->b, cscale, R,
+    return qt_launch_sd_gemm(X, c->K, T, xlo, c->w, s->serial[c->id], c->K, c->N, c->ntap, c->off, c->phases, T, Y, c->N, c->b, cscale, R,
                              sn ? sn->a : NULL, sn ? sn->ib : NULL, Y2, e, 0, s->st);
 }
 
