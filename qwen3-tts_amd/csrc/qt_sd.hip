@@ -195,6 +195,11 @@ __device__ __forceinline__ int sd_unit(int row, int kg) { return 16 * (kg ^ (((r
 // loaded once, split into planes on the way into LDS, and every tap runs from there, so a
 // 7-tap conv stages each input once; the weights' planes come straight from L2 in operand
 // order, one (slice, tap) ahead.  Two LDS buffers, one barrier per slice.
+// Bound by the matrix cores where there are rows enough: 7 taps of 384 -> 384 channels over 20 000
+// rows take 175 us = 236 TFLOP/s of f32 products, 1.42 PFLOP/s of plane products (the f32 matrix
+// cores: 450 us, 92 TFLOP/s; a 4096 x 4096 library product in bf16 reaches 1.13 PFLOP/s here); the
+// 96-channel convs are held by their f32 traffic as well (240 000 rows: 167 us, 185 TFLOP/s).
+// Weight planes two or three items ahead, in a loop unrolled over a ring: no faster.
 template <int WN, int NT, int WT, int MT, bool GRP>
 __global__ __launch_bounds__(SD_WG) __attribute__((amdgpu_waves_per_eu(2))) void k_sd_tile(SdGemmArgs a) {
     static_assert(WN * WT == QT_WAVES, "four waves");
@@ -319,7 +324,9 @@ __global__ __launch_bounds__(SD_WG) __attribute__((amdgpu_waves_per_eu(2))) void
 // A workgroup of eight waves computes 16 NT channels x 16 MT rows; wave g takes the layer's g-th
 // run of slices, with its operands straight from memory (no staging, no barrier until the
 // runs' sums meet in LDS), D (slice, tap) pairs in flight.  A call of a few frames leaves the
-// long-K layers with a few dozen such tiles: the time is the latency of one run.
+// long-K layers with a few dozen such tiles: the time is the latency of one run (10 rows: 512 -> 3072
+// 6.0 us, 1024 -> 512 5.8 us, where one wave per tile walked all of K in f32 in 16 to 21 us).  With more
+// rows it is held by L2: every tile reads its own operands, 550 TFLOP/s of plane products.
 template <int NT, int MT, int D>
 __global__ __launch_bounds__(64 * SD_GROUPS) void k_sd_split(SdGemmArgs a) {
     __shared__ __align__(16) qt_f32x4 part[SD_GROUPS][NT * MT][64];
@@ -650,7 +657,19 @@ extern "C" hipError_t qt_launch_sd_gemm(const float *X, int ldx, int Tx, int xlo
     const bool grp = a.slices >= SD_GROUP_SLICES;
     const int all = phases * a.tiles;
     const auto wgs = [&](int tt, int nt) { return (long long)((T + tt - 1) / tt) * ((all + nt - 1) / nt); };
-    if (tile == 0) tile = wgs(128, 8) >= 256 ? 128 : wgs(64, 8) >= 256 ? 64 : wgs(32, grp ? 2 : 4) >= 256 ? 32 : 16;
+    if (tile == 0) {
+        // 64-row tiles from about one a CU on; below that the layers with runs take k_sd_split
+        // (32 rows reach 550 TFLOP/s of plane products from L2; 16 rows while every tile has a CU of its
+        // own: 768 -> 768 channels, 7 taps, 320 rows: 74 us with 16, 37 with 32, 121 with 64, and at 32 rows
+        // 20 / 32 / 118) and the others the narrow tiles (384 channels, 1600 rows: 42 us against 59).
+        // 64 or 128 rows: by the rounds that the resident workgroups need, three of 64 rows a
+        // CU or two of 128 (768 -> 5 x 384 channels: 4000 rows 129 us with 128, 146 with 64; 768 -> 768,
+        // 12800 rows: 488 and 462)
+        const long long w64 = wgs(64, 8), w128 = wgs(128, 8);
+        if (grp && w64 < 224) tile = wgs(16, 1) <= 256 ? 16 : 32;
+        else if (!grp && w64 < 256) tile = wgs(32, 4) >= 256 ? 32 : 16;
+        else tile = 4 * ((w128 + 511) / 512) <= 3 * ((w64 + 767) / 768) ? 128 : 64;
+    }
 #define SD_TILE(WN, NT, WT, MT, G)                                                                                          \
     hipLaunchKernelGGL((k_sd_tile<WN, NT, WT, MT, G>),                                                                      \
                        dim3((T + 16 * MT * WT - 1) / (16 * MT * WT), (all + WN * NT - 1) / (WN * NT)), dim3(SD_WG), 0, st, a)

@@ -161,6 +161,48 @@ def test_op_sd_tiles_same_bits(T, cin, cout, k, d, s):
         assert np.array_equal(y.view(np.uint32), outs[0].view(np.uint32))
 
 
+@pytest.mark.parametrize("T,cin,cout,k,d,tile", [(70, 48, 20, 2, 60, 64), (200, 512, 32, 3, 40, 128), (33, 768, 100, 7, 9, 0),
+                                                 (129, 96, 36, 7, 9, 128), (1, 16, 4, 8, 1, 0), (65, 528, 288, 1, 1, 64)])
+def test_op_sd_conv_odd_shapes_vs_f64(T, cin, cout, k, d, tile):
+    """Shapes off the decoder's: taps that reach past a staged tile (60 and 80 rows back), K with half
+    a slice, channels that end inside a tile.  Bound: f32 rounding of the sum of cin * k products
+    (sqrt(cin k) 2^-24 relative to the product norm, with a factor 4)."""
+    rng = np.random.default_rng(T + cin + k + d)
+    x = rng.standard_normal((T, cin)).astype(np.float32)
+    w = (rng.standard_normal((cout, cin, k)) / np.sqrt(cin * k)).astype(np.float32)
+    y = np.empty((T, cout), np.float32)
+    hip.check(hip.lib().qwen_hip_op_sd_conv(y.ctypes.data, x.ctypes.data, w.ctypes.data, None, T, cin, cout, k, d, tile),
+              "op_sd_conv")
+    assert np.abs(y - _conv_ref(x, w, None, d)).max() < 4 * np.sqrt(cin * k) * 2.0 ** -24 + 2.0 ** -20
+
+
+@pytest.mark.parametrize("cin,tile", [(96, 16), (96, 128), (512, 16), (512, 32), (512, 64)])
+@pytest.mark.parametrize("what", ["x", "w"])
+def test_op_sd_conv_non_finite(cin, tile, what):
+    """Infinities, NaN and values past bf16's range reach exactly the outputs that plain f32
+    arithmetic gives them to; the others keep their values."""
+    rng = np.random.default_rng(cin + tile)
+    T, cout = 90, 40
+    x = rng.standard_normal((T, cin)).astype(np.float32)
+    w = (rng.standard_normal((cout, cin, 3)) / np.sqrt(cin * 3)).astype(np.float32)
+    if what == "x":
+        x[7, 3], x[40, 0], x[41, 5], x[80, 9], x[60, 1] = np.inf, -np.inf, np.nan, np.inf, 3.395e38
+        w[:, 1] = np.clip(w[:, 1], -0.1, 0.1)
+        x[80, 10] = -np.inf
+    else:
+        w[3, 2, 0], w[9, 5, 2], w[20, 0, 1] = np.inf, np.nan, -np.inf
+    y = np.empty((T, cout), np.float32)
+    hip.check(hip.lib().qwen_hip_op_sd_conv(y.ctypes.data, x.ctypes.data, w.ctypes.data, None, T, cin, cout, 3, 2, tile),
+              "op_sd_conv")
+    with np.errstate(invalid="ignore"):
+        xp = np.concatenate([np.zeros((4, cin)), x.astype(np.float64)])
+        want = sum((xp[2 * p:2 * p + T, None, :] * w[None, :, :, p].astype(np.float64)).sum(-1) for p in range(3))
+    assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isinf(y), np.isinf(want))
+    inf, ok = np.isinf(want), np.isfinite(want)
+    assert inf.any() and np.array_equal(np.sign(y[inf]), np.sign(want[inf]))
+    assert np.allclose(y[ok], want[ok], rtol=1e-5, atol=1e-5)
+
+
 @need_ref
 def test_sd_glue_over_reference_ctx():
     """The reference-side glue (qwen_hip_glue_sd_init over ctx->speech_safetensors, the
