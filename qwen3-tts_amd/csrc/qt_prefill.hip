@@ -14,7 +14,7 @@
 // the bf16 weights.  Both operands are read row-major exactly as stored: the MFMA A
 // operand is 16 weight rows x 8 consecutive k, the B operand 16 positions x 8
 // consecutive k of one plane, so neither needs a transpose.
-#include "qt_attn_mf.h"
+#include "qt_planes.h"
 
 #define QT_PF_WG 256
 
@@ -396,153 +396,264 @@ __global__ __launch_bounds__(QT_PF_WG) void k_pf_reduce_qkv_post(const float *pa
     }
 }
 
-// ---- causal attention, tiled -------------------------------------------------------
-// The same attention for 64 queries of one head per workgroup, over 64-key blocks held in
-// LDS (flash-style: per block, row max -> rescale of the running sums -> P.V).  Thread t
-// takes queries r = t/16 + 16a (a = 0..3) and, for the scores, keys t%16 + 16b, for P.V
-// the dims 4(t%16) + 64h + e (h = 0..1, e = 0..3); the 16 threads of a query row are one
-// DPP row, so row max and row sum are 16-lane reductions.  K rows are padded to 132
-// floats so the 16 key rows a wave reads at one offset fall in 16 different bank groups.
-#define QT_PF_KP 132
+// ---- causal attention ------------------------------------------------------------------------
+// A workgroup of eight waves takes 16 queries of the HPK heads of one kv head; wave w takes the
+// 32-key blocks w, w + 8, ..., each with its own running softmax, and the waves' sums are merged
+// through LDS at the end: no barrier in the key loop, and a prompt of a few hundred positions
+// gives every CU a workgroup (16 queries of 512 positions: 256 workgroups, the longest of two
+// blocks a wave).  Both products are f32 products on the bf16 matrix cores (qt_planes.h); K and V
+// are read from the f32 rows and split in registers, once for the HPK heads.
+//   scores: A = 16 keys, B = 16 queries: lane l ends with query l % 16 and keys 4 (l / 16) + r of
+//           each of the block's two 16-key tiles: the eight k of its group in the A operand of
+//           P.V, when k-index 8 g + e stands for key 16 (e / 4) + 4 g + e % 4.
+//   P.V:    column n of dim tile d is dim 8 n + d, so that a lane reads 8 neighbouring dims of
+//           its 8 keys (two 16-byte loads a key) and holds one column of all eight dim tiles;
+//           it ends with queries 4 (l / 16) + r and those 8 dims.
+// Bound by the latency of a wave's few blocks up to some 500 positions, then by the splitting of K
+// and V (VALU) next to the products.  16 heads, against 64 queries a workgroup over 64-key blocks in LDS on
+// the f32 matrix cores (16 to 64 queries on the VALU below 256 positions): 45 positions 8.6 -> 7.4 us,
+// 128 15.8 -> 8.8, 512 63 -> 26.7, 1024 122 -> 81, 4096 1622 -> 637; error against 64 bits at 1000 positions
+// 8.6e-7 -> 2.5e-7.
+#define QT_PF_AW 8
+#define QT_PF_AT (64 * QT_PF_AW)
+
+// One query of one head, one key after the other in f32: where an operand has no planes
+// (infinite or NaN).  One wave; sp: 64 floats of its own.
+__device__ __forceinline__ void pf_att_serial(const float *q, const float *K, const float *V, int ld, int n, float scale,
+                                              float *out, float *sp, int lane) {
+    float m = -INFINITY, l = 0.f, o0 = 0.f, o1 = 0.f;
+    for (int j0 = 0; j0 < n; j0 += 64) {
+        float s = -INFINITY;
+        if (j0 + lane < n) {
+            s = 0.f;
+            for (int d = 0; d < 128; d++) s = fmaf(q[d], K[(size_t)(j0 + lane) * ld + d], s);
+            s *= scale;
+        }
+        const float mn = fmaxf(m, group_max<64>(s)), mr = mn == -INFINITY ? 0.f : mn, c = expf(m - mr);
+        const float p = j0 + lane < n ? expf(s - mr) : 0.f;
+        __builtin_amdgcn_wave_barrier();
+        sp[lane] = p;
+        __builtin_amdgcn_s_waitcnt(0);
+        __builtin_amdgcn_wave_barrier();
+        l = l * c + group_sum<64>(p);
+        o0 *= c; o1 *= c;
+        for (int j = 0; j < min(64, n - j0); j++) {
+            o0 = fmaf(sp[j], V[(size_t)(j0 + j) * ld + lane], o0);
+            o1 = fmaf(sp[j], V[(size_t)(j0 + j) * ld + 64 + lane], o1);
+        }
+        m = mn;
+    }
+    out[lane] = o0 / l;
+    out[64 + lane] = o1 / l;
+}
+
 // P != NULL: the output goes out as the three planes of the O projection's input
 // (P[p][s][nh*128], plane stride Sp*nh*128; the same pieces k_pf_pieces makes of the f32
-// output), and the workgroup of the last query tile zeroes rows S <= s < Sp of its head.
-template <int QA>   // queries per thread: 16 * QA queries per workgroup
-__global__ __launch_bounds__(QT_PF_WG) void k_pf_fattn(const float *QKV, int ld, int S, int nh, int nkv, float scale,
-                                                        float *A, int lda, uint16_t *P, int Sp) {
-    constexpr int QB = 16 * QA;
-    __shared__ __align__(16) float qs[QB][128];
-    __shared__ __align__(16) float ks[64][QT_PF_KP];
-    __shared__ __align__(16) float vs[64][128];
-    __shared__ __align__(16) float ps[QB][68];
-    const int tid = threadIdx.x, rq = tid >> 4, cg = tid & 15;
-    const int q0 = blockIdx.x * QB, h = blockIdx.y, g = h / (nh / nkv);
+// output), and the workgroup of the last query tile zeroes rows S <= s < Sp of its heads.
+template <int HPK>
+__global__ __launch_bounds__(QT_PF_AT) __attribute__((amdgpu_waves_per_eu(2))) void k_pf_att(
+    const float *QKV, int ld, int S, int nh, int nkv, float scale, float *A, int lda, uint16_t *P, int Sp) {
+    constexpr int QB = HPK * 3 * 16 * 256;             // the queries' planes: [head][plane][16][128] bf16
+    constexpr int OB = HPK * 16 * 128 * 4;             // one wave's sums
+    static_assert(QB <= OB * QT_PF_AW, "the queries' planes and the sums share the LDS");
+    __shared__ __align__(16) uint8_t sm[OB * QT_PF_AW];
+    __shared__ float sst[2][QT_PF_AW][HPK][16];        // the waves' running maximum and sum
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, g = lane >> 4;
+    const int h0 = blockIdx.y * HPK, kvh = h0 / (nh / nkv);
+    const int qt = gridDim.x - 1 - blockIdx.x, q0 = 16 * qt;         // the longest first
     const int qd = nh * 128, kvd = nkv * 128;
-    // Q block (rows past S: zeros)
-    for (int i = tid; i < QB * 32; i += QT_PF_WG) {
-        const int r = i >> 5, c = (i & 31) * 4, q = q0 + r;
-        *reinterpret_cast<float4 *>(&qs[r][c]) =
-            q < S ? *reinterpret_cast<const float4 *>(QKV + (size_t)q * ld + h * 128 + c) : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    float m[QA], l[QA], o[QA][8];
+    const float *Kb = QKV + qd + kvh * 128, *Vb = Kb + kvd;
+    // each 32-k product is summed by itself: one rounding at the running sum's size, not six
+    const qt_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    float chk = 0.f;
+    for (int u = tid; u < HPK * 16 * 16; u += QT_PF_AT) {
+        const int h = u >> 8, row = (u >> 4) & 15, c = u & 15, q = q0 + row;
+        float v[8];
+        const float *src = QKV + (size_t)min(q, S - 1) * ld + (h0 + h) * 128 + 8 * c;
 #pragma unroll
-    for (int a = 0; a < QA; a++) {
-        m[a] = -INFINITY; l[a] = 0.f;
+        for (int e = 0; e < 2; e++) {
+            const float4 f = *reinterpret_cast<const float4 *>(src + 4 * e);
+            v[4 * e] = f.x; v[4 * e + 1] = f.y; v[4 * e + 2] = f.z; v[4 * e + 3] = f.w;
+        }
+        qt_u32x4 pl[3];
+        qt_planes8(v, pl, chk);
 #pragma unroll
-        for (int e = 0; e < 8; e++) o[a][e] = 0.f;
+        for (int p = 0; p < 3; p++)
+            *reinterpret_cast<qt_u32x4 *>(sm + (h * 3 + p) * 4096 + row * 256 + 16 * (c ^ row)) = pl[p];
     }
-    const int nkb = (q0 + QB - 1) / 64 + 1;              // key blocks up to the one holding the last query
-    for (int kb = 0; kb < nkb; kb++) {
-        const int j0 = kb * 64;
-        __syncthreads();                                // previous block's K/V/P reads done
-        for (int i = tid; i < 64 * 32; i += QT_PF_WG) {
-            const int r = i >> 5, c = (i & 31) * 4, j = j0 + r;
-            float4 kv = make_float4(0.f, 0.f, 0.f, 0.f), vv = kv;
-            if (j < S) {
-                kv = *reinterpret_cast<const float4 *>(QKV + (size_t)j * ld + qd + g * 128 + c);
-                vv = *reinterpret_cast<const float4 *>(QKV + (size_t)j * ld + qd + kvd + g * 128 + c);
+    __syncthreads();
+    float m[HPK], l[HPK];
+    qt_f32x4 o[HPK][8];
+#pragma unroll
+    for (int h = 0; h < HPK; h++) {
+        m[h] = -INFINITY; l[h] = 0.f;
+#pragma unroll
+        for (int d = 0; d < 8; d++) o[h][d] = zero;
+    }
+    float4 vr[8][2];
+    auto values = [&](int j0) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float *src = Vb + (size_t)min(j0 + 16 * (e >> 2) + 4 * g + (e & 3), S - 1) * ld + 8 * li;
+            vr[e][0] = *reinterpret_cast<const float4 *>(src);
+            vr[e][1] = *reinterpret_cast<const float4 *>(src + 4);
+        }
+    };
+    const int q = q0 + li, nkb = min(q0 + 15, S - 1) / 32 + 1;
+    for (int kb = wave; kb < nkb; kb += QT_PF_AW) {
+        const int j0 = 32 * kb;
+        if (HPK == 1) values(j0);
+        qt_f32x4 sc[HPK][2];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const float *src = Kb + (size_t)min(j0 + 16 * t + li, S - 1) * ld + 8 * g;
+            float4 kr[4][2];
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                kr[s][0] = *reinterpret_cast<const float4 *>(src + 32 * s);
+                kr[s][1] = *reinterpret_cast<const float4 *>(src + 32 * s + 4);
             }
-            *reinterpret_cast<float4 *>(&ks[r][c]) = kv;
-            *reinterpret_cast<float4 *>(&vs[r][c]) = vv;
+#pragma unroll
+            for (int h = 0; h < HPK; h++) sc[h][t] = zero;
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const float v[8] = {kr[s][0].x, kr[s][0].y, kr[s][0].z, kr[s][0].w, kr[s][1].x, kr[s][1].y, kr[s][1].z, kr[s][1].w};
+                qt_u32x4 kp[3], qp[3];
+                qt_planes8(v, kp, chk);
+#pragma unroll
+                for (int h = 0; h < HPK; h++) {
+#pragma unroll
+                    for (int p = 0; p < 3; p++)
+                        qp[p] = qt_lds16(sm + (h * 3 + p) * 4096 + li * 256 + 16 * ((4 * s + g) ^ li));
+                    sc[h][t] += qt_mma6(kp, qp, zero);
+                }
+            }
         }
-        __syncthreads();
-        // scores of queries rq + 16a with keys cg + 16b
-        float sc[QA][4];
-#pragma unroll
-        for (int a = 0; a < QA; a++)
-#pragma unroll
-            for (int b = 0; b < 4; b++) sc[a][b] = 0.f;
-        for (int d = 0; d < 128; d += 4) {
-            float4 qv[QA], kv[4];
-#pragma unroll
-            for (int a = 0; a < QA; a++) qv[a] = *reinterpret_cast<const float4 *>(&qs[rq + 16 * a][d]);
-#pragma unroll
-            for (int b = 0; b < 4; b++) kv[b] = *reinterpret_cast<const float4 *>(&ks[cg + 16 * b][d]);
-#pragma unroll
-            for (int a = 0; a < QA; a++)
-#pragma unroll
-                for (int b = 0; b < 4; b++)
-                    sc[a][b] = fmaf(qv[a].w, kv[b].w, fmaf(qv[a].z, kv[b].z, fmaf(qv[a].y, kv[b].y, fmaf(qv[a].x, kv[b].x, sc[a][b]))));
+        if (HPK == 2) {                                 // two heads' sums leave no room for them earlier
+            __builtin_amdgcn_sched_barrier(0);
+            values(j0);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        // causal mask (keys after the query, keys past S), block max, rescale, P
+        qt_u32x4 pp[HPK][3];
 #pragma unroll
-        for (int a = 0; a < QA; a++) {
-            const int q = q0 + rq + 16 * a;
+        for (int h = 0; h < HPK; h++) {
             float bm = -INFINITY;
 #pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const int j = j0 + cg + 16 * b;
-                sc[a][b] = (j <= q && j < S) ? sc[a][b] * scale : -INFINITY;
-                bm = fmaxf(bm, sc[a][b]);
-            }
-            bm = group_max<16>(bm);
-            const float mn = fmaxf(m[a], bm);
-            const float mr = mn == -INFINITY ? 0.f : mn;   // a query row past S has no key at all
-            const float c = expf(m[a] - mr);
-            float rs = 0.f;
+            for (int t = 0; t < 2; t++)
 #pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const float pv = expf(sc[a][b] - mr);
-                ps[rq + 16 * a][cg + 16 * b] = pv;
-                rs += pv;
-            }
-            l[a] = l[a] * c + group_sum<16>(rs);
-            m[a] = mn;
+                for (int r = 0; r < 4; r++) {
+                    const float sv = j0 + 16 * t + 4 * g + r <= q ? sc[h][t][r] * scale : -INFINITY;
+                    sc[h][t][r] = sv;
+                    bm = fmaxf(bm, sv);
+                }
+            bm = fmaxf(bm, __shfl_xor(bm, 16));
+            bm = fmaxf(bm, __shfl_xor(bm, 32));
+            const float mn = fmaxf(m[h], bm), mr = mn == -INFINITY ? 0.f : mn, alpha = expf(m[h] - mr);
+            float p8[8], rs = 0.f;
 #pragma unroll
-            for (int e = 0; e < 8; e++) o[a][e] *= c;
+            for (int e = 0; e < 8; e++) {
+                p8[e] = expf(sc[h][e >> 2][e & 3] - mr);
+                rs += p8[e];
+            }
+            rs += __shfl_xor(rs, 16);
+            rs += __shfl_xor(rs, 32);
+            l[h] = l[h] * alpha + rs;
+            m[h] = mn;
+            qt_planes8(p8, pp[h], chk);
+            float ar[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) ar[r] = __shfl(alpha, 4 * g + r);
+#pragma unroll
+            for (int d = 0; d < 8; d++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) o[h][d][r] *= ar[r];
         }
+#pragma unroll
+        for (int d = 0; d < 8; d++) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float4 f = vr[e][d >> 2];
+                v[e] = (d & 3) == 0 ? f.x : (d & 3) == 1 ? f.y : (d & 3) == 2 ? f.z : f.w;
+            }
+            qt_u32x4 vp[3];
+            qt_planes8(v, vp, chk);
+#pragma unroll
+            for (int h = 0; h < HPK; h++) o[h][d] += qt_mma6(pp[h], vp, zero);
+        }
+    }
+    // merge: the waves' maxima and sums, each wave's output scaled to the common maximum
+#pragma unroll
+    for (int h = 0; h < HPK; h++)
+        if (g == 0) { sst[0][wave][h][li] = m[h]; sst[1][wave][h][li] = l[h]; }
+    const bool serial = __syncthreads_or(chk != chk);
+    const int nw = min(nkb, QT_PF_AW);
+    if (!serial) {
+        float *os = reinterpret_cast<float *>(sm + wave * OB);
+#pragma unroll
+        for (int h = 0; h < HPK; h++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int row = 4 * g + r;
+                float M = -INFINITY;
+                for (int w = 0; w < nw; w++) M = fmaxf(M, sst[0][w][h][row]);
+                const float f = expf(sst[0][wave][h][row] - M);
+                if (wave < nw) {
+                    float *d = os + (h * 16 + row) * 128 + 8 * li;
+                    *reinterpret_cast<float4 *>(d) = make_float4(o[h][0][r] * f, o[h][1][r] * f, o[h][2][r] * f, o[h][3][r] * f);
+                    *reinterpret_cast<float4 *>(d + 4) = make_float4(o[h][4][r] * f, o[h][5][r] * f, o[h][6][r] * f, o[h][7][r] * f);
+                }
+            }
         __syncthreads();
-        // o[a][4h + e] += sum_j P[rq + 16a][j] * V[j][64h + 4cg + e]
-        for (int jj = 0; jj < 64; jj++) {
-            const float4 v0 = *reinterpret_cast<const float4 *>(&vs[jj][4 * cg]);
-            const float4 v1 = *reinterpret_cast<const float4 *>(&vs[jj][64 + 4 * cg]);
+    }
+    const size_t plane = (size_t)Sp * qd;
+    for (int u = tid; u < HPK * 16 * 32; u += QT_PF_AT) {
+        const int h = u >> 9, row = (u >> 5) & 15, c = 4 * (u & 31);
+        if (serial || q0 + row >= S) continue;
+        float M = -INFINITY, L = 0.f;
+        for (int w = 0; w < nw; w++) M = fmaxf(M, sst[0][w][h][row]);
+        qt_f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        for (int w = 0; w < nw; w++) {
+            L += sst[1][w][h][row] * expf(sst[0][w][h][row] - M);
+            v += *reinterpret_cast<const qt_f32x4 *>(sm + w * OB + ((h * 16 + row) * 128 + c) * 4);
+        }
+        const float inv = 1.0f / L;
+        const int col = (h0 + h) * 128 + c;
+        if (P) {
+            uint16_t pc[3][4];
 #pragma unroll
-            for (int a = 0; a < QA; a++) {
-                const float pv = ps[rq + 16 * a][jj];
-                o[a][0] = fmaf(pv, v0.x, o[a][0]); o[a][1] = fmaf(pv, v0.y, o[a][1]);
-                o[a][2] = fmaf(pv, v0.z, o[a][2]); o[a][3] = fmaf(pv, v0.w, o[a][3]);
-                o[a][4] = fmaf(pv, v1.x, o[a][4]); o[a][5] = fmaf(pv, v1.y, o[a][5]);
-                o[a][6] = fmaf(pv, v1.z, o[a][6]); o[a][7] = fmaf(pv, v1.w, o[a][7]);
-            }
+            for (int e = 0; e < 4; e++) qt_put_pieces(&pc[0][e], 4, __fmul_rn(v[e], inv));
+#pragma unroll
+            for (int p = 0; p < 3; p++)
+                *reinterpret_cast<uint2 *>(P + p * plane + (size_t)(q0 + row) * qd + col) =
+                    make_uint2((uint32_t)pc[p][0] | ((uint32_t)pc[p][1] << 16), (uint32_t)pc[p][2] | ((uint32_t)pc[p][3] << 16));
+        } else {
+            *reinterpret_cast<qt_f32x4 *>(A + (size_t)(q0 + row) * lda + col) = v * inv;
         }
     }
-    if (P) {
-        const int K = nh * 128;
-        const size_t plane = (size_t)Sp * K;
+    if (serial) {
+        float *out = reinterpret_cast<float *>(sm) + wave * 256;
+        for (int u = wave; u < HPK * 16; u += QT_PF_AW) {
+            const int h = u >> 4, qq = q0 + (u & 15);
+            if (qq >= S) continue;
+            pf_att_serial(QKV + (size_t)qq * ld + (h0 + h) * 128, Kb, Vb, ld, qq + 1, scale, out, out + 128, lane);
+            __builtin_amdgcn_s_waitcnt(0);
+            __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int a = 0; a < QA; a++) {
-            const int q = q0 + rq + 16 * a;
-            if (q >= S) continue;
-            const float inv = 1.0f / l[a];
-#pragma unroll
-            for (int hh = 0; hh < 2; hh++) {
-                uint16_t pc[3][4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) qt_put_pieces(&pc[0][e], 4, __fmul_rn(o[a][4 * hh + e], inv));
-                uint16_t *dst = P + (size_t)q * K + h * 128 + 64 * hh + 4 * cg;
-#pragma unroll
-                for (int p = 0; p < 3; p++)
-                    *reinterpret_cast<uint2 *>(dst + p * plane) =
-                        make_uint2((uint32_t)pc[p][0] | ((uint32_t)pc[p][1] << 16), (uint32_t)pc[p][2] | ((uint32_t)pc[p][3] << 16));
+            for (int e = 0; e < 2; e++) {
+                const size_t at = (size_t)qq * (P ? qd : lda) + (h0 + h) * 128 + 64 * e + lane;
+                if (P) qt_put_pieces(P + at, (int)plane, out[64 * e + lane]);
+                else A[at] = out[64 * e + lane];
             }
+            __builtin_amdgcn_wave_barrier();
         }
-        if (blockIdx.x == gridDim.x - 1)
-            for (int i = threadIdx.x; i < (Sp - S) * 32; i += QT_PF_WG) {
-                uint16_t *dst = P + (size_t)(S + i / 32) * K + h * 128 + 4 * (i % 32);
-#pragma unroll
-                for (int p = 0; p < 3; p++) *reinterpret_cast<uint2 *>(dst + p * plane) = make_uint2(0u, 0u);
-            }
-        return;
     }
+    if (P && qt == (int)gridDim.x - 1)
+        for (int i = tid; i < (Sp - S) * 32 * HPK; i += QT_PF_AT) {
+            uint16_t *dst = P + (size_t)(S + i / (32 * HPK)) * qd + h0 * 128 + 4 * (i % (32 * HPK));
 #pragma unroll
-    for (int a = 0; a < QA; a++) {
-        const int q = q0 + rq + 16 * a;
-        if (q >= S) continue;
-        const float inv = 1.0f / l[a];
-        float *out = A + (size_t)q * lda + h * 128;
-        *reinterpret_cast<float4 *>(out + 4 * cg) = make_float4(o[a][0] * inv, o[a][1] * inv, o[a][2] * inv, o[a][3] * inv);
-        *reinterpret_cast<float4 *>(out + 64 + 4 * cg) = make_float4(o[a][4] * inv, o[a][5] * inv, o[a][6] * inv, o[a][7] * inv);
-    }
+            for (int p = 0; p < 3; p++) *reinterpret_cast<uint2 *>(dst + p * plane) = make_uint2(0u, 0u);
+        }
 }
 
 // ---- launchers -------------------------------------------------------------------------
@@ -693,182 +804,21 @@ extern "C" hipError_t qt_launch_pf_qkv_post(float *QKV, int ld, int S, int nh, i
     return hipGetLastError();
 }
 
-// ---- causal attention on the f32 matrix cores -----------------------------------------
-// 64 queries of one head per workgroup, 16 per wave, over 64-key blocks staged in LDS (K
-// rows [key][dim]; V transposed, [dim][key]).  v_mfma_f32_16x16x4_f32 (lane l supplies
-// A[l%16][l/16] and B[l/16][l%16], receives D[4(l/16)+r][l%16]) computes the scores
-// transposed, S^T = K . Q^T, with k-step s of lane group g taking dim 32g + s: each lane
-// keeps its query's 32 dims (32g .. 32g+31) in registers and reads a key's four dims of
-// four steps as one float4.  Lane l then holds the scores of query l%16 with keys
-// 16t + 4g + r (tile t, register r) -- exactly the A operand of P.V when k-step s of tile
-// t takes key 16t + 4g + s, so the probabilities never leave the registers; the B
-// operand (4 keys of one dim) is one float4 of the transposed V.  Softmax per block as
-// in k_pf_fattn (scale, causal mask, block max, e^(s - m), running sums), the per-query
-// statistics exchanged across the four lane groups with shuffles; the P.V result rows
-// (queries 4g + r) take their rescale factors from the lanes that own those queries.
-#define QT_PF_VTP 68   // V^T row pitch (64 keys + 4: the float4 reads of a wave spread over banks)
-// P != NULL: output as the O projection's input planes, as k_pf_fattn does.
-__global__ __launch_bounds__(QT_PF_WG) __attribute__((amdgpu_waves_per_eu(2))) void k_pf_fattn_mf(
-    const float *QKV, int ld, int S, int nh, int nkv, float scale, float *A, int lda, uint16_t *P, int Sp) {
-    __shared__ __align__(16) float ks[64][QT_PF_KP];
-    __shared__ __align__(16) float vt[128][QT_PF_VTP];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, g = lane >> 4;
-    const int h = blockIdx.y, kvh = h / (nh / nkv);
-    const int q0 = blockIdx.x * 64, qw = q0 + 16 * wave, q = qw + li;
-    const int qd = nh * 128, kvd = nkv * 128;
-    float qf[32];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const float4 v = q < S ? *reinterpret_cast<const float4 *>(QKV + (size_t)q * ld + h * 128 + 32 * g + 4 * i)
-                               : make_float4(0.f, 0.f, 0.f, 0.f);
-        qf[4 * i] = v.x; qf[4 * i + 1] = v.y; qf[4 * i + 2] = v.z; qf[4 * i + 3] = v.w;
-    }
-    float m = -INFINITY, l = 0.f;           // statistics of query q (the same in the four lane groups)
-    qt_f32x4 o[8];                          // O[query 4g + r][dim 16 dt + li]
-#pragma unroll
-    for (int dt = 0; dt < 8; dt++) o[dt] = qt_f32x4{0.f, 0.f, 0.f, 0.f};
-    const int nkb = (min(q0 + 64, S) - 1) / 64 + 1;
-    // the next block's K and V rows wait in registers while the current block computes
-    // (thread t: rows t/32 + 8i, float4 column t%32, i < 8)
-    constexpr int NP = 64 * 32 / QT_PF_WG;
-    float4 pk[NP], pv[NP];
-    auto fetch = [&](int j0) {
-#pragma unroll
-        for (int i = 0; i < NP; i++) {
-            const int r = (tid >> 5) + 8 * i, c = (tid & 31) * 4, j = j0 + r;
-            pk[i] = pv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (j < S) {
-                pk[i] = *reinterpret_cast<const float4 *>(QKV + (size_t)j * ld + qd + kvh * 128 + c);
-                pv[i] = *reinterpret_cast<const float4 *>(QKV + (size_t)j * ld + qd + kvd + kvh * 128 + c);
-            }
-        }
-    };
-    fetch(0);
-    for (int kb = 0; kb < nkb; kb++) {
-        const int j0 = kb * 64;
-        __syncthreads();                                // previous block's K / V reads done
-#pragma unroll
-        for (int i = 0; i < NP; i++) {
-            const int r = (tid >> 5) + 8 * i, c = (tid & 31) * 4;
-            *reinterpret_cast<float4 *>(&ks[r][c]) = pk[i];
-            vt[c][r] = pv[i].x; vt[c + 1][r] = pv[i].y; vt[c + 2][r] = pv[i].z; vt[c + 3][r] = pv[i].w;
-        }
-        __syncthreads();
-        if (kb + 1 < nkb) fetch(j0 + 64);
-        if (j0 > qw + 15) continue;                     // every query of this wave precedes the block (wave-uniform)
-        qt_f32x4 st[4];
-#pragma unroll
-        for (int t = 0; t < 4; t++) st[t] = qt_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s4 = 0; s4 < 8; s4++)
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const float4 kv = *reinterpret_cast<const float4 *>(&ks[16 * t + li][32 * g + 4 * s4]);
-                st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.x, qf[4 * s4], st[t], 0, 0, 0);
-                st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.y, qf[4 * s4 + 1], st[t], 0, 0, 0);
-                st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.z, qf[4 * s4 + 2], st[t], 0, 0, 0);
-                st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.w, qf[4 * s4 + 3], st[t], 0, 0, 0);
-            }
-        float bm = -INFINITY;
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int j = j0 + 16 * t + 4 * g + r;
-                const float sv = (j <= q && j < S) ? st[t][r] * scale : -INFINITY;
-                st[t][r] = sv;
-                bm = fmaxf(bm, sv);
-            }
-        bm = fmaxf(bm, __shfl_xor(bm, 16));
-        bm = fmaxf(bm, __shfl_xor(bm, 32));
-        const float mn = fmaxf(m, bm);
-        const float mr = mn == -INFINITY ? 0.f : mn;     // a query row past S has no key at all
-        const float alpha = expf(m - mr);
-        float rs = 0.f;
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const float pv = expf(st[t][r] - mr);
-                st[t][r] = pv;
-                rs += pv;
-            }
-        rs += __shfl_xor(rs, 16);
-        rs += __shfl_xor(rs, 32);
-        l = l * alpha + rs;
-        m = mn;
-        float ar[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) ar[r] = __shfl(alpha, 4 * g + r);
-#pragma unroll
-        for (int dt = 0; dt < 8; dt++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) o[dt][r] *= ar[r];
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-            for (int dt = 0; dt < 8; dt++) {
-                const float4 vv = *reinterpret_cast<const float4 *>(&vt[16 * dt + li][16 * t + 4 * g]);
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(st[t][0], vv.x, o[dt], 0, 0, 0);
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(st[t][1], vv.y, o[dt], 0, 0, 0);
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(st[t][2], vv.z, o[dt], 0, 0, 0);
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(st[t][3], vv.w, o[dt], 0, 0, 0);
-            }
-    }
-    float lr[4];
-#pragma unroll
-    for (int r = 0; r < 4; r++) lr[r] = 1.0f / __shfl(l, 4 * g + r);
-    if (P) {
-        const size_t plane = (size_t)Sp * qd;
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int qq = qw + 4 * g + r;
-            if (qq >= S) continue;
-#pragma unroll
-            for (int dt = 0; dt < 8; dt++)
-                qt_put_pieces(P + (size_t)qq * qd + h * 128 + 16 * dt + li, (int)plane, __fmul_rn(o[dt][r], lr[r]));
-        }
-        if (blockIdx.x == gridDim.x - 1)
-            for (int i = tid; i < (Sp - S) * 32; i += QT_PF_WG) {
-                uint16_t *dst = P + (size_t)(S + i / 32) * qd + h * 128 + 4 * (i % 32);
-#pragma unroll
-                for (int p = 0; p < 3; p++) *reinterpret_cast<uint2 *>(dst + p * plane) = make_uint2(0u, 0u);
-            }
-        return;
-    }
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int qq = qw + 4 * g + r;
-        if (qq >= S) continue;
-#pragma unroll
-        for (int dt = 0; dt < 8; dt++) A[(size_t)qq * lda + h * 128 + 16 * dt + li] = o[dt][r] * lr[r];
-    }
-}
-
 // P != NULL (with planes): the output is written as the O projection's input planes
 // (rows padded to qt_pf_spad(S)) and *planes = 1; otherwise A gets the f32 rows.
 static hipError_t pf_attn(const float *QKV, int ld, int S, int nh, int nkv, float scale, float *A, int lda,
                           uint16_t *P, int *planes, hipStream_t st) {
     if (S <= 0 || nh <= 0 || nkv <= 0 || nh % nkv) return hipErrorInvalidValue;
-    if (planes) *planes = 0;
-    // the matrix-core kernel where it has at least 64 workgroups (1.7B prefill, 512
-    // positions: 8.37 ms against 8.72 with the VALU kernel; at 128 positions, 32
-    // workgroups, 3.84 against 3.77), else the VALU kernel with 64-, 32- or 16-query
-    // workgroups, the largest that still fills the CUs
     const int Sp = qt_pf_spad(S);
-    if (P && planes) *planes = 1;
-    else P = NULL;
-    if ((long long)((S + 63) / 64) * nh >= 64) {
-        hipLaunchKernelGGL(k_pf_fattn_mf, dim3((S + 63) / 64, nh), dim3(QT_PF_WG), 0, st, QKV, ld, S, nh, nkv, scale, A, lda,
-                           P, Sp);
-        return hipGetLastError();
-    }
-    if ((long long)((S + 63) / 64) * nh >= 256)
-        hipLaunchKernelGGL(k_pf_fattn<4>, dim3((S + 63) / 64, nh), dim3(QT_PF_WG), 0, st, QKV, ld, S, nh, nkv, scale, A, lda, P, Sp);
-    else if ((long long)((S + 31) / 32) * nh >= 256)
-        hipLaunchKernelGGL(k_pf_fattn<2>, dim3((S + 31) / 32, nh), dim3(QT_PF_WG), 0, st, QKV, ld, S, nh, nkv, scale, A, lda, P, Sp);
+    if (planes) *planes = P != NULL;
+    if (!planes) P = NULL;
+    // One head a workgroup while every such workgroup has a CU of its own, then two heads of a kv
+    // head, which split its keys and values once (16 heads: 8.8 us against 11.9 at 128 positions, 13.4
+    // against 17.3 at 256, then 28.2 against 21.1 at 384 and 40.1 against 26.7 at 512)
+    if ((nh / nkv) % 2 == 0 && (long long)((S + 15) / 16) * nh > 256)
+        hipLaunchKernelGGL(k_pf_att<2>, dim3((S + 15) / 16, nh / 2), dim3(QT_PF_AT), 0, st, QKV, ld, S, nh, nkv, scale, A, lda, P, Sp);
     else
-        hipLaunchKernelGGL(k_pf_fattn<1>, dim3((S + 15) / 16, nh), dim3(QT_PF_WG), 0, st, QKV, ld, S, nh, nkv, scale, A, lda, P, Sp);
+        hipLaunchKernelGGL(k_pf_att<1>, dim3((S + 15) / 16, nh), dim3(QT_PF_AT), 0, st, QKV, ld, S, nh, nkv, scale, A, lda, P, Sp);
     return hipGetLastError();
 }
 

@@ -23,7 +23,7 @@
 // and the six largest of the nine plane products of an f32 product are accumulated in f32
 // (the rest are under 2^-25 of it, below its own rounding).  The weights' planes are made
 // once, when the decoder is loaded; an input's on its way into LDS.
-#include "qt_attn_mf.h"
+#include "qt_planes.h"
 
 #define SD_WG 256
 #define SD_MAXTAP 8
@@ -38,32 +38,6 @@ enum { SD_EPI_BIAS = 1, SD_EPI_GELU = 2, SD_EPI_CSCALE = 4, SD_EPI_RESID = 8, SD
 // stored as its three planes, 64 lanes x 16 bytes each (3 KiB), in the order that a
 // workgroup walks: [K slice][tap][phase][channel tile].  K and the channels of a phase are
 // padded with zeros to 32 and 16.
-// An f32 value v is the sum of its planes exactly: v rounded to bf16, the rest rounded to
-// bf16, and what then remains (at most 8 significant bits).
-__device__ __forceinline__ uint32_t sd_bf16x2(float a, float b) {
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{a, b}), b2));
-}
-__device__ __forceinline__ float sd_lo(uint32_t u) { return __uint_as_float(u << 16); }
-__device__ __forceinline__ float sd_hi(uint32_t u) { return __uint_as_float(u & 0xFFFF0000u); }
-
-// the planes of 8 values; chk becomes NaN when a value has none (infinite, NaN, or past
-// bf16's range after rounding) and stays as it is otherwise
-__device__ __forceinline__ void sd_planes8(const float (&v)[8], qt_u32x4 (&p)[3], float &chk) {
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const float a = v[2 * i], b = v[2 * i + 1];
-        const uint32_t h = sd_bf16x2(a, b);
-        const float ra = a - sd_lo(h), rb = b - sd_hi(h);
-        const uint32_t m = sd_bf16x2(ra, rb);
-        chk = fmaf(ra, 0.f, fmaf(rb, 0.f, chk));
-        p[0][i] = h;
-        p[1][i] = m;
-        p[2][i] = sd_bf16x2(ra - sd_lo(m), rb - sd_hi(m));
-    }
-}
-
 // One tensor of the reference's layout (element [n][k][column] at n * sn + k * sk + column * sc)
 // into channels [n0, n0 + nn) and k [k0, k0 + kk) of the packed weights (n0, k0: whole tiles).
 // Tap p of phase z is column p (stride 0: a conv or linear layer) or z + p * stride (zero past the
@@ -88,7 +62,7 @@ __global__ __launch_bounds__(SD_WG) void k_sd_pack(SdPackArgs a) {
     for (int i = 0; i < 8; i++)
         v[i] = (n < a.nn && k + i < a.kk && col < a.cols) ? a.src[n * a.sn + (k + i) * a.sk + col * a.sc] : 0.f;
     qt_u32x4 pl[3];
-    sd_planes8(v, pl, chk);
+    qt_planes8(v, pl, chk);
     if (chk != chk) *a.bad = 1;
     uint16_t *d = a.dst + ((((size_t)(a.k0 / 32 + kc) * a.ntap + p) * a.phases + z) * a.tiles + a.n0 / 16 + j) * 1536 + 8 * lane;
 #pragma unroll
@@ -168,17 +142,6 @@ __device__ __forceinline__ void sd_epilogue(const SdGemmArgs &a, int t, int z, i
     *reinterpret_cast<qt_f32x4 *>(a.Y + o) = v;
 }
 
-// The six plane products that an f32 product needs (the other three are below 2^-25 of it),
-// the smallest first.
-__device__ __forceinline__ qt_f32x4 sd_mma6(const qt_u32x4 (&w)[3], const qt_u32x4 (&x)[3], qt_f32x4 c) {
-    c = qt_mfma_bf16(w[0], x[2], c);
-    c = qt_mfma_bf16(w[2], x[0], c);
-    c = qt_mfma_bf16(w[1], x[1], c);
-    c = qt_mfma_bf16(w[0], x[1], c);
-    c = qt_mfma_bf16(w[1], x[0], c);
-    return qt_mfma_bf16(w[0], x[0], c);
-}
-
 // Where a layer has at least SD_GROUP_SLICES slices of 32 k (512), its slices are SD_GROUPS
 // equal runs whose sums are added in order.  That is a property of the layer alone, so a
 // small call can give the runs to different waves and still return the bits of a large one.
@@ -236,7 +199,7 @@ __global__ __launch_bounds__(SD_WG) __attribute__((amdgpu_waves_per_eu(2))) void
 #pragma unroll
             for (int e = 0; e < 8; e++) v[e] = __uint_as_float(__float_as_uint(st[i][e]) & m);
             qt_u32x4 pl[3];
-            sd_planes8(v, pl, chk);
+            qt_planes8(v, pl, chk);
             uint8_t *d = xs + buf * BUF + row * 64 + sd_unit(row, u & 3);
 #pragma unroll
             for (int p = 0; p < 3; p++) *reinterpret_cast<qt_u32x4 *>(d + p * PS) = pl[p];
@@ -278,7 +241,7 @@ __global__ __launch_bounds__(SD_WG) __attribute__((amdgpu_waves_per_eu(2))) void
 #pragma unroll
                 for (int q = 0; q < 3; q++) x[q] = qt_lds16(x0 + i * 1024 + q * PS);
 #pragma unroll
-                for (int j = 0; j < NT; j++) acc[j][i] = sd_mma6(w[j], x, acc[j][i]);
+                for (int j = 0; j < NT; j++) acc[j][i] = qt_mma6(w[j], x, acc[j][i]);
             }
 #pragma unroll
             for (int j = 0; j < NT; j++)
@@ -377,9 +340,9 @@ __global__ __launch_bounds__(64 * SD_GROUPS) void k_sd_split(SdGemmArgs a) {
 #pragma unroll
                     for (int e = 0; e < 8; e++) v[e] = __uint_as_float(__float_as_uint(v[e]) & m);
                     qt_u32x4 pl[3];
-                    sd_planes8(v, pl, chk);
+                    qt_planes8(v, pl, chk);
 #pragma unroll
-                    for (int j = 0; j < NT; j++) acc[j][i] = sd_mma6(w[d][j], pl, acc[j][i]);
+                    for (int j = 0; j < NT; j++) acc[j][i] = qt_mma6(w[d][j], pl, acc[j][i]);
                 }
             }
             fetch(min(it + d + D, i1 - 1), d);

@@ -63,9 +63,8 @@ def test_op_prefill_gemm_planes_are_exact():
 
 @pytest.mark.parametrize("S,nh,nkv", [(1, 16, 8), (37, 16, 8), (100, 4, 2), (300, 16, 8), (1000, 16, 8)])
 def test_op_prefill_attention(oracle, S, nh, nkv):
-    """The tiled causal attention against the oracle's f32 attention (qwen_causal_attention
-    restated): the VALU kernel's 16-query workgroups (S = 1, 37, 100) and the matrix-core
-    kernel (S = 300, 1000)."""
+    """The causal attention against the oracle's f32 attention (qwen_causal_attention restated):
+    one head a workgroup (S = 1, 37, 100) and two (S = 300, 1000)."""
     print(f"[case] prefill attention S={S} nh={nh} nkv={nkv}", flush=True)
     rng = np.random.default_rng(S + nh)
     ld = (nh + 2 * nkv) * 128
@@ -91,6 +90,54 @@ def _tiny_talker(prec_code, quantize_to=-1, kv_max=64):
 def _kv_close(a, b):
     d = np.abs(synth.bf16_to_f32(a).astype(np.float64) - synth.bf16_to_f32(b))
     return (a != b).mean() < 0.02 and d.max() < 0.05
+
+
+def _attention64(qkv, S, nh, nkv):
+    x = qkv.astype(np.float64).reshape(S, nh + 2 * nkv, 128)
+    out = np.empty((S, nh, 128))
+    with np.errstate(invalid="ignore", over="ignore"):
+        for h in range(nh):
+            q, k, v = x[:, h], x[:, nh + h // (nh // nkv)], x[:, nh + nkv + h // (nh // nkv)]
+            for i in range(S):
+                s = (k[:i + 1] * q[i]).sum(1) / np.sqrt(128.0)
+                m = np.fmax.reduce(s)
+                p = np.exp(s - (m if np.isfinite(m) else 0.0 if m == -np.inf else m))
+                out[i, h] = (p[:, None] * v[:i + 1]).sum(0) / p.sum()
+    return out.reshape(S, nh * 128)
+
+
+def _attention_dev(qkv, S, nh, nkv):
+    out = np.empty((S, nh * 128), np.float32)
+    hip.check(hip.lib().qwen_hip_op_prefill_attention(out.ctypes.data, qkv.ctypes.data, S, nh, nkv,
+                                                      np.float32(1.0 / np.sqrt(128.0))), "prefill_attention")
+    return out
+
+
+@pytest.mark.parametrize("S,nh,nkv", [(1, 2, 1), (15, 2, 2), (16, 4, 1), (17, 3, 1), (33, 6, 2), (257, 2, 1), (290, 8, 2)])
+def test_op_prefill_attention_edges_vs_f64(S, nh, nkv):
+    """Query tiles of 16, key blocks of 32 over eight waves, one, two or an odd number of heads per
+    kv head, scores spread over +-40.  Bound: the f32 rounding of a 128-term score of that size
+    (40 x 2^-24 x sqrt(128)) moves a probability by the same relative amount."""
+    rng = np.random.default_rng(S + nh)
+    qkv = rng.standard_normal((S, (nh + 2 * nkv) * 128)).astype(np.float32)
+    qkv[:, :nh * 128] *= 4.0
+    err = np.abs(_attention_dev(qkv, S, nh, nkv) - _attention64(qkv, S, nh, nkv)).max()
+    assert err < 4 * 40 * np.sqrt(128) * 2.0 ** -24, err
+
+
+def test_op_prefill_attention_non_finite():
+    """An infinite or NaN key, value or query reaches the queries that see it and no others."""
+    S, nh, nkv = 70, 4, 2
+    rng = np.random.default_rng(5)
+    qkv = rng.standard_normal((S, (nh + 2 * nkv) * 128)).astype(np.float32)
+    clean = qkv.copy()
+    qkv[40, (nh + nkv) * 128 + 3] = np.inf        # a value of kv head 0
+    qkv[33, (nh + 1) * 128 + 9] = np.nan          # a key of kv head 1
+    y, want = _attention_dev(qkv, S, nh, nkv), _attention_dev(clean, S, nh, nkv)
+    assert np.allclose(y[:33], want[:33], rtol=1e-6, atol=1e-6)
+    assert np.allclose(y[33:40, :256], want[33:40, :256], rtol=1e-6, atol=1e-6)
+    assert np.isinf(y[40:, [3, 131]]).all() and np.isfinite(np.delete(y[40:, :256], [3, 131], 1)).all()
+    assert np.isnan(y[33:, 256:]).all()
 
 
 @pytest.mark.parametrize("quant", [-1, hip.INT8])
@@ -137,8 +184,7 @@ def test_prefill_async_replays_reproduce_the_prefill():
 @pytest.mark.parametrize("name,seq", [("mini", 100), ("mini17", 40), ("mini", 240)])
 def test_prefill_matches_oracle_layer_shapes(oracle, name, seq):
     """The 0.6B / 1.7B layer shapes (2 layers) against the oracle prefill, then one decode
-    step from each side's KV.  100 and 40 positions run the VALU attention, 240 the
-    matrix-core one (64 workgroups), with 16 padding rows in the O projection's planes."""
+    step from each side's KV.  240 positions leave 16 padding rows in the O projection's planes."""
     from oracle.oracle import talker_from_tensors
     print(f"[case] prefill oracle {name} seq={seq}", flush=True)
     d, shape, t = model_dir(name)
