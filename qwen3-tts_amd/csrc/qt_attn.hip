@@ -20,7 +20,7 @@
 // overlaps the prologue; the key at `pos` (appended by this workgroup) is not read from
 // memory but taken from LDS (knew/vnew).  The merging workgroup reuses that LDS for the
 // chunk partials, so a workgroup needs ~72 KB and two fit on a CU.
-#include "qt_attn_mf.h"
+#include "qt_planes.h"
 
 #define QT_HD 128
 #define QT_CH_MAX 256
@@ -45,6 +45,8 @@ struct QtAttnArgs {
     // partials and counters; d_pos + z is its position (batched step)
     long long q_bs, kv_bs, out_bs, part_bs;
     int min_chunk;           // chunks hold at least this many keys (0: ceil(L/G) rounded to 16)
+    uint16_t *planes;        // batched, may be NULL: the output as planes in operand order (row z of
+    int row_tiles;           // row_tiles tiles; qt_frag_at) instead of rows of out
     int onepass;             // !BATCH, chunks <= 512 keys: one softmax over the chunk under its
                              // maximum (qt_attn_mf.h) instead of a running state across blocks
 };
@@ -87,7 +89,8 @@ __device__ __forceinline__ void qt_lds_copy16(const void *src, void *dst) {
 // no workgroup barrier in the key loop, and the four wave states are merged at the end;
 // !BATCH keeps the arithmetic order of the fused step's attention phase, which it must
 // match bit for bit (waves share each 128-key block: scores, barrier, P.V per 32 dims).
-template <int HPK, bool PREP, bool BATCH, bool ONEPASS>
+// PL: the output goes to planes.
+template <int HPK, bool PREP, bool BATCH, bool ONEPASS, bool PL = false>
 __global__ __launch_bounds__(QT_WG) void k_attn(QtAttnArgs a) {
     static_assert(!(BATCH && ONEPASS), "one-pass chunks are single-stream");
     const int z = BATCH ? blockIdx.y : blockIdx.z;
@@ -376,6 +379,10 @@ __global__ __launch_bounds__(QT_WG) void k_attn(QtAttnArgs a) {
         qt_att_pv_n<HPK>((nk + 31) >> 5, &pp[0][0], KVB, &ml[0][0][0], s_v, 32 * wave, lane, o, M, l);
         qt_att_run_add(run, o, M, l);
     }
+    auto put = [&](int k, float v) {
+        if constexpr (PL) qt_put_pieces(a.planes + qt_frag_at(a.row_tiles, z, k), 512, v);
+        else a.out[k] = v;
+    };
     // lane: head pg, dims 32*wave + sub and + 16
     const int od = 32 * wave + sub;
 
@@ -383,8 +390,8 @@ __global__ __launch_bounds__(QT_WG) void k_attn(QtAttnArgs a) {
     if (nch == 1) {
         if (pg < HPK) {
             const float r = 1.0f / run.l;
-            a.out[(g * HPK + pg) * QT_HD + od] = run.o[0] * r;
-            a.out[(g * HPK + pg) * QT_HD + od + 16] = run.o[1] * r;
+            put((g * HPK + pg) * QT_HD + od, run.o[0] * r);
+            put((g * HPK + pg) * QT_HD + od + 16, run.o[1] * r);
         }
         return;
     }
@@ -436,7 +443,7 @@ __global__ __launch_bounds__(QT_WG) void k_attn(QtAttnArgs a) {
                 Lsum = fmaf(pr[1], f, Lsum);
                 V = fmaf(pr[2 + d], f, V);
             }
-            a.out[(g * HPK + h) * QT_HD + d] = V * (1.0f / Lsum);
+            put((g * HPK + h) * QT_HD + d, V * (1.0f / Lsum));
         }
     } else {
         const int half = lane >> 5, cc = lane & 31;
@@ -460,7 +467,8 @@ static hipError_t attn_launch(const QtAttnArgs &a, int prep, int head_dim, int G
     const bool batch = a.min_chunk > 0;
     const dim3 grid = batch ? dim3(a.n_kv, nz, G) : dim3(G, a.n_kv, nz);
 #define QT_ATT_CASE(H) \
-    if (batch && prep) hipLaunchKernelGGL((k_attn<H, true, true, false>), grid, dim3(QT_WG), 0, st, a); \
+    if (batch && prep && a.planes) hipLaunchKernelGGL((k_attn<H, true, true, false, true>), grid, dim3(QT_WG), 0, st, a); \
+    else if (batch && prep) hipLaunchKernelGGL((k_attn<H, true, true, false>), grid, dim3(QT_WG), 0, st, a); \
     else if (a.onepass && prep) hipLaunchKernelGGL((k_attn<H, true, false, true>), grid, dim3(QT_WG), 0, st, a); \
     else if (a.onepass) hipLaunchKernelGGL((k_attn<H, false, false, true>), grid, dim3(QT_WG), 0, st, a); \
     else if (prep) hipLaunchKernelGGL((k_attn<H, true, false, false>), grid, dim3(QT_WG), 0, st, a); \
@@ -484,6 +492,7 @@ extern "C" hipError_t qt_launch_attn(int prep, const float *q, const float *qn, 
     a.K = K; a.V = V; a.pos_stride = pos_stride; a.head_stride = head_stride;
     a.n_heads = n_heads; a.n_kv = n_kv; a.scale = scale; a.part = part; a.cnt = cnt; a.out = out;
     a.q_bs = a.kv_bs = a.out_bs = a.part_bs = 0;
+    a.planes = NULL; a.row_tiles = 0;
     a.min_chunk = 0;
     a.onepass = 0;
     return attn_launch(a, prep, head_dim, G, 1, st);
@@ -502,6 +511,7 @@ extern "C" hipError_t qt_launch_attn_onepass(int prep, const float *q, const flo
     a.K = K; a.V = V; a.pos_stride = pos_stride; a.head_stride = head_stride;
     a.n_heads = n_heads; a.n_kv = n_kv; a.scale = scale; a.part = part; a.cnt = cnt; a.out = out;
     a.q_bs = a.kv_bs = a.out_bs = a.part_bs = 0;
+    a.planes = NULL; a.row_tiles = 0;
     a.min_chunk = 0;
     a.onepass = 1;
     return attn_launch(a, prep, head_dim, G, 1, st);
@@ -509,7 +519,7 @@ extern "C" hipError_t qt_launch_attn_onepass(int prep, const float *q, const flo
 
 // B independent streams in one launch (the batched step): stream z uses q + z*q_bs,
 // K/V + z*kv_bs (its own cache), position d_pos[z], partials part + z*part_bs, counters
-// cnt + z*n_kv, output out + z*out_bs.  Ragged positions are fine: each stream's chunks
+// cnt + z*n_kv, output out + z*out_bs, or, with planes, row z of planes in operand order.  Ragged positions are fine: each stream's chunks
 // follow its own length.  Chunks hold at least QT_B_MIN_CHUNK keys: short streams use few
 // workgroups, fewer partials are merged, and each wave streams a dozen tiles; throughput,
 // not single-stream latency, is what the batch needs.  Measured on the whole batched step
@@ -524,8 +534,9 @@ extern "C" hipError_t qt_launch_attn_b(const float *q, long long q_bs, const flo
                                        uint16_t *K, uint16_t *V, long long kv_bs, long long pos_stride,
                                        long long head_stride, int n_heads, int n_kv, int head_dim, float scale,
                                        float *part, long long part_bs, unsigned *cnt, int G, float *out,
-                                       long long out_bs, int B, hipStream_t st) {
+                                       long long out_bs, uint16_t *planes, int B, hipStream_t st) {
     QtAttnArgs a;
+    a.planes = planes; a.row_tiles = (B + 15) / 16;
     a.q = q; a.qn = qn; a.kn = kn; a.rc = rc; a.rs = rs; a.eps = eps; a.d_pos = d_pos; a.Lval = 0;
     a.K = K; a.V = V; a.pos_stride = pos_stride; a.head_stride = head_stride;
     a.n_heads = n_heads; a.n_kv = n_kv; a.scale = scale; a.part = part; a.cnt = cnt; a.out = out;

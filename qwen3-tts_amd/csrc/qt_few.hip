@@ -1,0 +1,216 @@
+// qt_few.hip — bf16 projections of a few rows (the batched step's streams, a short prompt's
+// positions: at most 64) on gfx950.
+//
+// Y = X . W^T with W bf16 [N][K] as stored and X f32, as the exact products of qt_prefill.hip:
+// each activation is the sum of three bf16 planes, a plane times a weight is exact in f32, and
+// the matrix cores sum in f32.  Such a product is a stream of the weights, and what it costs
+// beyond that is latency: a launch is done in one pass, with nothing summed by another one.
+//
+// 0.6B, 28 layers: six streams 1.79 -> 1.08 ms a step; 45 positions 1.83 -> 1.47 ms.
+//
+//   * a workgroup owns 16 NT weight rows for all of K; its eight waves take an eighth of K each
+//     and their sums meet in LDS;
+//   * the activations come as planes in operand order (qt_frag_at), written so by whoever
+//     made them;
+//   * RMSNorm is applied around the product: the planes are those of x * gain, each maker of
+//     16 columns of x leaves the sum of their squares (one float a row), and the consumer
+//     scales its sums by 1/rms: the row's statistic needs no launch of its own.
+#include "qt_planes.h"
+
+#define QF_W 8                   // waves of a workgroup, and parts of K
+#define QF_T (64 * QF_W)
+#define QF_ROWS 64               // rows at most
+#define QF_PART 256              // partial sums of squares at most (hidden <= 4096)
+
+// (the values of qt_launch.h, which the .hip sources do not include)
+enum { QF_STORE = 0, QF_RESID = 1, QF_SWIGLU = 2 };
+
+struct QtFewArgs {
+    const uint16_t *W, *P;       // weights [N][K]; the input's planes
+    int N, K, S, RT;             // RT: row tiles of the planes
+    const float *ssp; int np;    // STORE, SWIGLU: the rows' partial sums of squares [row][np] (the input is normed)
+    float eps;
+    float *Y; int ldy;           // STORE: Y = v; RESID: Y += v
+    const float *gain;           // RESID with Pout: the next norm's gain
+    uint16_t *Pout; float *sspo; // RESID (may be NULL): planes of Y * gain and its partial sums; SWIGLU: planes of h
+};
+
+// planes of four neighbouring values (columns k..k+3 of a row, k a multiple of 4)
+__device__ __forceinline__ void qf_put4(uint16_t *P, int RT, int row, int k, qt_f32x4 v) {
+    uint16_t pc[3][4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) qt_put_pieces(&pc[0][e], 4, v[e]);
+    uint16_t *d = P + qt_frag_at(RT, row, k);
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+        *reinterpret_cast<uint2 *>(d + 512 * p) =
+            make_uint2((uint32_t)pc[p][0] | ((uint32_t)pc[p][1] << 16), (uint32_t)pc[p][2] | ((uint32_t)pc[p][3] << 16));
+}
+
+// A workgroup computes 16 NT weight rows for 16 activation rows; each wave has D slices of 32 k of
+// both in flight (all of its eighth of K where the registers hold it: one memory latency).
+template <int NT, int D, int EPI>
+__global__ __launch_bounds__(QF_T) void k_few(QtFewArgs a) {
+    __shared__ __align__(16) qt_f32x4 part[QF_W][NT][64];
+    __shared__ float s_inv[16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, kg = lane >> 4;
+    const int n0 = blockIdx.x * 16 * NT, rt = blockIdx.y, ns = a.K / 32;
+    const int s0 = ns * wave / QF_W, s1 = ns * (wave + 1) / QF_W;
+    // what the epilogue needs is asked for first: the rows' partial sums of squares (16 threads a
+    // row), and, in the waves that finish a tile, the residual and the next gain
+    constexpr bool NORM = EPI != QF_RESID;
+    qt_f32x4 sv[QF_PART / 64];
+    if (NORM) {
+        const float *ss = a.ssp + (size_t)min(16 * rt + ((tid >> 4) & 15), a.S - 1) * a.np;
+#pragma unroll
+        for (int i = 0; i < QF_PART / 64; i++) sv[i] = *reinterpret_cast<const qt_f32x4 *>(ss + min(64 * i + 4 * (tid & 15), a.np - 4));
+    }
+    const int row = 16 * rt + li, n = n0 + 16 * wave + 4 * kg;       // the output of a finishing wave
+    const bool mine = wave < NT && row < a.S;
+    qt_f32x4 old = {0.f, 0.f, 0.f, 0.f}, gn = old;
+    if (EPI == QF_RESID && mine) {
+        old = *reinterpret_cast<const qt_f32x4 *>(a.Y + (size_t)row * a.ldy + n);
+        if (a.Pout) gn = *reinterpret_cast<const qt_f32x4 *>(a.gain + n);
+    }
+    // rows past S repeat the last one: nothing more is read for them
+    const uint16_t *wp[NT], *xp = a.P + (size_t)rt * 1536 + 8 * (min(li, a.S - 1 - 16 * rt) + 16 * kg);
+#pragma unroll
+    for (int j = 0; j < NT; j++) wp[j] = a.W + (size_t)(n0 + 16 * j + li) * a.K + 8 * kg;
+    qt_u32x4 w[D][NT], x[D][3];
+    const size_t xs = (size_t)a.RT * 1536;
+    auto fetch = [&](int s, int d) {
+#pragma unroll
+        for (int j = 0; j < NT; j++) w[d][j] = *reinterpret_cast<const qt_u32x4 *>(wp[j] + 32 * s);
+#pragma unroll
+        for (int p = 0; p < 3; p++) x[d][p] = *reinterpret_cast<const qt_u32x4 *>(xp + s * xs + 512 * p);
+    };
+    qt_f32x4 acc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) acc[j] = qt_f32x4{0.f, 0.f, 0.f, 0.f};
+    auto mul = [&](int d) {
+#pragma unroll
+        for (int p = 0; p < 3; p++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) acc[j] = qt_mfma_bf16(w[d][j], x[d][2 - p], acc[j]);
+    };
+    // loads past the wave's last slice repeat it: no load is behind a branch, so that the waits count them
+    const int last = max(s1 - 1, 0);
+#pragma unroll
+    for (int d = 0; d < D; d++) fetch(min(s0 + d, last), d);
+    int s = s0;
+    for (; s + D < s1; s += D) {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            mul(d);
+            fetch(min(s + d + D, last), d);
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < D; d++)
+        if (s + d < s1) mul(d);
+#pragma unroll
+    for (int j = 0; j < NT; j++) part[wave][j][lane] = acc[j];
+    if (NORM) {
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < QF_PART / 64; i++) ss += 64 * i + 4 * (tid & 15) < a.np ? (sv[i][0] + sv[i][1]) + (sv[i][2] + sv[i][3]) : 0.f;
+        ss = group_sum<16>(ss);
+        if (tid < 256 && (tid & 15) == 0) s_inv[tid >> 4] = 1.0f / sqrtf(ss / (float)a.K + a.eps);
+    }
+    __syncthreads();
+    if (!mine) return;
+    qt_f32x4 v = part[0][wave][lane];
+#pragma unroll
+    for (int g = 1; g < QF_W; g++) v += part[g][wave][lane];
+    if (NORM) v *= s_inv[li];
+    if (EPI == QF_SWIGLU) {                        // rows 2i, 2i + 1 of W are gate_i, up_i
+        // rounded products, split as they are
+        const float h0 = __fmul_rn(v[0] / (1.0f + expf(-v[0])), v[1]), h1 = __fmul_rn(v[2] / (1.0f + expf(-v[2])), v[3]);
+        uint16_t pc[3][2];
+        qt_put_pieces(&pc[0][0], 2, h0);
+        qt_put_pieces(&pc[0][1], 2, h1);
+        uint16_t *d = a.Pout + qt_frag_at(a.RT, row, n >> 1);
+#pragma unroll
+        for (int p = 0; p < 3; p++) *reinterpret_cast<uint32_t *>(d + 512 * p) = (uint32_t)pc[p][0] | ((uint32_t)pc[p][1] << 16);
+    } else if (EPI == QF_RESID) {
+        v = old + v;
+        *reinterpret_cast<qt_f32x4 *>(a.Y + (size_t)row * a.ldy + n) = v;
+        if (a.Pout) {
+            qf_put4(a.Pout, a.RT, row, n, v * gn);
+            float sq = fmaf(v[3], v[3], fmaf(v[2], v[2], fmaf(v[1], v[1], v[0] * v[0])));
+            sq += __shfl_xor(sq, 16);              // a row's four lanes are all in the tile or all past S
+            sq += __shfl_xor(sq, 32);
+            if (kg == 0) a.sspo[(size_t)row * (a.N / 16) + blockIdx.x * NT + wave] = sq;
+        }
+    } else {
+        *reinterpret_cast<qt_f32x4 *>(a.Y + (size_t)row * a.ldy + n) = v;
+    }
+}
+
+// planes of x * gain and each row's sum of squares (as QF_FIRST partial sums, all but one zero)
+#define QF_FIRST 4
+__global__ __launch_bounds__(256) void k_few_planes(const float *X, int ldx, int K, int RT, const float *gain, uint16_t *P,
+                                                    float *ssp) {
+    __shared__ float red[QT_WAVES];
+    const int row = blockIdx.x;
+    const float *x = X + (size_t)row * ldx;
+    float ss = 0.f;
+    for (int k = 4 * threadIdx.x; k < K; k += 1024) {
+        qt_f32x4 v = *reinterpret_cast<const qt_f32x4 *>(x + k);
+        ss = fmaf(v[3], v[3], fmaf(v[2], v[2], fmaf(v[1], v[1], fmaf(v[0], v[0], ss))));
+        qf_put4(P, RT, row, k, v * *reinterpret_cast<const qt_f32x4 *>(gain + k));
+    }
+    ss = block_sum(ss, red);
+    if (threadIdx.x < QF_FIRST) ssp[row * QF_FIRST + threadIdx.x] = threadIdx.x ? 0.f : ss;
+}
+
+// ---- launchers ----------------------------------------------------------------------------
+// The rows fit while the widest projection has few enough tiles that its workgroups (of up to four)
+// run in about one round; with more rounds of one latency each the prefill's tiles are the faster ones.
+// 28 layers, 0.6B / 1.7B: 16 rows 1.23 against 1.75 / 1.80 against 2.21 ms, 32 rows - / 2.09 against
+// 2.32, 64 rows 1.48 against 1.93 / 2.80 against 2.55 (1.7B: 32 rows are the most).
+extern "C" int qt_few_ok(int S, int H, int F, int qd, int qkvr) {
+    return S >= 1 && S <= QF_ROWS && H % 64 == 0 && F % 64 == 0 && qd % 64 == 0 && qkvr % 64 == 0 && H / 16 <= QF_PART &&
+           (long long)(F / 8 > qkvr / 16 ? F / 8 : qkvr / 16) * ((S + 15) / 16) <= 1536;
+}
+extern "C" int qt_few_first(void) { return QF_FIRST; }
+extern "C" size_t qt_few_planes_elems(int S, int K) { return (size_t)((S + 15) / 16) * 16 * K * 3; }
+
+extern "C" hipError_t qt_launch_few_planes(const float *X, int ldx, int S, int K, const float *gain, uint16_t *P, float *ssp,
+                                           hipStream_t st) {
+    if (!X || !P || !gain || !ssp || S < 1 || S > QF_ROWS || K < 64 || K % 64 || ldx < K || ldx % 4) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_few_planes, dim3(S), dim3(256), 0, st, X, ldx, K, (S + 15) / 16, gain, P, ssp);
+    return hipGetLastError();
+}
+
+template <int NT, int D>
+static hipError_t few_launch(int epi, const QtFewArgs &a, hipStream_t st) {
+    const dim3 grid(a.N / (16 * NT), a.RT);
+    if (epi == QF_STORE) hipLaunchKernelGGL((k_few<NT, D, QF_STORE>), grid, dim3(QF_T), 0, st, a);
+    else if (epi == QF_RESID) hipLaunchKernelGGL((k_few<NT, D, QF_RESID>), grid, dim3(QF_T), 0, st, a);
+    else hipLaunchKernelGGL((k_few<NT, D, QF_SWIGLU>), grid, dim3(QF_T), 0, st, a);
+    return hipGetLastError();
+}
+
+extern "C" hipError_t qt_launch_few_gemm(int epi, const uint16_t *W, int N, int K, const uint16_t *P, int S, const float *ssp,
+                                         int np, float eps, float *Y, int ldy, const float *gain, uint16_t *Pout,
+                                         float *sspo, hipStream_t st) {
+    if (!W || !P || S < 1 || S > QF_ROWS || N < 64 || N % 64 || K < 64 || K % 64 || epi < 0 || epi > 2 ||
+        (epi != QF_RESID && (!ssp || np < 4 || np % 4 || np > QF_PART)) || (epi != QF_SWIGLU && (!Y || ldy < N || ldy % 4)) ||
+        (epi == QF_SWIGLU && !Pout) || (epi == QF_RESID && Pout && (!gain || !sspo || N / 16 > QF_PART)))
+        return hipErrorInvalidValue;
+    const QtFewArgs a = {W, P, N, K, S, (S + 15) / 16, ssp, np, eps, Y, ldy, gain, Pout, sspo};
+    // the tile whose busiest CU reads the fewest bytes (16 K (2 NT + 6) a workgroup), one workgroup a CU
+    int nt = 1;
+    long long best = -1;
+    for (int t = 1; t <= 4; t++) {
+        if (N % (16 * t)) continue;
+        const long long c = ((long long)(N / (16 * t)) * a.RT + 255) / 256 * (2 * t + 6);
+        if (best < 0 || c < best) { best = c; nt = t; }
+    }
+    const int per = (K / 32 + QF_W - 1) / QF_W;    // slices of a wave
+    if (nt == 1) return per <= 4 ? few_launch<1, 4>(epi, a, st) : per <= 8 ? few_launch<1, 8>(epi, a, st) : few_launch<1, 12>(epi, a, st);
+    if (nt == 2) return per <= 4 ? few_launch<2, 4>(epi, a, st) : few_launch<2, 8>(epi, a, st);
+    if (nt == 3) return per <= 4 ? few_launch<3, 4>(epi, a, st) : few_launch<3, 8>(epi, a, st);
+    return few_launch<4, 4>(epi, a, st);
+}

@@ -32,7 +32,7 @@ hipError_t qt_launch_attn_b(const float *q, long long q_bs, const float *qn, con
                             const float *rs, float eps, const int *d_pos, uint16_t *K, uint16_t *V, long long kv_bs,
                             long long pos_stride, long long head_stride, int n_heads, int n_kv, int head_dim,
                             float scale, float *part, long long part_bs, unsigned *cnt, int G, float *out,
-                            long long out_bs, int B, hipStream_t st);
+                            long long out_bs, uint16_t *planes, int B, hipStream_t st);
 int qt_attn_grid(int max_len);
 /* batched projections (qt_batch.hip) */
 hipError_t qt_launch_bpieces(const float *x, long long xstride, const float *norm_w, float eps, int K, int B, int Bp,
@@ -185,8 +185,17 @@ hipError_t qt_launch_pf_attn(const float *QKV, int ld, int S, int nh, int nkv, f
                              hipStream_t st);
 /* as qt_launch_pf_attn, the output going out as the O projection's input planes P instead
  * (*planes = 1) */
-hipError_t qt_launch_pf_attn_planes(const float *QKV, int ld, int S, int nh, int nkv, float scale, float *A, int lda,
-                                    uint16_t *P, int *planes, hipStream_t st);
+hipError_t qt_launch_pf_attn_planes(const float *QKV, int ld, int S, int nh, int nkv, float scale, uint16_t *P, int frag,
+                                    hipStream_t st);
+
+/* bf16 projections of at most 64 rows (qt_few.hip); planes: [K/32][row tile][3][512] */
+int qt_few_ok(int S, int H, int F, int qd, int qkvr);
+int qt_few_first(void);
+size_t qt_few_planes_elems(int S, int K);
+hipError_t qt_launch_few_planes(const float *X, int ldx, int S, int K, const float *gain, uint16_t *P, float *ssp,
+                                hipStream_t st);
+hipError_t qt_launch_few_gemm(int epi, const uint16_t *W, int N, int K, const uint16_t *P, int S, const float *ssp, int np,
+                              float eps, float *Y, int ldy, const float *gain, uint16_t *Pout, float *sspo, hipStream_t st);
 
 /* speech decoder (qt_sd.hip) */
 size_t qt_sd_pack_elems(int K, int N, int ntap, int phases);

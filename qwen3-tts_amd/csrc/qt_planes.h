@@ -31,6 +31,12 @@ __device__ __forceinline__ void qt_planes8(const float (&v)[8], qt_u32x4 (&p)[3]
     }
 }
 
+// Activation planes in the matrix core's operand order, [k / 32][row tile][plane][64 lanes][8]
+// with lane = row % 16 + 16 (k % 32 / 8): where (row, k) of plane 0 is; the planes are 512 apart.
+__device__ __forceinline__ size_t qt_frag_at(int row_tiles, int row, int k) {
+    return ((size_t)((k >> 5) * row_tiles + (row >> 4)) * 3) * 512 + ((row & 15) + 16 * ((k & 31) >> 3)) * 8 + (k & 7);
+}
+
 __device__ __forceinline__ qt_f32x4 qt_mma6(const qt_u32x4 (&a)[3], const qt_u32x4 (&b)[3], qt_f32x4 c) {
     c = qt_mfma_bf16(a[0], b[2], c);
     c = qt_mfma_bf16(a[2], b[0], c);

@@ -447,12 +447,13 @@ __device__ __forceinline__ void pf_att_serial(const float *q, const float *K, co
     out[64 + lane] = o1 / l;
 }
 
-// P != NULL: the output goes out as the three planes of the O projection's input
-// (P[p][s][nh*128], plane stride Sp*nh*128; the same pieces k_pf_pieces makes of the f32
-// output), and the workgroup of the last query tile zeroes rows S <= s < Sp of its heads.
+// P != NULL: the output goes out as the three planes of the O projection's input: RT == 0:
+// P[p][s][nh*128], plane stride Sp*nh*128 (the same pieces k_pf_pieces makes of the f32 output), and
+// the workgroup of the last query tile zeroes rows S <= s < Sp of its heads; RT > 0: in operand
+// order over RT row tiles (qt_frag_at).
 template <int HPK>
 __global__ __launch_bounds__(QT_PF_AT) __attribute__((amdgpu_waves_per_eu(2))) void k_pf_att(
-    const float *QKV, int ld, int S, int nh, int nkv, float scale, float *A, int lda, uint16_t *P, int Sp) {
+    const float *QKV, int ld, int S, int nh, int nkv, float scale, float *A, int lda, uint16_t *P, int Sp, int RT) {
     constexpr int QB = HPK * 3 * 16 * 256;             // the queries' planes: [head][plane][16][128] bf16
     constexpr int OB = HPK * 16 * 128 * 4;             // one wave's sums
     static_assert(QB <= OB * QT_PF_AW, "the queries' planes and the sums share the LDS");
@@ -606,7 +607,8 @@ __global__ __launch_bounds__(QT_PF_AT) __attribute__((amdgpu_waves_per_eu(2))) v
             }
         __syncthreads();
     }
-    const size_t plane = (size_t)Sp * qd;
+    const size_t plane = RT ? 512 : (size_t)Sp * qd;
+    const auto at = [&](int row, int col) { return RT ? qt_frag_at(RT, row, col) : (size_t)row * qd + col; };
     for (int u = tid; u < HPK * 16 * 32; u += QT_PF_AT) {
         const int h = u >> 9, row = (u >> 5) & 15, c = 4 * (u & 31);
         if (serial || q0 + row >= S) continue;
@@ -625,7 +627,7 @@ __global__ __launch_bounds__(QT_PF_AT) __attribute__((amdgpu_waves_per_eu(2))) v
             for (int e = 0; e < 4; e++) qt_put_pieces(&pc[0][e], 4, __fmul_rn(v[e], inv));
 #pragma unroll
             for (int p = 0; p < 3; p++)
-                *reinterpret_cast<uint2 *>(P + p * plane + (size_t)(q0 + row) * qd + col) =
+                *reinterpret_cast<uint2 *>(P + p * plane + at(q0 + row, col)) =
                     make_uint2((uint32_t)pc[p][0] | ((uint32_t)pc[p][1] << 16), (uint32_t)pc[p][2] | ((uint32_t)pc[p][3] << 16));
         } else {
             *reinterpret_cast<qt_f32x4 *>(A + (size_t)(q0 + row) * lda + col) = v * inv;
@@ -641,14 +643,14 @@ __global__ __launch_bounds__(QT_PF_AT) __attribute__((amdgpu_waves_per_eu(2))) v
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
             for (int e = 0; e < 2; e++) {
-                const size_t at = (size_t)qq * (P ? qd : lda) + (h0 + h) * 128 + 64 * e + lane;
-                if (P) qt_put_pieces(P + at, (int)plane, out[64 * e + lane]);
-                else A[at] = out[64 * e + lane];
+                const int col = (h0 + h) * 128 + 64 * e + lane;
+                if (P) qt_put_pieces(P + at(qq, col), (int)plane, out[64 * e + lane]);
+                else A[(size_t)qq * lda + col] = out[64 * e + lane];
             }
             __builtin_amdgcn_wave_barrier();
         }
     }
-    if (P && qt == (int)gridDim.x - 1)
+    if (P && !RT && qt == (int)gridDim.x - 1)
         for (int i = tid; i < (Sp - S) * 32 * HPK; i += QT_PF_AT) {
             uint16_t *dst = P + (size_t)(S + i / (32 * HPK)) * qd + h0 * 128 + 4 * (i % (32 * HPK));
 #pragma unroll
@@ -804,29 +806,27 @@ extern "C" hipError_t qt_launch_pf_qkv_post(float *QKV, int ld, int S, int nh, i
     return hipGetLastError();
 }
 
-// P != NULL (with planes): the output is written as the O projection's input planes
-// (rows padded to qt_pf_spad(S)) and *planes = 1; otherwise A gets the f32 rows.
 static hipError_t pf_attn(const float *QKV, int ld, int S, int nh, int nkv, float scale, float *A, int lda,
-                          uint16_t *P, int *planes, hipStream_t st) {
+                          uint16_t *P, int frag, hipStream_t st) {
     if (S <= 0 || nh <= 0 || nkv <= 0 || nh % nkv) return hipErrorInvalidValue;
-    const int Sp = qt_pf_spad(S);
-    if (planes) *planes = P != NULL;
-    if (!planes) P = NULL;
+    const int Sp = qt_pf_spad(S), rt = frag ? (S + 15) / 16 : 0;
     // One head a workgroup while every such workgroup has a CU of its own, then two heads of a kv
     // head, which split its keys and values once (16 heads: 8.8 us against 11.9 at 128 positions, 13.4
     // against 17.3 at 256, then 28.2 against 21.1 at 384 and 40.1 against 26.7 at 512)
     if ((nh / nkv) % 2 == 0 && (long long)((S + 15) / 16) * nh > 256)
-        hipLaunchKernelGGL(k_pf_att<2>, dim3((S + 15) / 16, nh / 2), dim3(QT_PF_AT), 0, st, QKV, ld, S, nh, nkv, scale, A, lda, P, Sp);
+        hipLaunchKernelGGL(k_pf_att<2>, dim3((S + 15) / 16, nh / 2), dim3(QT_PF_AT), 0, st, QKV, ld, S, nh, nkv, scale, A, lda, P, Sp, rt);
     else
-        hipLaunchKernelGGL(k_pf_att<1>, dim3((S + 15) / 16, nh), dim3(QT_PF_AT), 0, st, QKV, ld, S, nh, nkv, scale, A, lda, P, Sp);
+        hipLaunchKernelGGL(k_pf_att<1>, dim3((S + 15) / 16, nh), dim3(QT_PF_AT), 0, st, QKV, ld, S, nh, nkv, scale, A, lda, P, Sp, rt);
     return hipGetLastError();
 }
 
 extern "C" hipError_t qt_launch_pf_attn(const float *QKV, int ld, int S, int nh, int nkv, float scale, float *A,
                                         int lda, hipStream_t st) {
-    return pf_attn(QKV, ld, S, nh, nkv, scale, A, lda, NULL, NULL, st);
+    return pf_attn(QKV, ld, S, nh, nkv, scale, A, lda, NULL, 0, st);
 }
-extern "C" hipError_t qt_launch_pf_attn_planes(const float *QKV, int ld, int S, int nh, int nkv, float scale, float *A,
-                                               int lda, uint16_t *P, int *planes, hipStream_t st) {
-    return pf_attn(QKV, ld, S, nh, nkv, scale, A, lda, P, planes, st);
+// the output as the O projection's input planes: P[p][s][nh*128] (rows padded to qt_pf_spad(S)), or,
+// with frag, in operand order (qt_frag_at)
+extern "C" hipError_t qt_launch_pf_attn_planes(const float *QKV, int ld, int S, int nh, int nkv, float scale, uint16_t *P,
+                                               int frag, hipStream_t st) {
+    return pf_attn(QKV, ld, S, nh, nkv, scale, NULL, 0, P, frag, st);
 }

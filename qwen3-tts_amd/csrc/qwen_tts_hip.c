@@ -363,6 +363,25 @@ static hipError_t stack_body(stack_t *s, float *x, const int *d_pos, hipStream_t
     return stack_body_ex(s, x, d_pos, st, NULL);
 }
 
+typedef struct { uint16_t *x, *a, *h; float *ss; } few_t;
+
+/* The buffers of qt_few.hip's projections: the planes of the normed input, of the attention
+ * output and of the SwiGLU output, and the rows' partial sums of squares. */
+static int few_alloc(few_t *f, const stack_t *s) {
+    HCK(hipMalloc((void **)&f->x, qt_few_planes_elems(64, s->H) * sizeof(uint16_t)));
+    HCK(hipMalloc((void **)&f->a, qt_few_planes_elems(64, s->qd) * sizeof(uint16_t)));
+    HCK(hipMalloc((void **)&f->h, qt_few_planes_elems(64, s->F) * sizeof(uint16_t)));
+    HCK(hipMalloc((void **)&f->ss, (size_t)64 * (s->H / 16) * sizeof(float)));
+    return 0;
+fail:
+    return -1;
+}
+static void few_free(few_t *f) {
+    void *b[] = {f->x, f->a, f->h, f->ss};
+    for (size_t i = 0; i < sizeof b / sizeof b[0]; i++) if (b[i]) (void)hipFree(b[i]);
+    memset(f, 0, sizeof *f);
+}
+
 /* ---- Talker state ------------------------------------------------------------------ */
 
 typedef struct {
@@ -409,10 +428,11 @@ typedef struct {
      * are bf16, else owned copies made on the first prefill) and position buffers */
     dmat_t *pf_qkv, *pf_o, *pf_gu, *pf_dn;
     int pf_cap;             /* positions the buffers below hold */
-    float *pf_x, *pf_qkvb, *pf_attn, *pf_h;
+    float *pf_x, *pf_qkvb, *pf_h;
     float *pf_e;            /* the last prefill's embeddings (pf_x becomes the residual stream) */
     float *pf_part;         /* split-K partial sums, PF_PART_FLOATS */
     uint16_t *pf_p;         /* activation planes [3][spad][max(H, qd, F)] */
+    few_t pf_few;           /* prompts of at most 64 positions */
 } talker_t;
 
 /* QWEN_HIP_RSTEP=0 keeps the single-role persistent kernel (qt_pstep.hip) for shapes the
@@ -462,8 +482,9 @@ static void talker_destroy(talker_t *t) {
     void *bufs[] = {t->io, t->d_pos, t->d_frame, t->d_tok, t->d_hist, t->codec_head, t->codec_emb, t->logits,
                     t->smp_hist, t->smp_seed, t->smp_done, t->gen_codes, t->gen_pad,
                     t->ps_layers, t->ps_ring, t->ps_xin, t->ps_epoch, t->ps_err, t->rs_reg, t->rs_slots,
-                    t->pf_x, t->pf_qkvb, t->pf_attn, t->pf_h, t->pf_p, t->pf_part, t->pf_e};
+                    t->pf_x, t->pf_qkvb, t->pf_h, t->pf_p, t->pf_part, t->pf_e};
     for (size_t i = 0; i < sizeof bufs / sizeof bufs[0]; i++) if (bufs[i]) (void)hipFree(bufs[i]);
+    few_free(&t->pf_few);
     if (t->h_in) (void)hipHostFree(t->h_in);
     if (t->h_out) (void)hipHostFree(t->h_out);
     if (t->h_pos) (void)hipHostFree(t->h_pos);
@@ -897,6 +918,20 @@ int qwen_hip_talker_download_kv(void *state, uint16_t *kv_k, uint16_t *kv_v, int
 
 /* -- Talker prefill (qwen_talker_prefill, qwen_tts_talker.c:730-1038) ------------------ */
 
+/* Layer l after its attention (planes in f->a): O + residual, gate|up + SwiGLU, down + residual
+ * over the rows x [n][H]; leaves the planes of x times the next layer's input gain. */
+static hipError_t few_mlp(const stack_t *s, int l, const dmat_t *wo, const dmat_t *wgu, const dmat_t *wdn, const few_t *f,
+                          float *x, int n, hipStream_t st) {
+    const int H = s->H, F = s->F, last = l + 1 == s->L;
+    hipError_t e;
+    if ((e = qt_launch_few_gemm(QT_PF_RESID, (const uint16_t *)wo[l].w, H, s->qd, f->a, n, NULL, 0, s->eps, x, H,
+                                s->post_norm[l], f->x, f->ss, st))) return e;
+    if ((e = qt_launch_few_gemm(QT_PF_SWIGLU, (const uint16_t *)wgu[l].w, 2 * F, H, f->x, n, f->ss, H / 16, s->eps, NULL, 0,
+                                NULL, f->h, NULL, st))) return e;
+    return qt_launch_few_gemm(QT_PF_RESID, (const uint16_t *)wdn[l].w, H, F, f->h, n, NULL, 0, s->eps, x, H,
+                              last ? NULL : s->in_norm[l + 1], last ? NULL : f->x, last ? NULL : f->ss, st);
+}
+
 /* The prefill's layer loop (qwen_tts_talker.c:780-1030) over pf_x (seq residual rows):
  * planes of the normed input -> q|k|v GEMM, whose reduce does the per-head norm, RoPE and
  * KV store -> causal
@@ -915,6 +950,21 @@ static hipError_t pf_layers(talker_t *t, const dmat_t *wq, const dmat_t *wo, con
     const int x_planes = (long long)seq * H <= PF_PART_FLOATS;
     hipError_t e;
 #define PFE(x) do { if ((e = (x)) != hipSuccess) return e; } while (0)
+    if (qt_few_ok(seq, H, F, qd, qkvr)) {
+        /* at most 64 positions: one pass a projection (qt_few.hip), six launches a layer */
+        const few_t *f = &t->pf_few;
+        PFE(qt_launch_few_planes(t->pf_x, H, seq, H, s->in_norm[0], f->x, f->ss, t->st));
+        for (int l = 0; l < L; l++) {
+            const size_t lay = (size_t)l * s->nkv * s->kv_max * s->hd;
+            PFE(qt_launch_few_gemm(QT_PF_STORE, (const uint16_t *)wq[l].w, qkvr, H, f->x, seq, f->ss, l ? H / 16 : qt_few_first(), s->eps,
+                                   t->pf_qkvb, qkvr, NULL, NULL, NULL, t->st));
+            PFE(qt_launch_pf_qkv_post(t->pf_qkvb, qkvr, seq, s->nh, s->nkv, s->qn[l], s->kn[l], s->rope_cos, s->rope_sin,
+                                      s->eps, s->kc + lay, s->vc + lay, s->kv_max, t->st));
+            PFE(qt_launch_pf_attn_planes(t->pf_qkvb, qkvr, seq, s->nh, s->nkv, scale, f->a, 1, t->st));
+            PFE(few_mlp(s, l, wo, wgu, wdn, f, t->pf_x, seq, t->st));
+        }
+        return hipSuccess;
+    }
     for (int l = 0; l < L; l++) {
         const size_t lay = (size_t)l * s->nkv * s->kv_max * s->hd;
         /* layer 0's input planes; later layers get them from the previous down projection */
@@ -928,10 +978,7 @@ static hipError_t pf_layers(talker_t *t, const dmat_t *wq, const dmat_t *wo, con
             PFE(qt_launch_pf_qkv_post(t->pf_qkvb, qkvr, seq, s->nh, s->nkv, s->qn[l], s->kn[l], s->rope_cos, s->rope_sin,
                                       s->eps, s->kc + lay, s->vc + lay, s->kv_max, t->st));
         }
-        int att_planes = 0;
-        PFE(qt_launch_pf_attn_planes(t->pf_qkvb, qkvr, seq, s->nh, s->nkv, scale, t->pf_attn, qd, t->pf_p, &att_planes,
-                                     t->st));
-        if (!att_planes) PFE(qt_launch_pf_pieces(t->pf_attn, qd, seq, qd, NULL, 0.f, t->pf_p, t->st));
+        PFE(qt_launch_pf_attn_planes(t->pf_qkvb, qkvr, seq, s->nh, s->nkv, scale, t->pf_p, 0, t->st));
         if (x_planes) {
             PFE(qt_launch_pf_gemm_resid_planes((const uint16_t *)wo[l].w, t->pf_p, seq, H, qd, t->pf_x, H, s->post_norm[l],
                                                s->eps, t->pf_p, t->pf_part, PF_PART_FLOATS, t->st));
@@ -988,9 +1035,10 @@ fail:
 }
 
 static void pf_free_bufs(talker_t *t) {
-    void *b[] = {t->pf_x, t->pf_qkvb, t->pf_attn, t->pf_h, t->pf_p, t->pf_part, t->pf_e};
+    void *b[] = {t->pf_x, t->pf_qkvb, t->pf_h, t->pf_p, t->pf_part, t->pf_e};
     for (size_t i = 0; i < sizeof b / sizeof b[0]; i++) if (b[i]) (void)hipFree(b[i]);
-    t->pf_x = t->pf_qkvb = t->pf_attn = t->pf_h = t->pf_part = t->pf_e = NULL; t->pf_p = NULL; t->pf_cap = 0;
+    few_free(&t->pf_few);
+    t->pf_x = t->pf_qkvb = t->pf_h = t->pf_part = t->pf_e = NULL; t->pf_p = NULL; t->pf_cap = 0;
 }
 
 int qwen_hip_talker_prefill(void *state, const qwen_hip_layer_t *bf16_layers, const float *embeds, int seq) {
@@ -1021,11 +1069,11 @@ int qwen_hip_talker_prefill(void *state, const qwen_hip_layer_t *bf16_layers, co
         if (F > km) km = F;
         HCK(hipMalloc((void **)&t->pf_x, (size_t)seq * H * sizeof(float)));
         HCK(hipMalloc((void **)&t->pf_qkvb, (size_t)seq * qkvr * sizeof(float)));
-        HCK(hipMalloc((void **)&t->pf_attn, (size_t)seq * qd * sizeof(float)));
         HCK(hipMalloc((void **)&t->pf_h, (size_t)seq * F * sizeof(float)));
         HCK(hipMalloc((void **)&t->pf_p, (size_t)3 * sp * km * sizeof(uint16_t)));
         HCK(hipMalloc((void **)&t->pf_part, (size_t)PF_PART_FLOATS * sizeof(float)));
         HCK(hipMalloc((void **)&t->pf_e, (size_t)seq * H * sizeof(float)));
+        if (qt_few_ok(1, H, F, qd, qkvr) && few_alloc(&t->pf_few, s) != 0) goto fail;
         t->pf_cap = seq;
     }
     HCK(hipMemcpyAsync(t->pf_e, embeds, (size_t)seq * H * sizeof(float), hipMemcpyDefault, t->st));
@@ -1917,7 +1965,8 @@ typedef struct {
     uint16_t *kc, *vc;         /* [B][L][nkv][kv_max][hd] */
     float *x, *qkv, *attn, *h, *hid;
     int8_t *pc; float *ps;     /* activation pieces [Kmax/64][3*Bp][64], scales [Bp] */
-    uint16_t *pf_p; float *pf_part; /* bf16: activation planes [3][64][Kmax], split-K partials (PF_PART_FLOATS) */
+    few_t few;                 /* bf16: the projections' buffers (qt_few.hip) where it takes the shape, else */
+    uint16_t *pf_p; float *pf_part; /* activation planes [3][64][Kmax], split-K partials (PF_PART_FLOATS) */
     int *g2_part; unsigned *g2_cnt; /* int8: split-K tiles and counters of qt_launch_bgemm2_i8 */
     int fold;                  /* int8: pieces made inside each projection launch (qt_launch_bgemm2_i8_px) */
     unsigned *px_sync;         /* in-launch pieces: count + per-workgroup go flags (128-byte lines), error word */
@@ -1938,6 +1987,7 @@ static void batch_destroy(batch_t *bt) {
     void *bufs[] = {bt->kc, bt->vc, bt->x, bt->qkv, bt->attn, bt->h, bt->hid, bt->pc, bt->ps, bt->part, bt->cnt, bt->d_pos,
                     bt->kv_stage, bt->pf_p, bt->pf_part, bt->g2_part, bt->g2_cnt, bt->px_sync};
     for (size_t i = 0; i < sizeof bufs / sizeof bufs[0]; i++) if (bufs[i]) (void)hipFree(bufs[i]);
+    few_free(&bt->few);
     hpipe_free(&bt->up);
     if (bt->h_io) (void)hipHostFree(bt->h_io);
     if (bt->h_pos) (void)hipHostFree(bt->h_pos);
@@ -1979,7 +2029,9 @@ static batch_t *batch_create(const stack_t *s, int B, int is_cp) {
     HCK(hipMalloc((void **)&bt->h, (size_t)B * s->F * sizeof(float)));
     HCK(hipMalloc((void **)&bt->pc, (size_t)K * 3 * bt->Bp));
     HCK(hipMalloc((void **)&bt->ps, (size_t)bt->Bp * sizeof(float)));
-    if (s->prec == QWEN_HIP_BF16) {
+    if (s->prec == QWEN_HIP_BF16 && qt_few_ok(B, s->H, s->F, s->qd, s->qd + 2 * s->kvd)) {
+        if (few_alloc(&bt->few, s) != 0) goto fail;
+    } else if (s->prec == QWEN_HIP_BF16) {
         HCK(hipMalloc((void **)&bt->pf_p, (size_t)3 * qt_pf_spad(B) * K * sizeof(uint16_t)));
         HCK(hipMalloc((void **)&bt->pf_part, (size_t)PF_PART_FLOATS * sizeof(float)));
     }
@@ -2055,22 +2107,28 @@ static hipError_t batch_body(void *arg) {
     const float scale = 1.0f / sqrtf((float)s->hd);
     const int H = s->H, F = s->F, QKV = s->qd + 2 * s->kvd;
     const long long per = (long long)s->L * s->nkv * bt->kv_max * s->hd;
-    /* bf16 weights: each reduce writes the next projection's input planes (the SwiGLU
-     * output, the normed residual), so only layer 0's input and the attention output get a
-     * plane kernel of their own */
-    const int fused = s->prec == QWEN_HIP_BF16 && (long long)bt->B * 2 * F <= PF_PART_FLOATS;
+    /* bf16 weights: each projection writes the next one's input planes (qt_few.hip), or each reduce
+     * of the prefill's projections does (then only layer 0's input and the attention output get a
+     * plane kernel of their own) */
+    const few_t *f = bt->few.x ? &bt->few : NULL;
+    const int fused = !f && s->prec == QWEN_HIP_BF16 && (long long)bt->B * 2 * F <= PF_PART_FLOATS;
+    if (fused && (e = qt_launch_pf_pieces(bt->x, H, bt->B, H, s->in_norm[0], s->eps, bt->pf_p, bt->st))) return e;
+    if (f && (e = qt_launch_few_planes(bt->x, H, bt->B, H, s->in_norm[0], f->x, f->ss, bt->st))) return e;
     for (int l = 0; l < s->L; l++) {
         const size_t lay = (size_t)l * s->nkv * bt->kv_max * s->hd;
-        if (fused) {
-            if (l == 0 && (e = qt_launch_pf_pieces(bt->x, H, bt->B, H, s->in_norm[0], s->eps, bt->pf_p, bt->st))) return e;
-            if ((e = qt_launch_pf_gemm(QT_PF_STORE, (const uint16_t *)s->qkv[l].w, bt->pf_p, bt->B, QKV, H, bt->qkv, QKV,
-                                       bt->pf_part, PF_PART_FLOATS, bt->st))) return e;
-        } else if ((e = batch_proj(bt, &s->qkv[l], QT_EPI_STORE, s->in_norm[l], bt->x, H, bt->qkv, QKV))) return e;
+        if (f) e = qt_launch_few_gemm(QT_PF_STORE, (const uint16_t *)s->qkv[l].w, QKV, H, f->x, bt->B, f->ss, l ? H / 16 : qt_few_first(),
+                                      s->eps, bt->qkv, QKV, NULL, NULL, NULL, bt->st);
+        else if (fused) e = qt_launch_pf_gemm(QT_PF_STORE, (const uint16_t *)s->qkv[l].w, bt->pf_p, bt->B, QKV, H, bt->qkv, QKV,
+                                              bt->pf_part, PF_PART_FLOATS, bt->st);
+        else e = batch_proj(bt, &s->qkv[l], QT_EPI_STORE, s->in_norm[l], bt->x, H, bt->qkv, QKV);
+        if (e) return e;
         if ((e = qt_launch_attn_b(bt->qkv, QKV, s->qn[l], s->kn[l], s->rope_cos, s->rope_sin, s->eps, bt->d_pos,
                                   bt->kc + lay, bt->vc + lay, per, s->hd, (long long)bt->kv_max * s->hd, s->nh, s->nkv,
                                   s->hd, scale, bt->part, (long long)s->nkv * bt->attn_G * (s->nh / s->nkv) * 130,
-                                  bt->cnt, bt->attn_G, bt->attn, s->qd, bt->B, bt->st))) return e;
-        if (fused) {
+                                  bt->cnt, bt->attn_G, bt->attn, s->qd, f ? f->a : NULL, bt->B, bt->st))) return e;
+        if (f) {
+            if ((e = few_mlp(s, l, s->o, s->gu, s->dn, f, bt->x, bt->B, bt->st))) return e;
+        } else if (fused) {
             if ((e = qt_launch_pf_pieces(bt->attn, s->qd, bt->B, s->qd, NULL, 0.f, bt->pf_p, bt->st))) return e;
             if ((e = qt_launch_pf_gemm_resid_planes((const uint16_t *)s->o[l].w, bt->pf_p, bt->B, H, s->qd, bt->x, H,
                                                     s->post_norm[l], s->eps, bt->pf_p, bt->pf_part, PF_PART_FLOATS,

@@ -235,6 +235,39 @@ def test_batch_step_ragged_vs_oracle(oracle, prec, B):
     g.free()
 
 
+@pytest.mark.parametrize("name,B", [("tiny", 1), ("tiny", 31), ("mini", 5), ("mini", 16), ("mini", 49), ("mini17", 17),
+                                    ("mini17", 64)])
+def test_batch_bf16_row_tiles_vs_oracle(oracle, name, B):
+    """bf16 projections of B rows: whole and partial tiles of 16, K from a slice per wave up to 24,
+    every weight tile width.  Each stream is at one of three positions with that position's cache;
+    the bars are the ragged test's."""
+    from oracle.oracle import talker_from_tensors
+    print(f"[case] batch bf16 {name} B={B}", flush=True)
+    _, shape, t = model_dir(name)
+    cos, sin = synth.rope_tables(shape.head_dim, shape.rope_theta, 64)
+    g = hip.Talker(shape, hip.layers_from_tensors(t, shape), synth.bf16_to_f32(t["talker.model.norm.weight"]), cos, sin,
+                   hip.BF16, 64)
+    ot, keep = talker_from_tensors(oracle, t, shape, "bf16", 64, cos, sin)
+    rng = np.random.default_rng(B)
+    at = [0, 3, 21]
+    for p in range(at[-1]):
+        oracle.talker_step(ot, rng.normal(0, 0.5, shape.hidden).astype(np.float32), p)
+    kvk, kvv = keep["kv_k"].copy(), keep["kv_v"].copy()
+    bt = hip.TalkerBatch(g, B)
+    pos = np.array([at[b % 3] for b in range(B)], np.int32)
+    ks, vs = np.stack([kvk] * B), np.stack([kvv] * B)
+    for b in range(B):
+        bt.upload_slot(b, ks, vs, int(pos[b]))
+    E = rng.normal(0, 0.5, (B, shape.hidden)).astype(np.float32)
+    got = bt.step(E, pos)
+    for b in range(B):
+        keep["kv_k"][:], keep["kv_v"][:] = kvk, kvv
+        want, _ = oracle.talker_step(ot, E[b], int(pos[b]))
+        assert rel_l2(got[b], want) <= 1e-3 and np.abs(got[b] - want).max() <= 2e-2, (b, rel_l2(got[b], want))
+    bt.free()
+    g.free()
+
+
 @need_ref
 def test_batch_of_identical_streams_matches_single_step():
     """B copies of one stream (the reference's batch self-test, cu:657-730 /

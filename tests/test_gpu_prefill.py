@@ -181,7 +181,8 @@ def test_prefill_async_replays_reproduce_the_prefill():
     tk.free()
 
 
-@pytest.mark.parametrize("name,seq", [("mini", 100), ("mini17", 40), ("mini", 240)])
+@pytest.mark.parametrize("name,seq", [("mini", 100), ("mini17", 40), ("mini", 240), ("tiny", 64), ("mini", 65), ("mini17", 49),
+                                      ("mini", 1)])
 def test_prefill_matches_oracle_layer_shapes(oracle, name, seq):
     """The 0.6B / 1.7B layer shapes (2 layers) against the oracle prefill, then one decode
     step from each side's KV.  240 positions leave 16 padding rows in the O projection's planes."""
