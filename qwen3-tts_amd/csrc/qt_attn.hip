@@ -72,6 +72,7 @@ __device__ __forceinline__ void qt_wait_vm() {
 }
 __device__ __forceinline__ void qt_wait_lgkm0() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 #define QT_B_MIN_CHUNK 1536  // batched step: minimum keys per chunk
+#define QT_B_MIN_CHUNK_FEW 384   // ... with at most 128 (stream, kv head) pairs
 
 // 16 bytes per lane from global memory straight into LDS (global_load_lds_dwordx4):
 // lane i's bytes land at dst + 16*i, dst wave-uniform.  Counted by vmcnt like a load.
@@ -528,7 +529,10 @@ extern "C" hipError_t qt_launch_attn_onepass(int prep, const float *q, const flo
 // 3.20 / 3.41 / 3.59 ms/step.  Shared 128-key blocks (scores, barrier, P.V) had given 3.76 /
 // 3.49 / 3.43 / 3.58 at 128 / 256 / 512 / 1024, and shared 64-key blocks (four workgroups
 // per CU) 3.16 / 3.13 / 3.13 / 3.22 / 3.24 / 3.20 / 3.28 at 256 / 320 / 384 / 448 / 512 /
-// 768 / 1024.
+// 768 / 1024.  With at most 128 (stream, kv head) pairs the chunks are what fills the CUs, and
+// they hold 384 keys (96 / 192 / 384 / 768 / 1536: 12 streams of 200..900 keys, 1.7B q4_0 2.33 / 2.25 /
+// 2.24 / 2.34 / 2.34 ms/step; 16 of 100..2000, 0.6B int8 1.78 / 1.62 / 1.52 / 1.62 / 1.74; 4 of 1000..3000
+// 1.44 / 1.32 / 1.31 / 1.41 / 1.61; six of 60..500 the same from 64 to 1536).
 extern "C" hipError_t qt_launch_attn_b(const float *q, long long q_bs, const float *qn, const float *kn,
                                        const float *rc, const float *rs, float eps, const int *d_pos,
                                        uint16_t *K, uint16_t *V, long long kv_bs, long long pos_stride,
@@ -541,7 +545,7 @@ extern "C" hipError_t qt_launch_attn_b(const float *q, long long q_bs, const flo
     a.K = K; a.V = V; a.pos_stride = pos_stride; a.head_stride = head_stride;
     a.n_heads = n_heads; a.n_kv = n_kv; a.scale = scale; a.part = part; a.cnt = cnt; a.out = out;
     a.q_bs = q_bs; a.kv_bs = kv_bs; a.out_bs = out_bs; a.part_bs = part_bs;
-    a.min_chunk = QT_B_MIN_CHUNK;
+    a.min_chunk = (long long)B * n_kv <= 128 ? QT_B_MIN_CHUNK_FEW : QT_B_MIN_CHUNK;
     a.onepass = 0;
     return attn_launch(a, 1, head_dim, G, B, st);
 }
