@@ -65,6 +65,8 @@ hipError_t qt_launch_select(const float *logits, int n, int mode, int *d_frame, 
                             int *d_pos, hipStream_t st);
 hipError_t qt_launch_gather(const int *tok, int tok_max, const uint16_t *table, int dim, float *out,
                             hipStream_t st);
+hipError_t qt_launch_host_in(float *dst, const float *src, int n, int *d_pos, const int *h_pos, int np, int pos, hipStream_t st);
+hipError_t qt_launch_host_out(float *dst, const float *src, int n, const int *err, int *h_err, hipStream_t st);
 hipError_t qt_launch_copy_f32(const float *src, float *dst, int n, hipStream_t st);
 hipError_t qt_launch_quant_int8(const uint16_t *src, int rows, int cols, uint8_t *dst, float *scale,
                                 hipStream_t st);

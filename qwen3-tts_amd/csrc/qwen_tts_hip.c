@@ -752,20 +752,18 @@ static int talker_step_impl(talker_t *t, const float *embed, float *hidden_out, 
     if (pos >= 0 && talker_grow_kv(t, pos + 1) != 0) return -1;   /* qwen_talker_step grows first (t.c:574) */
     REQ(pos >= 0 && pos < t->s.kv_max && pos < t->s.rope_len, "pos %d out of range (kv_max %d, rope %d)",
         pos, t->s.kv_max, t->s.rope_len);
-    if (talker_set_pos(t, pos) != 0) goto fail;
     memcpy(t->h_in, embed, (size_t)H * sizeof(float));
     if (use_graph && t->ps_on) {
-        HCK(hipMemcpyAsync(t->ps_xin, t->h_in, (size_t)H * sizeof(float), hipMemcpyHostToDevice, t->st));
+        HCK(qt_launch_host_in(t->ps_xin, t->h_in, H, t->d_pos, NULL, 0, t->dev_pos == pos ? -1 : pos, t->st));
         HCK(ps_launch(t, 1, 0));
-        HCK(hipMemcpyAsync(t->h_out, t->io, (size_t)2 * H * sizeof(float), hipMemcpyDeviceToHost, t->st));
-        HCK(hipMemcpyAsync(t->h_err, t->ps_err, sizeof(int), hipMemcpyDeviceToHost, t->st));
+        HCK(qt_launch_host_out(t->h_out, t->io, 2 * H, t->ps_err, t->h_err, t->st));
         HCK(hipStreamSynchronize(t->st));
         if (ps_check(t) != 0) goto fail;
         t->dev_pos = pos + 1;
         if (hidden_out) memcpy(hidden_out, t->h_out, (size_t)H * sizeof(float));
         return 0;
     }
-    HCK(hipMemcpyAsync(t->io + H, t->h_in, (size_t)H * sizeof(float), hipMemcpyHostToDevice, t->st));
+    HCK(qt_launch_host_in(t->io + H, t->h_in, H, t->d_pos, NULL, 0, t->dev_pos == pos ? -1 : pos, t->st));
     if (use_graph && graphs_enabled()) {
         if (!t->graph_ready) {
             if (capture(t->st, &t->exec, talker_body_cb, t) != 0) goto fail;
@@ -775,7 +773,7 @@ static int talker_step_impl(talker_t *t, const float *embed, float *hidden_out, 
     } else {
         HCK(talker_body(t));
     }
-    HCK(hipMemcpyAsync(t->h_out, t->io, (size_t)2 * H * sizeof(float), hipMemcpyDeviceToHost, t->st));
+    HCK(qt_launch_host_out(t->h_out, t->io, 2 * H, NULL, NULL, t->st));
     HCK(hipStreamSynchronize(t->st));
     t->dev_pos = pos + 1;
     if (hidden_out) memcpy(hidden_out, t->h_out, (size_t)H * sizeof(float));
@@ -1081,7 +1079,7 @@ int qwen_hip_talker_prefill(void *state, const qwen_hip_layer_t *bf16_layers, co
     HCK(pf_layers(t, wq, wo, wgu, wdn, seq));
     /* dec_x = the last position's residual (t.c:1032-1033), where get_dec_x reads it */
     HCK(hipMemcpyAsync(t->io + H, t->pf_x + (size_t)(seq - 1) * H, (size_t)H * sizeof(float), hipMemcpyDeviceToDevice, t->st));
-    HCK(hipMemcpyAsync(t->h_out + H, t->io + H, (size_t)H * sizeof(float), hipMemcpyDeviceToHost, t->st));
+    HCK(qt_launch_host_out(t->h_out + H, t->io + H, H, NULL, NULL, t->st));
     HCK(hipStreamSynchronize(t->st));
     return 0;
 fail:
@@ -2066,7 +2064,8 @@ static batch_t *batch_create(const stack_t *s, int B, int is_cp) {
     HCK(hipMemsetAsync(bt->cnt, 0, (size_t)B * s->nkv * sizeof(unsigned), bt->st));
     HCK(hipMalloc((void **)&bt->d_pos, (size_t)B * sizeof(int)));
     HCK(hipHostMalloc((void **)&bt->h_io, (size_t)B * s->H * sizeof(float), hipHostMallocDefault));
-    HCK(hipHostMalloc((void **)&bt->h_pos, (size_t)B * sizeof(int), hipHostMallocDefault));
+    /* the positions, then the error word that a step brings back */
+    HCK(hipHostMalloc((void **)&bt->h_pos, (size_t)(B + 1) * sizeof(int), hipHostMallocDefault));
     HCK(hipStreamSynchronize(bt->st));
     return bt;
 fail:
@@ -2181,8 +2180,7 @@ static int batch_step_run(batch_t *bt, const float *in, const int *pos_arr, floa
     memcpy(bt->h_io, in, (size_t)B * H * sizeof(float));
     memcpy(bt->h_pos, pos_arr, (size_t)B * sizeof(int));
     bt->last_async = 0;
-    HCK(hipMemcpyAsync(bt->x, bt->h_io, (size_t)B * H * sizeof(float), hipMemcpyHostToDevice, bt->st));
-    HCK(hipMemcpyAsync(bt->d_pos, bt->h_pos, (size_t)B * sizeof(int), hipMemcpyHostToDevice, bt->st));
+    HCK(qt_launch_host_in(bt->x, bt->h_io, B * H, bt->d_pos, bt->h_pos, B, -1, bt->st));
     if (use_graph && graphs_enabled()) {
         if (!bt->graph_ready) {
             if (capture(bt->st, &bt->exec, batch_body, bt) != 0) goto fail;
@@ -2193,9 +2191,11 @@ static int batch_step_run(batch_t *bt, const float *in, const int *pos_arr, floa
         HCK(batch_body(bt));
     }
     bt->stepped = 1;
-    HCK(hipMemcpyAsync(bt->h_io, bt->is_cp ? bt->x : bt->hid, (size_t)B * H * sizeof(float), hipMemcpyDeviceToHost, bt->st));
+    bt->h_pos[B] = 0;
+    HCK(qt_launch_host_out(bt->h_io, bt->is_cp ? bt->x : bt->hid, B * H, bt->px_sync ? (const int *)bt->px_sync + 32 * (1 + bt->px_wgs) : NULL,
+                           bt->h_pos + B, bt->st));
     HCK(hipStreamSynchronize(bt->st));
-    if (batch_check_err(bt)) return -1;
+    REQ(bt->h_pos[B] == 0, "batched step: a projection gave up waiting for its in-launch activation pieces");
     if (out) memcpy(out, bt->h_io, (size_t)B * H * sizeof(float));
     return 0;
 fail:
