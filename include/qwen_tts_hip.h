@@ -168,8 +168,9 @@ int   qwen_hip_talker_launch_kernel(void *state, int kernel, int layer, int n);
  * batch_talker_step_impl, qwen_tts_talker.c:1192-1270, qwen_tts_batch.h:87-98) ----
  * B <= 64 streams share the single state's device weights (read once per step for all
  * streams: every precision runs each projection as one GEMM over the B streams on the
- * matrix cores -- int8 and q4_0 on the integer MFMA with exact int8 activation pieces,
- * bf16 on the bf16 MFMA with exact bf16 activation planes); each stream has its
+ * matrix cores -- int8 on the integer MFMA with exact int8 activation pieces, bf16 and q4_0
+ * on the bf16 MFMA with exact bf16 activation planes; q4_0 past qt_few_ok's stream counts as
+ * int8); each stream has its
  * own bf16 KV cache (single state's kv_max) and its own position (ragged).  Free the
  * batch before the single state. */
 

@@ -1,17 +1,22 @@
-// qt_few.hip — bf16 projections of a few rows (the batched step's streams, a short prompt's
-// positions: at most 64) on gfx950.
+// qt_few.hip — bf16 and q4_0 projections of a few rows (the batched step's streams, a short
+// prompt's positions: at most 64) on gfx950.
 //
 // Y = X . W^T with W bf16 [N][K] as stored and X f32, as the exact products of qt_prefill.hip:
 // each activation is the sum of three bf16 planes, a plane times a weight is exact in f32, and
 // the matrix cores sum in f32.  Such a product is a stream of the weights, and what it costs
 // beyond that is latency: a launch is done in one pass, with nothing summed by another one.
 //
-// 0.6B, 28 layers: six streams 1.79 -> 1.08 ms a step; 45 positions 1.83 -> 1.47 ms.
+// bf16, 0.6B, 28 layers: six streams 1.79 -> 1.08 ms a step; 45 positions 1.83 -> 1.47 ms.
+// q4_0 (before: int8 pieces of the activations on the integer matrix cores): 1.7B, 2 streams 2.09 ->
+// 1.53, 12 2.23 -> 1.70, 32 2.63 -> 2.1 ms; 0.6B, 4 1.65 -> 1.1, 48 2.46 -> 1.7; error against 64 bits
+// of 12 streams 3.2e-5 -> 1.1e-5.
 //
 //   * a workgroup owns 16 NT weight rows for all of K; its eight waves take an eighth of K each
 //     and their sums meet in LDS;
 //   * the activations come as planes in operand order (qt_frag_at), written so by whoever
 //     made them;
+//   * a q4_0 block is 32 k, one matrix instruction deep: its weights n - 8 are exact in bf16, its
+//     sums start from zero, and its f16 scale multiplies them in f32;
 //   * RMSNorm is applied around the product: the planes are those of x * gain, each maker of
 //     16 columns of x leaves the sum of their squares (one float a row), and the consumer
 //     scales its sums by 1/rms: the row's statistic needs no launch of its own.
@@ -20,13 +25,16 @@
 #define QF_W 8                   // waves of a workgroup, and parts of K
 #define QF_T (64 * QF_W)
 #define QF_ROWS 64               // rows at most
+#define QF_QPER 32               // q4_0: K slices of a wave at most (K <= 8192)
 #define QF_PART 256              // partial sums of squares at most (hidden <= 4096)
 
 // (the values of qt_launch.h, which the .hip sources do not include)
 enum { QF_STORE = 0, QF_RESID = 1, QF_SWIGLU = 2 };
 
 struct QtFewArgs {
-    const uint16_t *W, *P;       // weights [N][K]; the input's planes
+    const void *W;               // bf16 [N][K], or q4_0 nibbles [N][K / 2] ...
+    const uint16_t *s16;         // ... and f16 block scales [N][K / 32]
+    const uint16_t *P;           // the input's planes
     int N, K, S, RT;             // RT: row tiles of the planes
     const float *ssp; int np;    // STORE, SWIGLU: the rows' partial sums of squares [row][np] (the input is normed)
     float eps;
@@ -47,12 +55,25 @@ __device__ __forceinline__ void qf_put4(uint16_t *P, int RT, int row, int k, qt_
             make_uint2((uint32_t)pc[p][0] | ((uint32_t)pc[p][1] << 16), (uint32_t)pc[p][2] | ((uint32_t)pc[p][3] << 16));
 }
 
+// 8 weights as a lane's operand: bf16 as they are, q4_0 nibbles (element e in bits 4 e, + 8) unpacked
+template <bool Q4> struct QfWord { using t = qt_u32x4; };
+template <> struct QfWord<true> { using t = uint32_t; };
+__device__ __forceinline__ qt_u32x4 qf_q4(uint32_t n) {
+    const int v = (int)(n ^ 0x88888888u);           // two's complement nibbles of n - 8
+    qt_u32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; i++) r[i] = qt_bf16x2((float)(v << (28 - 8 * i) >> 28), (float)(v << (24 - 8 * i) >> 28));
+    return r;
+}
+
 // A workgroup computes 16 NT weight rows for 16 activation rows; each wave has D slices of 32 k of
 // both in flight (all of its eighth of K where the registers hold it: one memory latency).
-template <int NT, int D, int EPI>
+template <int NT, int D, int EPI, bool Q4>
 __global__ __launch_bounds__(QF_T) void k_few(QtFewArgs a) {
     __shared__ __align__(16) qt_f32x4 part[QF_W][NT][64];
     __shared__ float s_inv[16];
+    // q4_0: the block scales of each wave's slices, [slice][weight row], filled and read by that wave
+    __shared__ __align__(16) float s_sc[Q4 ? QF_W : 1][Q4 ? QF_QPER : 1][16 * NT];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, kg = lane >> 4;
     const int n0 = blockIdx.x * 16 * NT, rt = blockIdx.y, ns = a.K / 32;
     const int s0 = ns * wave / QF_W, s1 = ns * (wave + 1) / QF_W;
@@ -73,41 +94,88 @@ __global__ __launch_bounds__(QF_T) void k_few(QtFewArgs a) {
         if (a.Pout) gn = *reinterpret_cast<const qt_f32x4 *>(a.gain + n);
     }
     // rows past S repeat the last one: nothing more is read for them
-    const uint16_t *wp[NT], *xp = a.P + (size_t)rt * 1536 + 8 * (min(li, a.S - 1 - 16 * rt) + 16 * kg);
+    const uint8_t *wp[NT];
+    const uint16_t *xp = a.P + (size_t)rt * 1536 + 8 * (min(li, a.S - 1 - 16 * rt) + 16 * kg);
 #pragma unroll
-    for (int j = 0; j < NT; j++) wp[j] = a.W + (size_t)(n0 + 16 * j + li) * a.K + 8 * kg;
-    qt_u32x4 w[D][NT], x[D][3];
+    for (int j = 0; j < NT; j++)
+        wp[j] = (const uint8_t *)a.W + (Q4 ? (size_t)(n0 + 16 * j + li) * (a.K / 2) + 4 * kg : ((size_t)(n0 + 16 * j + li) * a.K + 8 * kg) * 2);
+    using wt = typename QfWord<Q4>::t;              // 8 weights of a lane
+    wt w[D][NT];
+    qt_u32x4 x[D][3];
     const size_t xs = (size_t)a.RT * 1536;
     auto fetch = [&](int s, int d) {
 #pragma unroll
-        for (int j = 0; j < NT; j++) w[d][j] = *reinterpret_cast<const qt_u32x4 *>(wp[j] + 32 * s);
+        for (int j = 0; j < NT; j++) w[d][j] = *reinterpret_cast<const wt *>(wp[j] + s * (Q4 ? 16 : 64));
 #pragma unroll
         for (int p = 0; p < 3; p++) x[d][p] = *reinterpret_cast<const qt_u32x4 *>(xp + s * xs + 512 * p);
     };
     qt_f32x4 acc[NT];
 #pragma unroll
     for (int j = 0; j < NT; j++) acc[j] = qt_f32x4{0.f, 0.f, 0.f, 0.f};
-    auto mul = [&](int d) {
+    auto mul = [&](int s, int d) {
+        if constexpr (Q4) {
 #pragma unroll
-        for (int p = 0; p < 3; p++)
+            for (int j = 0; j < NT; j++) {
+                const qt_u32x4 q = qf_q4(w[d][j]);
+                qt_f32x4 c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int j = 0; j < NT; j++) acc[j] = qt_mfma_bf16(w[d][j], x[d][2 - p], acc[j]);
+                for (int p = 0; p < 3; p++) c = qt_mfma_bf16(q, x[d][2 - p], c);
+                const qt_f32x4 sc = *reinterpret_cast<const qt_f32x4 *>(&s_sc[wave][s - s0][16 * j + 4 * kg]);
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[j][r] = fmaf(c[r], sc[r], acc[j][r]);
+            }
+        } else {
+#pragma unroll
+            for (int p = 0; p < 3; p++)
+#pragma unroll
+                for (int j = 0; j < NT; j++) acc[j] = qt_mfma_bf16(w[d][j], x[d][2 - p], acc[j]);
+        }
     };
+    // q4_0: four blocks' scales of a weight row a load, asked for ahead of the weights (K a multiple of
+    // 1024: a wave's slices are whole fours)
+    const bool fours = Q4 && a.K % 1024 == 0;
+    uint2 sr[QF_QPER / 16][NT];
+    if (fours) {
+#pragma unroll
+        for (int i = 0; i < QF_QPER / 16; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+                sr[i][j] = *reinterpret_cast<const uint2 *>(a.s16 + (size_t)(n0 + 16 * j + li) * ns + s0 + min(4 * kg + 16 * i, s1 - s0 - 4));
+    }
     // loads past the wave's last slice repeat it: no load is behind a branch, so that the waits count them
     const int last = max(s1 - 1, 0);
 #pragma unroll
     for (int d = 0; d < D; d++) fetch(min(s0 + d, last), d);
+    if constexpr (Q4) {
+        if (fours) {
+#pragma unroll
+            for (int i = 0; i < QF_QPER / 16; i++)
+                if (4 * kg + 16 * i < s1 - s0)
+#pragma unroll
+                    for (int j = 0; j < NT; j++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            s_sc[wave][4 * kg + 16 * i + e][16 * j + li] =
+                                ref_f16_to_f32(((e < 2 ? sr[i][j].x : sr[i][j].y) >> (16 * (e & 1))) & 0xFFFFu);
+        } else {
+            for (int i = kg; i < s1 - s0; i += 4)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+                    s_sc[wave][i][16 * j + li] = ref_f16_to_f32(a.s16[(size_t)(n0 + 16 * j + li) * ns + s0 + i]);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
     int s = s0;
     for (; s + D < s1; s += D) {
 #pragma unroll
         for (int d = 0; d < D; d++) {
-            mul(d);
+            mul(s + d, d);
             fetch(min(s + d + D, last), d);
         }
     }
 #pragma unroll
     for (int d = 0; d < D; d++)
-        if (s + d < s1) mul(d);
+        if (s + d < s1) mul(s + d, d);
 #pragma unroll
     for (int j = 0; j < NT; j++) part[wave][j][lane] = acc[j];
     if (NORM) {
@@ -183,34 +251,54 @@ extern "C" hipError_t qt_launch_few_planes(const float *X, int ldx, int S, int K
     return hipGetLastError();
 }
 
-template <int NT, int D>
+template <int NT, int D, bool Q4>
 static hipError_t few_launch(int epi, const QtFewArgs &a, hipStream_t st) {
     const dim3 grid(a.N / (16 * NT), a.RT);
-    if (epi == QF_STORE) hipLaunchKernelGGL((k_few<NT, D, QF_STORE>), grid, dim3(QF_T), 0, st, a);
-    else if (epi == QF_RESID) hipLaunchKernelGGL((k_few<NT, D, QF_RESID>), grid, dim3(QF_T), 0, st, a);
-    else hipLaunchKernelGGL((k_few<NT, D, QF_SWIGLU>), grid, dim3(QF_T), 0, st, a);
+    if (epi == QF_STORE) hipLaunchKernelGGL((k_few<NT, D, QF_STORE, Q4>), grid, dim3(QF_T), 0, st, a);
+    else if (epi == QF_RESID) hipLaunchKernelGGL((k_few<NT, D, QF_RESID, Q4>), grid, dim3(QF_T), 0, st, a);
+    else hipLaunchKernelGGL((k_few<NT, D, QF_SWIGLU, Q4>), grid, dim3(QF_T), 0, st, a);
     return hipGetLastError();
+}
+
+static hipError_t few_gemm(int epi, const void *W, const uint16_t *s16, int N, int K, const uint16_t *P, int S, const float *ssp,
+                           int np, float eps, float *Y, int ldy, const float *gain, uint16_t *Pout, float *sspo,
+                           hipStream_t st) {
+    if (!W || !P || S < 1 || S > QF_ROWS || N < 64 || N % 64 || K < 64 || K % 64 || (s16 && K > 256 * QF_QPER) || epi < 0 || epi > 2 ||
+        (epi != QF_RESID && (!ssp || np < 4 || np % 4 || np > QF_PART)) ||
+        (epi != QF_SWIGLU && (!Y || ldy < N || ldy % 4)) ||
+        (epi == QF_SWIGLU && !Pout) || (epi == QF_RESID && Pout && (!gain || !sspo || N / 16 > QF_PART)))
+        return hipErrorInvalidValue;
+    const QtFewArgs a = {W, s16, P, N, K, S, (S + 15) / 16, ssp, np, eps, Y, ldy, gain, Pout, sspo};
+    // the tile whose busiest CU reads the fewest bytes (16 K (2 NT + 6) a workgroup; q4_0: NT / 2 + 6), one
+    // workgroup a CU
+    int nt = 1;
+    long long best = -1;
+    for (int t = 1; t <= 4; t++) {
+        if (N % (16 * t)) continue;
+        const long long c = ((long long)(N / (16 * t)) * a.RT + 255) / 256 * (s16 ? t + 12 : 4 * t + 12);
+        if (best < 0 || c < best) { best = c; nt = t; }
+    }
+    const int per = (K / 32 + QF_W - 1) / QF_W;    // slices of a wave
+    if (s16) {
+        if (nt == 1) return per <= 4 ? few_launch<1, 4, true>(epi, a, st) : per <= 8 ? few_launch<1, 8, true>(epi, a, st) : few_launch<1, 12, true>(epi, a, st);
+        if (nt == 2) return per <= 4 ? few_launch<2, 4, true>(epi, a, st) : few_launch<2, 8, true>(epi, a, st);
+        if (nt == 3) return per <= 4 ? few_launch<3, 4, true>(epi, a, st) : few_launch<3, 8, true>(epi, a, st);
+        return per <= 4 ? few_launch<4, 4, true>(epi, a, st) : few_launch<4, 8, true>(epi, a, st);
+    }
+    if (nt == 1) return per <= 4 ? few_launch<1, 4, false>(epi, a, st) : per <= 8 ? few_launch<1, 8, false>(epi, a, st) : few_launch<1, 12, false>(epi, a, st);
+    if (nt == 2) return per <= 4 ? few_launch<2, 4, false>(epi, a, st) : few_launch<2, 8, false>(epi, a, st);
+    if (nt == 3) return per <= 4 ? few_launch<3, 4, false>(epi, a, st) : few_launch<3, 8, false>(epi, a, st);
+    return few_launch<4, 4, false>(epi, a, st);
 }
 
 extern "C" hipError_t qt_launch_few_gemm(int epi, const uint16_t *W, int N, int K, const uint16_t *P, int S, const float *ssp,
                                          int np, float eps, float *Y, int ldy, const float *gain, uint16_t *Pout,
                                          float *sspo, hipStream_t st) {
-    if (!W || !P || S < 1 || S > QF_ROWS || N < 64 || N % 64 || K < 64 || K % 64 || epi < 0 || epi > 2 ||
-        (epi != QF_RESID && (!ssp || np < 4 || np % 4 || np > QF_PART)) || (epi != QF_SWIGLU && (!Y || ldy < N || ldy % 4)) ||
-        (epi == QF_SWIGLU && !Pout) || (epi == QF_RESID && Pout && (!gain || !sspo || N / 16 > QF_PART)))
-        return hipErrorInvalidValue;
-    const QtFewArgs a = {W, P, N, K, S, (S + 15) / 16, ssp, np, eps, Y, ldy, gain, Pout, sspo};
-    // the tile whose busiest CU reads the fewest bytes (16 K (2 NT + 6) a workgroup), one workgroup a CU
-    int nt = 1;
-    long long best = -1;
-    for (int t = 1; t <= 4; t++) {
-        if (N % (16 * t)) continue;
-        const long long c = ((long long)(N / (16 * t)) * a.RT + 255) / 256 * (2 * t + 6);
-        if (best < 0 || c < best) { best = c; nt = t; }
-    }
-    const int per = (K / 32 + QF_W - 1) / QF_W;    // slices of a wave
-    if (nt == 1) return per <= 4 ? few_launch<1, 4>(epi, a, st) : per <= 8 ? few_launch<1, 8>(epi, a, st) : few_launch<1, 12>(epi, a, st);
-    if (nt == 2) return per <= 4 ? few_launch<2, 4>(epi, a, st) : few_launch<2, 8>(epi, a, st);
-    if (nt == 3) return per <= 4 ? few_launch<3, 4>(epi, a, st) : few_launch<3, 8>(epi, a, st);
-    return few_launch<4, 4>(epi, a, st);
+    return few_gemm(epi, W, NULL, N, K, P, S, ssp, np, eps, Y, ldy, gain, Pout, sspo, st);
+}
+extern "C" hipError_t qt_launch_few_gemm_q4(int epi, const uint8_t *W, const uint16_t *s16, int N, int K, const uint16_t *P,
+                                            int S, const float *ssp, int np, float eps, float *Y, int ldy, const float *gain,
+                                            uint16_t *Pout, float *sspo, hipStream_t st) {
+    if (!s16) return hipErrorInvalidValue;
+    return few_gemm(epi, W, s16, N, K, P, S, ssp, np, eps, Y, ldy, gain, Pout, sspo, st);
 }

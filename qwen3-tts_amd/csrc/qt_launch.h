@@ -198,6 +198,9 @@ hipError_t qt_launch_few_planes(const float *X, int ldx, int S, int K, const flo
                                 hipStream_t st);
 hipError_t qt_launch_few_gemm(int epi, const uint16_t *W, int N, int K, const uint16_t *P, int S, const float *ssp, int np,
                               float eps, float *Y, int ldy, const float *gain, uint16_t *Pout, float *sspo, hipStream_t st);
+hipError_t qt_launch_few_gemm_q4(int epi, const uint8_t *W, const uint16_t *s16, int N, int K, const uint16_t *P, int S,
+                                 const float *ssp, int np, float eps, float *Y, int ldy, const float *gain, uint16_t *Pout,
+                                 float *sspo, hipStream_t st);
 
 /* speech decoder (qt_sd.hip) */
 size_t qt_sd_pack_elems(int K, int N, int ntap, int phases);

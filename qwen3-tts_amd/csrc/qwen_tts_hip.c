@@ -916,18 +916,24 @@ int qwen_hip_talker_download_kv(void *state, uint16_t *kv_k, uint16_t *kv_v, int
 
 /* -- Talker prefill (qwen_talker_prefill, qwen_tts_talker.c:730-1038) ------------------ */
 
+/* one projection of a few rows in the matrix's own precision (bf16 or q4_0) */
+static hipError_t few_proj(const dmat_t *m, int epi, const uint16_t *P, int n, const float *ss, int np, float eps, float *y,
+                           const float *gain, uint16_t *Pout, float *sso, hipStream_t st) {
+    if (m->prec == QWEN_HIP_Q4_0)
+        return qt_launch_few_gemm_q4(epi, m->w, m->s16, m->rows, m->cols, P, n, ss, np, eps, y, m->rows, gain, Pout, sso, st);
+    return qt_launch_few_gemm(epi, (const uint16_t *)m->w, m->rows, m->cols, P, n, ss, np, eps, y, m->rows, gain, Pout, sso, st);
+}
+
 /* Layer l after its attention (planes in f->a): O + residual, gate|up + SwiGLU, down + residual
  * over the rows x [n][H]; leaves the planes of x times the next layer's input gain. */
 static hipError_t few_mlp(const stack_t *s, int l, const dmat_t *wo, const dmat_t *wgu, const dmat_t *wdn, const few_t *f,
                           float *x, int n, hipStream_t st) {
-    const int H = s->H, F = s->F, last = l + 1 == s->L;
+    const int last = l + 1 == s->L;
     hipError_t e;
-    if ((e = qt_launch_few_gemm(QT_PF_RESID, (const uint16_t *)wo[l].w, H, s->qd, f->a, n, NULL, 0, s->eps, x, H,
-                                s->post_norm[l], f->x, f->ss, st))) return e;
-    if ((e = qt_launch_few_gemm(QT_PF_SWIGLU, (const uint16_t *)wgu[l].w, 2 * F, H, f->x, n, f->ss, H / 16, s->eps, NULL, 0,
-                                NULL, f->h, NULL, st))) return e;
-    return qt_launch_few_gemm(QT_PF_RESID, (const uint16_t *)wdn[l].w, H, F, f->h, n, NULL, 0, s->eps, x, H,
-                              last ? NULL : s->in_norm[l + 1], last ? NULL : f->x, last ? NULL : f->ss, st);
+    if ((e = few_proj(&wo[l], QT_PF_RESID, f->a, n, NULL, 0, s->eps, x, s->post_norm[l], f->x, f->ss, st))) return e;
+    if ((e = few_proj(&wgu[l], QT_PF_SWIGLU, f->x, n, f->ss, s->H / 16, s->eps, NULL, NULL, f->h, NULL, st))) return e;
+    return few_proj(&wdn[l], QT_PF_RESID, f->h, n, NULL, 0, s->eps, x, last ? NULL : s->in_norm[l + 1], last ? NULL : f->x,
+                    last ? NULL : f->ss, st);
 }
 
 /* The prefill's layer loop (qwen_tts_talker.c:780-1030) over pf_x (seq residual rows):
@@ -954,8 +960,8 @@ static hipError_t pf_layers(talker_t *t, const dmat_t *wq, const dmat_t *wo, con
         PFE(qt_launch_few_planes(t->pf_x, H, seq, H, s->in_norm[0], f->x, f->ss, t->st));
         for (int l = 0; l < L; l++) {
             const size_t lay = (size_t)l * s->nkv * s->kv_max * s->hd;
-            PFE(qt_launch_few_gemm(QT_PF_STORE, (const uint16_t *)wq[l].w, qkvr, H, f->x, seq, f->ss, l ? H / 16 : qt_few_first(), s->eps,
-                                   t->pf_qkvb, qkvr, NULL, NULL, NULL, t->st));
+            PFE(few_proj(&wq[l], QT_PF_STORE, f->x, seq, f->ss, l ? H / 16 : qt_few_first(), s->eps, t->pf_qkvb, NULL, NULL, NULL,
+                         t->st));
             PFE(qt_launch_pf_qkv_post(t->pf_qkvb, qkvr, seq, s->nh, s->nkv, s->qn[l], s->kn[l], s->rope_cos, s->rope_sin,
                                       s->eps, s->kc + lay, s->vc + lay, s->kv_max, t->st));
             PFE(qt_launch_pf_attn_planes(t->pf_qkvb, qkvr, seq, s->nh, s->nkv, scale, f->a, 1, t->st));
@@ -1947,11 +1953,12 @@ fail:
  *   pieces(RMSNorm(x)) -> MFMA QKV -> attention (q/k norm, RoPE, KV append, split-K over
  *   each stream's own length, B streams in one grid) -> pieces(attn) -> MFMA O + residual
  *   -> pieces(RMSNorm(x)) -> MFMA gate|up + SwiGLU -> pieces(h) -> MFMA down + residual,
- * captured once into a hipGraph (positions live on the device).  q4_0 weights take the
- * same pieces into qt_launch_bgemm_q4 (per-32-block integer sums, block scale in f32);
- * bf16 weights take the prefill's projection GEMM (three exact bf16 activation planes on
- * the bf16 MFMA, split K for the residual projections).  Every weight is read once per
- * step for all B streams in every precision. */
+ * captured once into a hipGraph (positions live on the device).  bf16 and q4_0 weights take
+ * qt_few.hip's projections (three exact bf16 activation planes on the bf16 MFMA, the norms
+ * applied around the products, five launches a layer); past the widths and stream counts that
+ * qt_few_ok states, bf16 takes the prefill's projection GEMM and q4_0 the int8 pieces into
+ * qt_launch_bgemm_q4 (per-32-block integer sums, block scale in f32).  Every weight is read from
+ * HBM once per step for all B streams in every precision. */
 
 #define QWEN_HIP_BATCH_MAX 64
 
@@ -1963,7 +1970,7 @@ typedef struct {
     uint16_t *kc, *vc;         /* [B][L][nkv][kv_max][hd] */
     float *x, *qkv, *attn, *h, *hid;
     int8_t *pc; float *ps;     /* activation pieces [Kmax/64][3*Bp][64], scales [Bp] */
-    few_t few;                 /* bf16: the projections' buffers (qt_few.hip) where it takes the shape, else */
+    few_t few;                 /* bf16, q4_0: the projections' buffers (qt_few.hip) where it takes the shape, else (bf16) */
     uint16_t *pf_p; float *pf_part; /* activation planes [3][64][Kmax], split-K partials (PF_PART_FLOATS) */
     int *g2_part; unsigned *g2_cnt; /* int8: split-K tiles and counters of qt_launch_bgemm2_i8 */
     int fold;                  /* int8: pieces made inside each projection launch (qt_launch_bgemm2_i8_px) */
@@ -2027,7 +2034,8 @@ static batch_t *batch_create(const stack_t *s, int B, int is_cp) {
     HCK(hipMalloc((void **)&bt->h, (size_t)B * s->F * sizeof(float)));
     HCK(hipMalloc((void **)&bt->pc, (size_t)K * 3 * bt->Bp));
     HCK(hipMalloc((void **)&bt->ps, (size_t)bt->Bp * sizeof(float)));
-    if (s->prec == QWEN_HIP_BF16 && qt_few_ok(B, s->H, s->F, s->qd, s->qd + 2 * s->kvd)) {
+    if (s->prec != QWEN_HIP_INT8 && qt_few_ok(B, s->H, s->F, s->qd, s->qd + 2 * s->kvd) &&
+        (s->prec == QWEN_HIP_BF16 || K <= 8192)) {
         if (few_alloc(&bt->few, s) != 0) goto fail;
     } else if (s->prec == QWEN_HIP_BF16) {
         HCK(hipMalloc((void **)&bt->pf_p, (size_t)3 * qt_pf_spad(B) * K * sizeof(uint16_t)));
@@ -2106,17 +2114,17 @@ static hipError_t batch_body(void *arg) {
     const float scale = 1.0f / sqrtf((float)s->hd);
     const int H = s->H, F = s->F, QKV = s->qd + 2 * s->kvd;
     const long long per = (long long)s->L * s->nkv * bt->kv_max * s->hd;
-    /* bf16 weights: each projection writes the next one's input planes (qt_few.hip), or each reduce
-     * of the prefill's projections does (then only layer 0's input and the attention output get a
-     * plane kernel of their own) */
+    /* bf16 and q4_0 weights: each projection writes the next one's input planes (qt_few.hip); past
+     * its shapes, bf16: each reduce of the prefill's projections does (then only layer 0's input and
+     * the attention output get a plane kernel of their own) */
     const few_t *f = bt->few.x ? &bt->few : NULL;
     const int fused = !f && s->prec == QWEN_HIP_BF16 && (long long)bt->B * 2 * F <= PF_PART_FLOATS;
     if (fused && (e = qt_launch_pf_pieces(bt->x, H, bt->B, H, s->in_norm[0], s->eps, bt->pf_p, bt->st))) return e;
     if (f && (e = qt_launch_few_planes(bt->x, H, bt->B, H, s->in_norm[0], f->x, f->ss, bt->st))) return e;
     for (int l = 0; l < s->L; l++) {
         const size_t lay = (size_t)l * s->nkv * bt->kv_max * s->hd;
-        if (f) e = qt_launch_few_gemm(QT_PF_STORE, (const uint16_t *)s->qkv[l].w, QKV, H, f->x, bt->B, f->ss, l ? H / 16 : qt_few_first(),
-                                      s->eps, bt->qkv, QKV, NULL, NULL, NULL, bt->st);
+        if (f) e = few_proj(&s->qkv[l], QT_PF_STORE, f->x, bt->B, f->ss, l ? H / 16 : qt_few_first(), s->eps, bt->qkv, NULL, NULL,
+                            NULL, bt->st);
         else if (fused) e = qt_launch_pf_gemm(QT_PF_STORE, (const uint16_t *)s->qkv[l].w, bt->pf_p, bt->B, QKV, H, bt->qkv, QKV,
                                               bt->pf_part, PF_PART_FLOATS, bt->st);
         else e = batch_proj(bt, &s->qkv[l], QT_EPI_STORE, s->in_norm[l], bt->x, H, bt->qkv, QKV);

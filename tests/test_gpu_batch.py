@@ -235,19 +235,20 @@ def test_batch_step_ragged_vs_oracle(oracle, prec, B):
     g.free()
 
 
+@pytest.mark.parametrize("prec", ["bf16", "int4"])
 @pytest.mark.parametrize("name,B", [("tiny", 1), ("tiny", 31), ("mini", 5), ("mini", 16), ("mini", 49), ("mini17", 17),
                                     ("mini17", 64)])
-def test_batch_bf16_row_tiles_vs_oracle(oracle, name, B):
-    """bf16 projections of B rows: whole and partial tiles of 16, K from a slice per wave up to 24,
+def test_batch_row_tiles_vs_oracle(oracle, name, B, prec):
+    """bf16 and q4_0 projections of B rows: whole and partial tiles of 16, K from a slice per wave up to 24,
     every weight tile width.  Each stream is at one of three positions with that position's cache;
     the bars are the ragged test's."""
     from oracle.oracle import talker_from_tensors
-    print(f"[case] batch bf16 {name} B={B}", flush=True)
+    print(f"[case] batch {prec} {name} B={B}", flush=True)
     _, shape, t = model_dir(name)
     cos, sin = synth.rope_tables(shape.head_dim, shape.rope_theta, 64)
     g = hip.Talker(shape, hip.layers_from_tensors(t, shape), synth.bf16_to_f32(t["talker.model.norm.weight"]), cos, sin,
-                   hip.BF16, 64)
-    ot, keep = talker_from_tensors(oracle, t, shape, "bf16", 64, cos, sin)
+                   hip.BF16, 64, quantize_to=-1 if prec == "bf16" else hip.PREC[prec])
+    ot, keep = talker_from_tensors(oracle, t, shape, prec, 64, cos, sin)
     rng = np.random.default_rng(B)
     at = [0, 3, 21]
     for p in range(at[-1]):
