@@ -168,9 +168,9 @@ int   qwen_hip_talker_launch_kernel(void *state, int kernel, int layer, int n);
  * batch_talker_step_impl, qwen_tts_talker.c:1192-1270, qwen_tts_batch.h:87-98) ----
  * B <= 64 streams share the single state's device weights (read once per step for all
  * streams: every precision runs each projection as one GEMM over the B streams on the
- * matrix cores -- int8 on the integer MFMA with exact int8 activation pieces, bf16 and q4_0
- * on the bf16 MFMA with exact bf16 activation planes; q4_0 past qt_few_ok's stream counts as
- * int8); each stream has its
+ * matrix cores -- on the bf16 MFMA with exact bf16 activation planes; int8 and q4_0 past
+ * qt_few_ok's stream counts on the integer MFMA with exact int8 activation pieces); each
+ * stream has its
  * own bf16 KV cache (single state's kv_max) and its own position (ragged).  Free the
  * batch before the single state. */
 
@@ -204,7 +204,8 @@ void *qwen_hip_talker_batch_stream(void *state);
 /* Test/measurement switch (no reference counterpart): int8 projections make their
  * activation pieces inside the projection launch (on = 1, the default wherever every
  * projection shape allows it) or in a launch of their own (0); both give the same bytes.
- * Applies to Talker and CP batch states.  Returns the mode in effect, -1 on error. */
+ * Applies to Talker and CP batch states; one that runs on the bf16 planes (few streams) goes
+ * over to the pieces with the first call.  Returns the mode in effect, -1 on error. */
 int   qwen_hip_batch_fold_pieces(void *state, int on);
 
 /* ---- level 2: Code Predictor (qwen_tts_cuda_talker.cu:751-841; qwen_tts_metal.m:2246) ---- */

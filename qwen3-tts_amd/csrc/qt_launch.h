@@ -190,17 +190,15 @@ hipError_t qt_launch_pf_attn(const float *QKV, int ld, int S, int nh, int nkv, f
 hipError_t qt_launch_pf_attn_planes(const float *QKV, int ld, int S, int nh, int nkv, float scale, uint16_t *P, int frag,
                                     hipStream_t st);
 
-/* bf16 projections of at most 64 rows (qt_few.hip); planes: [K/32][row tile][3][512] */
-int qt_few_ok(int S, int H, int F, int qd, int qkvr);
+/* projections of at most 64 rows (qt_few.hip); planes: [K/32][row tile][3][512] */
+int qt_few_ok(int prec, int S, int H, int F, int qd, int qkvr);
 int qt_few_first(void);
 size_t qt_few_planes_elems(int S, int K);
 hipError_t qt_launch_few_planes(const float *X, int ldx, int S, int K, const float *gain, uint16_t *P, float *ssp,
                                 hipStream_t st);
-hipError_t qt_launch_few_gemm(int epi, const uint16_t *W, int N, int K, const uint16_t *P, int S, const float *ssp, int np,
-                              float eps, float *Y, int ldy, const float *gain, uint16_t *Pout, float *sspo, hipStream_t st);
-hipError_t qt_launch_few_gemm_q4(int epi, const uint8_t *W, const uint16_t *s16, int N, int K, const uint16_t *P, int S,
-                                 const float *ssp, int np, float eps, float *Y, int ldy, const float *gain, uint16_t *Pout,
-                                 float *sspo, hipStream_t st);
+hipError_t qt_launch_few_gemm(int prec, int epi, const void *W, const float *scale, const uint16_t *s16, int N, int K,
+                              const uint16_t *P, int S, const float *ssp, int np, float eps, float *Y, int ldy,
+                              const float *gain, uint16_t *Pout, float *sspo, hipStream_t st);
 
 /* speech decoder (qt_sd.hip) */
 size_t qt_sd_pack_elems(int K, int N, int ntap, int phases);

@@ -916,12 +916,11 @@ int qwen_hip_talker_download_kv(void *state, uint16_t *kv_k, uint16_t *kv_v, int
 
 /* -- Talker prefill (qwen_talker_prefill, qwen_tts_talker.c:730-1038) ------------------ */
 
-/* one projection of a few rows in the matrix's own precision (bf16 or q4_0) */
+/* one projection of a few rows in the matrix's own precision */
 static hipError_t few_proj(const dmat_t *m, int epi, const uint16_t *P, int n, const float *ss, int np, float eps, float *y,
                            const float *gain, uint16_t *Pout, float *sso, hipStream_t st) {
-    if (m->prec == QWEN_HIP_Q4_0)
-        return qt_launch_few_gemm_q4(epi, m->w, m->s16, m->rows, m->cols, P, n, ss, np, eps, y, m->rows, gain, Pout, sso, st);
-    return qt_launch_few_gemm(epi, (const uint16_t *)m->w, m->rows, m->cols, P, n, ss, np, eps, y, m->rows, gain, Pout, sso, st);
+    return qt_launch_few_gemm(m->prec, epi, m->w, m->scale, m->s16, m->rows, m->cols, P, n, ss, np, eps, y, m->rows, gain, Pout, sso,
+                              st);
 }
 
 /* Layer l after its attention (planes in f->a): O + residual, gate|up + SwiGLU, down + residual
@@ -954,7 +953,7 @@ static hipError_t pf_layers(talker_t *t, const dmat_t *wq, const dmat_t *wo, con
     const int x_planes = (long long)seq * H <= PF_PART_FLOATS;
     hipError_t e;
 #define PFE(x) do { if ((e = (x)) != hipSuccess) return e; } while (0)
-    if (qt_few_ok(seq, H, F, qd, qkvr)) {
+    if (qt_few_ok(QWEN_HIP_BF16, seq, H, F, qd, qkvr)) {
         /* at most 64 positions: one pass a projection (qt_few.hip), six launches a layer */
         const few_t *f = &t->pf_few;
         PFE(qt_launch_few_planes(t->pf_x, H, seq, H, s->in_norm[0], f->x, f->ss, t->st));
@@ -1077,7 +1076,7 @@ int qwen_hip_talker_prefill(void *state, const qwen_hip_layer_t *bf16_layers, co
         HCK(hipMalloc((void **)&t->pf_p, (size_t)3 * sp * km * sizeof(uint16_t)));
         HCK(hipMalloc((void **)&t->pf_part, (size_t)PF_PART_FLOATS * sizeof(float)));
         HCK(hipMalloc((void **)&t->pf_e, (size_t)seq * H * sizeof(float)));
-        if (qt_few_ok(1, H, F, qd, qkvr) && few_alloc(&t->pf_few, s) != 0) goto fail;
+        if (qt_few_ok(QWEN_HIP_BF16, 1, H, F, qd, qkvr) && few_alloc(&t->pf_few, s) != 0) goto fail;
         t->pf_cap = seq;
     }
     HCK(hipMemcpyAsync(t->pf_e, embeds, (size_t)seq * H * sizeof(float), hipMemcpyDefault, t->st));
@@ -1953,10 +1952,10 @@ fail:
  *   pieces(RMSNorm(x)) -> MFMA QKV -> attention (q/k norm, RoPE, KV append, split-K over
  *   each stream's own length, B streams in one grid) -> pieces(attn) -> MFMA O + residual
  *   -> pieces(RMSNorm(x)) -> MFMA gate|up + SwiGLU -> pieces(h) -> MFMA down + residual,
- * captured once into a hipGraph (positions live on the device).  bf16 and q4_0 weights take
- * qt_few.hip's projections (three exact bf16 activation planes on the bf16 MFMA, the norms
- * applied around the products, five launches a layer); past the widths and stream counts that
- * qt_few_ok states, bf16 takes the prefill's projection GEMM and q4_0 the int8 pieces into
+ * captured once into a hipGraph (positions live on the device).  Up to the widths and stream
+ * counts that qt_few_ok states the projections are qt_few.hip's instead (three exact bf16
+ * activation planes on the bf16 MFMA, the norms applied around the products, five launches a
+ * layer); past them bf16 takes the prefill's projection GEMM and q4_0 the int8 pieces into
  * qt_launch_bgemm_q4 (per-32-block integer sums, block scale in f32).  Every weight is read from
  * HBM once per step for all B streams in every precision. */
 
@@ -1970,10 +1969,11 @@ typedef struct {
     uint16_t *kc, *vc;         /* [B][L][nkv][kv_max][hd] */
     float *x, *qkv, *attn, *h, *hid;
     int8_t *pc; float *ps;     /* activation pieces [Kmax/64][3*Bp][64], scales [Bp] */
-    few_t few;                 /* bf16, q4_0: the projections' buffers (qt_few.hip) where it takes the shape, else (bf16) */
+    few_t few;                 /* the projections' buffers (qt_few.hip) where it takes the shape, else (bf16) */
     uint16_t *pf_p; float *pf_part; /* activation planes [3][64][Kmax], split-K partials (PF_PART_FLOATS) */
     int *g2_part; unsigned *g2_cnt; /* int8: split-K tiles and counters of qt_launch_bgemm2_i8 */
-    int fold;                  /* int8: pieces made inside each projection launch (qt_launch_bgemm2_i8_px) */
+    int fold;                  /* int8 pieces: made inside each projection launch (qt_launch_bgemm2_i8_px) */
+    int pieces;                /* int8: on the pieces although few has its buffers (qwen_hip_batch_fold_pieces) */
     unsigned *px_sync;         /* in-launch pieces: count + per-workgroup go flags (128-byte lines), error word */
     int px_wgs;                /* workgroups px_sync has flags for */
     float *part; unsigned *cnt;
@@ -2034,8 +2034,7 @@ static batch_t *batch_create(const stack_t *s, int B, int is_cp) {
     HCK(hipMalloc((void **)&bt->h, (size_t)B * s->F * sizeof(float)));
     HCK(hipMalloc((void **)&bt->pc, (size_t)K * 3 * bt->Bp));
     HCK(hipMalloc((void **)&bt->ps, (size_t)bt->Bp * sizeof(float)));
-    if (s->prec != QWEN_HIP_INT8 && qt_few_ok(B, s->H, s->F, s->qd, s->qd + 2 * s->kvd) &&
-        (s->prec == QWEN_HIP_BF16 || K <= 8192)) {
+    if (qt_few_ok(s->prec, B, s->H, s->F, s->qd, s->qd + 2 * s->kvd)) {
         if (few_alloc(&bt->few, s) != 0) goto fail;
     } else if (s->prec == QWEN_HIP_BF16) {
         HCK(hipMalloc((void **)&bt->pf_p, (size_t)3 * qt_pf_spad(B) * K * sizeof(uint16_t)));
@@ -2114,10 +2113,10 @@ static hipError_t batch_body(void *arg) {
     const float scale = 1.0f / sqrtf((float)s->hd);
     const int H = s->H, F = s->F, QKV = s->qd + 2 * s->kvd;
     const long long per = (long long)s->L * s->nkv * bt->kv_max * s->hd;
-    /* bf16 and q4_0 weights: each projection writes the next one's input planes (qt_few.hip); past
+    /* each projection writes the next one's input planes (qt_few.hip); past
      * its shapes, bf16: each reduce of the prefill's projections does (then only layer 0's input and
      * the attention output get a plane kernel of their own) */
-    const few_t *f = bt->few.x ? &bt->few : NULL;
+    const few_t *f = bt->few.x && !bt->pieces ? &bt->few : NULL;
     const int fused = !f && s->prec == QWEN_HIP_BF16 && (long long)bt->B * 2 * F <= PF_PART_FLOATS;
     if (fused && (e = qt_launch_pf_pieces(bt->x, H, bt->B, H, s->in_norm[0], s->eps, bt->pf_p, bt->st))) return e;
     if (f && (e = qt_launch_few_planes(bt->x, H, bt->B, H, s->in_norm[0], f->x, f->ss, bt->st))) return e;
@@ -2318,16 +2317,19 @@ fail:
 }
 /* int8 projections: make the activation pieces inside each projection launch (on = 1,
  * the default where every projection shape allows it) or in a launch of their own (0).
+ * A batch that runs on the bf16 planes (qt_few.hip) goes over to the pieces either way.
  * The two give the same bytes; the switch is for tests and measurement.  Returns the
  * mode in effect, -1 on error. */
 int qwen_hip_batch_fold_pieces(void *state, int on) {
     batch_t *bt = (batch_t *)state;
     if (!bt || bt->dead) { SETERR("batch state is dead or NULL"); return -1; }
     const int want = on && batch_px_ok(bt);
-    if (want != bt->fold) {
+    const int pieces = bt->s->prec == QWEN_HIP_INT8;
+    if (want != bt->fold || pieces != bt->pieces) {
         HCK(hipStreamSynchronize(bt->st));
         if (bt->graph_ready) { (void)hipGraphExecDestroy(bt->exec); bt->graph_ready = 0; }
         bt->fold = want;
+        bt->pieces = pieces;
     }
     return bt->fold;
 fail:

@@ -235,11 +235,11 @@ def test_batch_step_ragged_vs_oracle(oracle, prec, B):
     g.free()
 
 
-@pytest.mark.parametrize("prec", ["bf16", "int4"])
+@pytest.mark.parametrize("prec", ["bf16", "int8", "int4"])
 @pytest.mark.parametrize("name,B", [("tiny", 1), ("tiny", 31), ("mini", 5), ("mini", 16), ("mini", 49), ("mini17", 17),
                                     ("mini17", 64)])
 def test_batch_row_tiles_vs_oracle(oracle, name, B, prec):
-    """bf16 and q4_0 projections of B rows: whole and partial tiles of 16, K from a slice per wave up to 24,
+    """Projections of B rows: whole and partial tiles of 16, K from a slice per wave up to 24,
     every weight tile width.  Each stream is at one of three positions with that position's cache;
     the bars are the ragged test's."""
     from oracle.oracle import talker_from_tensors
