@@ -268,38 +268,49 @@ __global__ __launch_bounds__(QT_PF_WG) void k_pf_reduce_swiglu_planes(const floa
 // The residual epilogue of the summed K ranges for one position row per workgroup (Y[s] +=
 // acc, as k_pf_reduce<RESID>), then that row RMS-normalised with `gain` and written as the
 // next projection's three input planes (P[p][s][N], plane stride Sp*N; rows S <= s < Sp
-// zero): the row is kept in LDS and the norm and pieces are k_pf_pieces' arithmetic in its
-// order (thread t sums x[t + 256 j]^2, block_sum, (x * inv) * g), one launch fewer.
-__global__ __launch_bounds__(QT_PF_WG) void k_pf_reduce_resid_planes(const float *part, int nz, int S, int Sp, int N,
+// zero): one launch fewer than with k_pf_pieces.  A hundred rows leave most of the chip idle and
+// the time is the row's chain of latencies, so a row has eight waves (hidden 2048: one round of
+// loads, all of them issued before the sums) and a thread norms the elements that it summed: no
+// barrier but the statistic's.  1.7B: 128
+// positions 7.2 -> 5.8 us with eight waves for four, 512 8.1 -> 7.3.
+#define PF_ROW_T 512
+__global__ __launch_bounds__(PF_ROW_T) void k_pf_reduce_resid_planes(const float *part, int nz, int S, int Sp, int N,
                                                                      float *Y, int ldy, const float *gain, float eps,
                                                                      uint16_t *P) {
-    extern __shared__ __align__(16) float xr[];
-    __shared__ float red[QT_WAVES];
-    const int s = blockIdx.x, tid = threadIdx.x;
+    extern __shared__ __align__(16) float xr[];                // a thread's own elements, past its first four
+    __shared__ float red[PF_ROW_T / 64];
+    const int s = blockIdx.x, tid = threadIdx.x, n0 = 4 * tid;
     const size_t plane = (size_t)Sp * N;
     uint16_t *p0 = P + (size_t)s * N;
     if (s >= S) {
-        for (int k = tid * 8; k < N; k += QT_PF_WG * 8)
+        for (int k = tid * 8; k < N; k += PF_ROW_T * 8)
 #pragma unroll
             for (int p = 0; p < 3; p++) *reinterpret_cast<uint4 *>(p0 + p * plane + k) = make_uint4(0u, 0u, 0u, 0u);
         return;
     }
-    for (int n = 4 * tid; n < N; n += 4 * QT_PF_WG) {
-        const float4 acc = pf_sum_ranges(part, nz, S, N, s, n);
+    float4 first = make_float4(0.f, 0.f, 0.f, 0.f), g0 = first;
+    if (n0 < N) g0 = *reinterpret_cast<const float4 *>(gain + n0);
+    float ss = 0.f;
+    for (int n = n0; n < N; n += 4 * PF_ROW_T) {
         float4 *y = reinterpret_cast<float4 *>(Y + (size_t)s * ldy + n);
         const float4 o = *y;
+        const float4 acc = pf_sum_ranges(part, nz, S, N, s, n);
         const float4 r = make_float4(o.x + acc.x, o.y + acc.y, o.z + acc.z, o.w + acc.w);
         *y = r;
-        *reinterpret_cast<float4 *>(xr + n) = r;
+        if (n == n0) first = r;
+        else *reinterpret_cast<float4 *>(xr + n) = r;
+        ss = fmaf(r.w, r.w, fmaf(r.z, r.z, fmaf(r.y, r.y, fmaf(r.x, r.x, ss))));
     }
+    ss = group_sum<64>(ss);
+    if ((tid & 63) == 0) red[tid >> 6] = ss;
     __syncthreads();
-    float ss = 0.f;
-    for (int k = tid; k < N; k += QT_PF_WG) ss = fmaf(xr[k], xr[k], ss);
-    ss = block_sum(ss, red);
+    ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < PF_ROW_T / 64; i++) ss += red[i];
     const float inv = 1.0f / sqrtf(ss / (float)N + eps);
-    for (int k = tid * 4; k < N; k += QT_PF_WG * 4) {
-        float4 v = *reinterpret_cast<const float4 *>(xr + k);
-        const float4 g = *reinterpret_cast<const float4 *>(gain + k);
+    for (int k = n0; k < N; k += 4 * PF_ROW_T) {
+        float4 v = k == n0 ? first : *reinterpret_cast<const float4 *>(xr + k);
+        const float4 g = k == n0 ? g0 : *reinterpret_cast<const float4 *>(gain + k);
         v.x = (v.x * inv) * g.x; v.y = (v.y * inv) * g.y; v.z = (v.z * inv) * g.z; v.w = (v.w * inv) * g.w;
         uint16_t pc[3][4];
         const float e[4] = {v.x, v.y, v.z, v.w};
@@ -352,7 +363,9 @@ __global__ __launch_bounds__(QT_PF_WG) void k_pf_qkv_post(float *QKV, int ld, in
 
 // The q|k|v projection's summed K ranges for one position row per workgroup, kept in LDS,
 // then k_pf_qkv_post's work on that row (per-head q/k norm, RoPE, KV store) with the same
-// arithmetic; the row (q, k rotated, v as summed) is written once.  One launch fewer.
+// arithmetic; the row (q, k rotated, v as summed) is written once.  One launch fewer.  Sixteen
+// waves a row, for the same reason: one round of loads, two heads a wave.  1.7B: 128 positions 7.7 ->
+// 5.5 us with sixteen for four, 512 7.9 -> 6.9.
 struct PfQkvPost {
     int nh, nkv;
     const float *qn, *kn, *rc, *rs;
@@ -360,24 +373,25 @@ struct PfQkvPost {
     uint16_t *kc, *vc;
     long long kv_max;
 };
-__global__ __launch_bounds__(QT_PF_WG) void k_pf_reduce_qkv_post(const float *part, int nz, int S, int N, float *QKV,
+#define PF_QKV_T 1024
+__global__ __launch_bounds__(PF_QKV_T) void k_pf_reduce_qkv_post(const float *part, int nz, int S, int N, float *QKV,
                                                                  int ld, PfQkvPost a) {
     extern __shared__ __align__(16) float xr[];
     const int s = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int n = 4 * tid; n < N; n += 4 * QT_PF_WG)
+    const float c = a.rc[(size_t)s * 64 + lane], sn = a.rs[(size_t)s * 64 + lane];
+    const float qn0 = a.qn[lane], qn1 = a.qn[lane + 64], kn0 = a.kn[lane], kn1 = a.kn[lane + 64];
+    for (int n = 4 * tid; n < N; n += 4 * PF_QKV_T)
         *reinterpret_cast<float4 *>(xr + n) = pf_sum_ranges(part, nz, S, N, s, n);
     __syncthreads();
     float *row = QKV + (size_t)s * ld;
-    const float c = a.rc[(size_t)s * 64 + lane], sn = a.rs[(size_t)s * 64 + lane];
-    for (int hr = wave; hr < a.nh + 2 * a.nkv; hr += QT_WAVES) {
+    for (int hr = wave; hr < a.nh + 2 * a.nkv; hr += PF_QKV_T / 64) {
         float *x = row + hr * 128;
         const float x0 = xr[hr * 128 + lane], x1 = xr[hr * 128 + lane + 64];
         if (hr < a.nh + a.nkv) {
             const bool isk = hr >= a.nh;
-            const float *w = isk ? a.kn : a.qn;
             const float ss = group_sum<64>(x0 * x0 + x1 * x1);
             const float inv = 1.0f / sqrtf(ss / 128.0f + a.eps);
-            const float n0 = (x0 * inv) * w[lane], n1 = (x1 * inv) * w[lane + 64];
+            const float n0 = (x0 * inv) * (isk ? kn0 : qn0), n1 = (x1 * inv) * (isk ? kn1 : qn1);
             const float r0 = fmaf(n0, c, -(n1 * sn)), r1 = fmaf(n1, c, n0 * sn);
             x[lane] = r0;
             x[lane + 64] = r1;
@@ -744,7 +758,7 @@ static hipError_t pf_gemm(int epi, const uint16_t *W, const uint16_t *P, int S, 
         QT_PF_GEMM(QT_PF_PART, part, N)
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_pf_reduce_qkv_post, dim3(S), dim3(QT_PF_WG), (size_t)N * sizeof(float), st, part, sk, S, N, Y,
+        hipLaunchKernelGGL(k_pf_reduce_qkv_post, dim3(S), dim3(PF_QKV_T), (size_t)N * sizeof(float), st, part, sk, S, N, Y,
                            ldy, *qp);
     } else if (Pout) {
         QT_PF_GEMM(QT_PF_PART, part, N)
@@ -754,7 +768,7 @@ static hipError_t pf_gemm(int epi, const uint16_t *W, const uint16_t *P, int S, 
             hipLaunchKernelGGL(k_pf_reduce_swiglu_planes, dim3((Sp * N / 4 + QT_PF_WG - 1) / QT_PF_WG), dim3(QT_PF_WG), 0,
                                st, part, sk, S, Sp, N, Pout);
         else
-            hipLaunchKernelGGL(k_pf_reduce_resid_planes, dim3(Sp), dim3(QT_PF_WG), (size_t)N * sizeof(float), st, part, sk,
+            hipLaunchKernelGGL(k_pf_reduce_resid_planes, dim3(Sp), dim3(PF_ROW_T), (size_t)N * sizeof(float), st, part, sk,
                                S, Sp, N, Y, ldy, gain, eps, Pout);
     } else if (sk > 1) {
         QT_PF_GEMM(QT_PF_PART, part, N)
