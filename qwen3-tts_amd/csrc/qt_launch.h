@@ -220,7 +220,7 @@ hipError_t qt_launch_sd_dwln(const float *x, const float *dw, const float *db, c
                              float *out, int T, int C, int xlo, hipStream_t st);
 hipError_t qt_launch_sd_final(const float *x, const float *w, const float *b, float *audio, int T, int C, int xlo,
                               hipStream_t st);
-hipError_t qt_launch_sd_shift(float *buf, int H, int T, int C, hipStream_t st);
+hipError_t qt_launch_sd_shift(int n, float *const *buf, const int *H, const int *T, const int *C, hipStream_t st);
 #ifdef __cplusplus
 }
 #endif

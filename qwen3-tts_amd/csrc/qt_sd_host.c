@@ -721,18 +721,23 @@ static int sds_chunk(sds_t *q, int n) {
     }
     SCK(qt_launch_sd_final(sds_new_rows(&q->S[3]), s->fw, s->fb, q->daudio, T, 96, -q->S[3].H, st));
     /* histories for the next chunk: each buffer's last H rows (of H + its rows this chunk) */
-    SCK(qt_launch_sd_shift(q->V.p, q->V.H, n, 512, st));
-    for (int l = 0; l < 8; l++) SCK(qt_launch_sd_shift(q->Q[l].p, SDS_KH, n, 3072, st));
-    SCK(qt_launch_sd_shift(q->U[0].p, q->U[0].H, 2 * n, 1024, st));
-    SCK(qt_launch_sd_shift(q->U[1].p, q->U[1].H, 4 * n, 1024, st));
-    SCK(qt_launch_sd_shift(q->I.p, q->I.H, 4 * n, 1024, st));
-    SCK(qt_launch_sd_shift(q->C0.p, q->C0.H, 4 * n, 1536, st));
+    float *sb[32];
+    int sh[32], srows[32], sch[32], ns = 0;
+#define SHIFT(buf_, H_, T_, C_) (sb[ns] = (buf_), sh[ns] = (H_), srows[ns] = (T_), sch[ns] = (C_), ns++)
+    SHIFT(q->V.p, q->V.H, n, 512);
+    for (int l = 0; l < 8; l++) SHIFT(q->Q[l].p, SDS_KH, n, 3072);
+    SHIFT(q->U[0].p, q->U[0].H, 2 * n, 1024);
+    SHIFT(q->U[1].p, q->U[1].H, 4 * n, 1024);
+    SHIFT(q->I.p, q->I.H, 4 * n, 1024);
+    SHIFT(q->C0.p, q->C0.H, 4 * n, 1536);
     T = 4 * n;
     for (int b = 0; b < 4; b++) {
         T *= UP_RATE[b];
-        SCK(qt_launch_sd_shift(q->S[b].p, q->S[b].H, T, UP_CH[b], st));
-        for (int u = 0; u < 3; u++) SCK(qt_launch_sd_shift(q->F1[b][u].p, q->F1[b][u].H, T, UP_CH[b], st));
+        SHIFT(q->S[b].p, q->S[b].H, T, UP_CH[b]);
+        for (int u = 0; u < 3; u++) SHIFT(q->F1[b][u].p, q->F1[b][u].H, T, UP_CH[b]);
     }
+#undef SHIFT
+    SCK(qt_launch_sd_shift(ns, sb, sh, srows, sch, st));
     q->frames += n;
     return 0;
 }
