@@ -41,7 +41,7 @@ enum { SD_EPI_BIAS = 1, SD_EPI_GELU = 2, SD_EPI_CSCALE = 4, SD_EPI_RESID = 8, SD
 // One tensor of the reference's layout (element [n][k][column] at n * sn + k * sk + column * sc)
 // into channels [n0, n0 + nn) and k [k0, k0 + kk) of the packed weights (n0, k0: whole tiles).
 // Tap p of phase z is column p (stride 0: a conv or linear layer) or z + p * stride (zero past the
-// kernel's columns).  A value without planes (infinite, NaN or too large) sets *bad.
+// kernel's columns).  A value without planes (infinite or NaN) sets *bad.
 struct SdPackArgs {
     const float *src;
     long long sn, sk, sc;
@@ -61,8 +61,23 @@ __global__ __launch_bounds__(SD_WG) void k_sd_pack(SdPackArgs a) {
 #pragma unroll
     for (int i = 0; i < 8; i++)
         v[i] = (n < a.nn && k + i < a.kk && col < a.cols) ? a.src[n * a.sn + (k + i) * a.sk + col * a.sc] : 0.f;
+    // a finite value that rounds past bf16's range: its planes are cut instead of rounded (qt_put_pieces)
+    float big[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        big[i] = fabsf(v[i]) > 0x1.fep127f && fabsf(v[i]) < INFINITY ? v[i] : 0.f;
+        if (big[i] != 0.f) v[i] = 0.f;
+    }
     qt_u32x4 pl[3];
     qt_planes8(v, pl, chk);
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        if (big[i] != 0.f) {
+            uint16_t pc[3];
+            qt_put_pieces(pc, 1, big[i]);
+#pragma unroll
+            for (int q = 0; q < 3; q++) pl[q][i / 2] |= (uint32_t)pc[q] << (16 * (i & 1));
+        }
     if (chk != chk) *a.bad = 1;
     uint16_t *d = a.dst + ((((size_t)(a.k0 / 32 + kc) * a.ntap + p) * a.phases + z) * a.tiles + a.n0 / 16 + j) * 1536 + 8 * lane;
 #pragma unroll

@@ -189,6 +189,7 @@ def test_op_sd_conv_non_finite(cin, tile, what):
         x[7, 3], x[40, 0], x[41, 5], x[80, 9], x[60, 1] = np.inf, -np.inf, np.nan, np.inf, 3.395e38
         w[:, 1] = np.clip(w[:, 1], -0.1, 0.1)
         x[80, 10] = -np.inf
+        x[62, 1] = -3.40e38                       # finite, rounds to an infinite bf16
     else:
         w[3, 2, 0], w[9, 5, 2], w[20, 0, 1] = np.inf, np.nan, -np.inf
     y = np.empty((T, cout), np.float32)
@@ -200,6 +201,31 @@ def test_op_sd_conv_non_finite(cin, tile, what):
     assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isinf(y), np.isinf(want))
     inf, ok = np.isinf(want), np.isfinite(want)
     assert inf.any() and np.array_equal(np.sign(y[inf]), np.sign(want[inf]))
+    assert np.allclose(y[ok], want[ok], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("cin,tile", [(96, 16), (96, 128), (512, 16), (512, 32), (512, 64)])
+@pytest.mark.parametrize("beside", [0.0, np.inf])
+def test_op_sd_conv_weight_past_bf16_range(cin, tile, beside):
+    """A finite weight that rounds to an infinite bf16 (from 3.396e38 on) counts with its value, alone
+    and in a layer that holds an infinite weight as well.  The bounds are those of the test above."""
+    rng = np.random.default_rng(cin + tile)
+    T, cout = 70, 40
+    x = rng.standard_normal((T, cin)).astype(np.float32)
+    x[:, 7] = np.clip(x[:, 7], -0.1, 0.1)
+    w = (rng.standard_normal((cout, cin, 3)) / np.sqrt(cin * 3)).astype(np.float32)
+    w[30, 7, 1], w[31, 7, 0], w[5, 7, 2] = 3.40e38, -np.finfo(np.float32).max, 3.395e38
+    if beside:
+        w[12, 4, 1] = beside
+    y = np.empty((T, cout), np.float32)
+    hip.check(hip.lib().qwen_hip_op_sd_conv(y.ctypes.data, x.ctypes.data, w.ctypes.data, None, T, cin, cout, 3, 2, tile),
+              "op_sd_conv")
+    with np.errstate(invalid="ignore"):
+        xp = np.concatenate([np.zeros((4, cin)), x.astype(np.float64)])
+        want = sum((xp[2 * p:2 * p + T, None, :] * w[None, :, :, p].astype(np.float64)).sum(-1) for p in range(3))
+    ok = np.isfinite(want)
+    assert ok[:, 30].all() and np.abs(want[2:, [5, 30, 31]]).max() > 1e37 and ok[:, 12].all() == (beside == 0.0)
+    assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isinf(y), np.isinf(want))
     assert np.allclose(y[ok], want[ok], rtol=1e-5, atol=1e-5)
 
 
