@@ -203,8 +203,8 @@ hipError_t qt_launch_few_gemm(int prec, int epi, const void *W, const float *sca
 /* speech decoder (qt_sd.hip) */
 size_t qt_sd_pack_elems(int K, int N, int ntap, int phases);
 hipError_t qt_launch_sd_pack(const float *src, long long sn, long long sk, long long sc, int cols, int stride, int ntap,
-                             int phases, int N, int n0, int nn, int k0, int kk, uint16_t *dst, int *bad, hipStream_t st);
-hipError_t qt_launch_sd_gemm(const float *X, int ldx, int Tx, int xlo, const uint16_t *W, int serial, int K, int N, int ntap,
+                             int phases, int N, int n0, int nn, int k0, int kk, uint16_t *dst, hipStream_t st);
+hipError_t qt_launch_sd_gemm(const float *X, int ldx, int Tx, int xlo, const uint16_t *W, int K, int N, int ntap,
                              const int *off, int phases, int T, float *Y, int ldy, const float *bias, const float *cscale,
                              const float *R, const float *sa, const float *sib, float *Y2, int epi, int tile,
                              hipStream_t st);

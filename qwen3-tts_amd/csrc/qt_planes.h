@@ -31,6 +31,11 @@ __device__ __forceinline__ void qt_planes8(const float (&v)[8], qt_u32x4 (&p)[3]
     }
 }
 
+__device__ __forceinline__ void qt_planes8(const float (&v)[8], qt_u32x4 (&p)[3]) {
+    float unused = 0.f;
+    qt_planes8(v, p, unused);
+}
+
 // Activation planes in the matrix core's operand order, [k / 32][row tile][plane][64 lanes][8]
 // with lane = row % 16 + 16 (k % 32 / 8): where (row, k) of plane 0 is; the planes are 512 apart.
 __device__ __forceinline__ size_t qt_frag_at(int row_tiles, int row, int k) {

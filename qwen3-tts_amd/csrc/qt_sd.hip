@@ -41,14 +41,13 @@ enum { SD_EPI_BIAS = 1, SD_EPI_GELU = 2, SD_EPI_CSCALE = 4, SD_EPI_RESID = 8, SD
 // One tensor of the reference's layout (element [n][k][column] at n * sn + k * sk + column * sc)
 // into channels [n0, n0 + nn) and k [k0, k0 + kk) of the packed weights (n0, k0: whole tiles).
 // Tap p of phase z is column p (stride 0: a conv or linear layer) or z + p * stride (zero past the
-// kernel's columns).  A value without planes (infinite or NaN) sets *bad.
+// kernel's columns).  The planes of an infinite or NaN value give NaN sums (sd_redo).
 struct SdPackArgs {
     const float *src;
     long long sn, sk, sc;
     int cols, stride, ntap, phases, tiles;         // tiles: channel tiles of a phase
     int n0, nn, k0, kk;
     uint16_t *dst;
-    int *bad;
 };
 __global__ __launch_bounds__(SD_WG) void k_sd_pack(SdPackArgs a) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -57,7 +56,7 @@ __global__ __launch_bounds__(SD_WG) void k_sd_pack(SdPackArgs a) {
     const int kc = t / (a.ntap * nt), r = t - kc * a.ntap * nt, p = r / nt, j = r - p * nt;
     if (kc >= (a.kk + 31) / 32) return;
     const int n = 16 * j + (lane & 15), k = 32 * kc + 8 * (lane >> 4), col = a.stride ? z + p * a.stride : p;
-    float v[8], chk = 0.f;
+    float v[8];
 #pragma unroll
     for (int i = 0; i < 8; i++)
         v[i] = (n < a.nn && k + i < a.kk && col < a.cols) ? a.src[n * a.sn + (k + i) * a.sk + col * a.sc] : 0.f;
@@ -69,7 +68,7 @@ __global__ __launch_bounds__(SD_WG) void k_sd_pack(SdPackArgs a) {
         if (big[i] != 0.f) v[i] = 0.f;
     }
     qt_u32x4 pl[3];
-    qt_planes8(v, pl, chk);
+    qt_planes8(v, pl);
 #pragma unroll
     for (int i = 0; i < 8; i++)
         if (big[i] != 0.f) {
@@ -78,7 +77,6 @@ __global__ __launch_bounds__(SD_WG) void k_sd_pack(SdPackArgs a) {
 #pragma unroll
             for (int q = 0; q < 3; q++) pl[q][i / 2] |= (uint32_t)pc[q] << (16 * (i & 1));
         }
-    if (chk != chk) *a.bad = 1;
     uint16_t *d = a.dst + ((((size_t)(a.k0 / 32 + kc) * a.ntap + p) * a.phases + z) * a.tiles + a.n0 / 16 + j) * 1536 + 8 * lane;
 #pragma unroll
     for (int q = 0; q < 3; q++) *reinterpret_cast<qt_u32x4 *>(d + 512 * q) = pl[q];
@@ -92,7 +90,6 @@ struct SdGemmArgs {
     int off[SD_MAXTAP];
     int omin, span;                       // smallest offset; largest minus smallest
     int tps;                              // taps that share a staged slice (ntap, or 1 where span is too long)
-    int serial;                           // weights without planes: every output by sd_serial
     int T;                                // output rows per phase (t < T)
     float *Y; int ldy, os;                // output row t*os + phase
     const float *bias, *cscale;
@@ -112,26 +109,68 @@ __device__ __forceinline__ float sd_snake(float x, float a, float ib) {
     return fmaf(ib, s * s, x);
 }
 
-// Channels n..n+3 of output row t, phase z, one product after the other in f32: what a tile
-// falls back to when an operand has no planes (an infinite or NaN input must reach the
-// outputs that it reaches in plain arithmetic, and only those).
-__device__ __forceinline__ qt_f32x4 sd_serial(const SdGemmArgs &a, int t, int tile, int n) {
+// Channels n..n+3 of output row t from the f32 operands, by a whole wave: each lane takes units of
+// 8 k, in an order of their own that depends on nothing but the layer.  A channel's NaN is final:
+// the sum ends once every channel in `want` (bits) has one.
+__device__ __forceinline__ qt_f32x4 sd_redo(const SdGemmArgs &a, int t, int tile, int n, unsigned want, int lane) {
     qt_f32x4 s = {0.f, 0.f, 0.f, 0.f};
-    for (int p = 0; p < a.ntap; p++) {
-        const int xr = t + a.off[p];
-        const bool ok = t < a.T && xr >= a.xlo && xr < a.Tx;
-        for (int k = 0; k < a.K; k++) {
-            const float x = ok ? a.X[(ptrdiff_t)xr * a.ldx + k] : 0.f;
-            const uint16_t *w = a.W + (((size_t)(k / 32) * a.ntap + p) * a.phases * a.tiles + tile) * 1536 +
-                                8 * ((n & 15) + 16 * ((k % 32) / 8)) + k % 8;
+    const int units = 4 * a.slices * a.ntap;
+    for (int u0 = 0; u0 < units; u0 += 64) {
+        const int u = u0 + lane, kg = u & 3, kc = (u >> 2) / a.ntap, p = (u >> 2) - kc * a.ntap, k = 32 * kc + 8 * kg;
+        if (u < units && k < a.K) {
+            const int xr = t + a.off[p];
+            float4 x[2] = {make_float4(0.f, 0.f, 0.f, 0.f), make_float4(0.f, 0.f, 0.f, 0.f)};
+            if (xr >= a.xlo && xr < a.Tx) {
+                const float4 *src = reinterpret_cast<const float4 *>(a.X + (ptrdiff_t)xr * a.ldx + k);
+                x[0] = src[0]; x[1] = src[1];
+            }
+            const float xv[8] = {x[0].x, x[0].y, x[0].z, x[0].w, x[1].x, x[1].y, x[1].z, x[1].w};
+            const uint16_t *w = a.W + (((size_t)kc * a.ntap + p) * a.phases * a.tiles + tile) * 1536 + 8 * ((n & 15) + 16 * kg);
+#pragma unroll
             for (int r = 0; r < 4; r++) {
-                const float w0 = __uint_as_float((uint32_t)w[8 * r] << 16), w1 = __uint_as_float((uint32_t)w[8 * r + 512] << 16),
-                            w2 = __uint_as_float((uint32_t)w[8 * r + 1024] << 16);
-                s[r] = fmaf(x, (w0 - w0 == 0.f) ? w0 + (w1 + w2) : w0, s[r]);
+                qt_u32x4 wq[3];
+#pragma unroll
+                for (int q = 0; q < 3; q++) wq[q] = *reinterpret_cast<const qt_u32x4 *>(w + 8 * r + 512 * q);
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    float wf[3];
+#pragma unroll
+                    for (int q = 0; q < 3; q++) wf[q] = e & 1 ? qt_bf_hi(wq[q][e / 2]) : qt_bf_lo(wq[q][e / 2]);
+                    // an infinite or NaN weight is its first plane
+                    s[r] = fmaf(xv[e], fabsf(wf[0]) < INFINITY ? wf[0] + (wf[1] + wf[2]) : wf[0], s[r]);
+                }
             }
         }
+        bool open = false;
+#pragma unroll
+        for (int r = 0; r < 4; r++) open = open || ((want >> r & 1) && !__any(s[r] != s[r]));
+        if (!open) break;
     }
+#pragma unroll
+    for (int r = 0; r < 4; r++) s[r] = group_sum<64>(s[r]);
     return s;
+}
+
+// A sum of plane products is finite unless an operand is infinite, NaN or past bf16's range, or the
+// sum itself is out of range: then the planes cannot say whether the result is an infinity, a NaN or
+// a finite value, and that output is taken again from the f32 operands.  An output is redone for its
+// own operands only, so every other one keeps the bits that it has in any call and any tile; and what
+// it costs is a matter of the outputs concerned (a wave's latency each, the first product where the row is
+// NaN throughout).  Every lane of the wave calls this (v, t, tile, n: its own; live: its output exists).
+__device__ __forceinline__ qt_f32x4 sd_finite(const SdGemmArgs &a, qt_f32x4 v, int t, int tile, int n, bool live, int lane) {
+    unsigned bad = 0;
+#pragma unroll
+    for (int r = 0; r < 4; r++) bad |= fabsf(v[r]) < INFINITY ? 0u : 1u << r;
+    for (unsigned long long m = __ballot(live && bad); m; m &= m - 1) {
+        const int l = __builtin_ctzll(m);
+        const unsigned want = __builtin_amdgcn_readlane(bad, l);
+        const qt_f32x4 s = sd_redo(a, __builtin_amdgcn_readlane(t, l), __builtin_amdgcn_readlane(tile, l),
+                                   __builtin_amdgcn_readlane(n, l), want, lane);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if (lane == l && (want >> r & 1)) v[r] = s[r];
+    }
+    return v;
 }
 
 // The four channels n..n+3 (n: channel of the phase) of output row t: bias, GELU, column
@@ -187,7 +226,6 @@ __global__ __launch_bounds__(SD_WG) __attribute__((amdgpu_waves_per_eu(2))) void
     const int t0 = blockIdx.x * TT, all = a.phases * a.tiles;
     const int j0 = (blockIdx.y * WN + wave % WN) * NT, tw = 16 * MT * (wave / WN);
     const int rows = TT + (a.tps > 1 ? a.span : 0), ns = a.slices * (a.ntap / a.tps);
-    float chk = 0.f;
     float st[NU][8];
     unsigned ok = 0;
     auto fetch = [&](int s) {
@@ -214,7 +252,7 @@ __global__ __launch_bounds__(SD_WG) __attribute__((amdgpu_waves_per_eu(2))) void
 #pragma unroll
             for (int e = 0; e < 8; e++) v[e] = __uint_as_float(__float_as_uint(st[i][e]) & m);
             qt_u32x4 pl[3];
-            qt_planes8(v, pl, chk);
+            qt_planes8(v, pl);
             uint8_t *d = xs + buf * BUF + row * 64 + sd_unit(row, u & 3);
 #pragma unroll
             for (int p = 0; p < 3; p++) *reinterpret_cast<qt_u32x4 *>(d + p * PS) = pl[p];
@@ -278,10 +316,10 @@ __global__ __launch_bounds__(SD_WG) __attribute__((amdgpu_waves_per_eu(2))) void
         if (s + 1 < ns) put((s + 1) & 1);
         __syncthreads();
     }
-    const bool serial = __syncthreads_or(chk != chk || a.serial);
-    // the sums through LDS, so that a row's channels go out (and its residual comes in) together
+    // the sums through LDS (free: the last slice's barrier is behind), so that a row's channels go out (and its residual comes in) together
     constexpr int TN = 16 * WN * NT, LD = TN + 4;
     static_assert(TT * LD * 4 <= 2 * BUF, "the tile's sums fit in the staging buffers");
+    static_assert(TT * TN / 4 % SD_WG == 0, "no thread leaves the last loop early");
     float *ys = reinterpret_cast<float *>(xs);
 #pragma unroll
     for (int j = 0; j < NT; j++)
@@ -292,9 +330,10 @@ __global__ __launch_bounds__(SD_WG) __attribute__((amdgpu_waves_per_eu(2))) void
     __syncthreads();
     for (int e = tid; e < TT * TN / 4; e += SD_WG) {
         const int row = e / (TN / 4), c = 4 * (e % (TN / 4)), t = t0 + row, tile = blockIdx.y * (WN * NT) + c / 16;
-        if (tile >= all || t >= a.T) continue;
         const int z = tile / a.tiles, n = 16 * (tile - z * a.tiles) + c % 16;
-        sd_epilogue(a, t, z, n, serial ? sd_serial(a, t, tile, n) : *reinterpret_cast<qt_f32x4 *>(ys + row * LD + c));
+        const bool live = tile < all && t < a.T && n < a.N;
+        const qt_f32x4 v = sd_finite(a, *reinterpret_cast<qt_f32x4 *>(ys + row * LD + c), t, tile, n, live, lane);
+        if (live) sd_epilogue(a, t, z, n, v);
     }
 }
 
@@ -318,7 +357,6 @@ __global__ __launch_bounds__(64 * SD_GROUPS) void k_sd_split(SdGemmArgs a) {
     qt_u32x4 w[D][NT][3];
     float4 xa[D][MT], xb[D][MT];
     unsigned ok[D];
-    float chk = 0.f;
     auto fetch = [&](int it, int d) {
         const int kc = it / a.ntap, p = it - kc * a.ntap, k = 32 * kc + 8 * kg, o = a.off[p];
         unsigned m = 0;
@@ -355,7 +393,7 @@ __global__ __launch_bounds__(64 * SD_GROUPS) void k_sd_split(SdGemmArgs a) {
 #pragma unroll
                     for (int e = 0; e < 8; e++) v[e] = __uint_as_float(__float_as_uint(v[e]) & m);
                     qt_u32x4 pl[3];
-                    qt_planes8(v, pl, chk);
+                    qt_planes8(v, pl);
 #pragma unroll
                     for (int j = 0; j < NT; j++) acc[j][i] = qt_mma6(w[d][j], pl, acc[j][i]);
                 }
@@ -367,7 +405,7 @@ __global__ __launch_bounds__(64 * SD_GROUPS) void k_sd_split(SdGemmArgs a) {
     for (int j = 0; j < NT; j++)
 #pragma unroll
         for (int i = 0; i < MT; i++) part[wave][j * MT + i][lane] = acc[j][i];
-    const bool serial = __syncthreads_or(chk != chk || a.serial);
+    __syncthreads();
     for (int c = wave; c < NT * MT; c += SD_GROUPS) {
         const int j = c / MT, i = c - j * MT;
         if (j0 + j >= all) continue;
@@ -375,7 +413,7 @@ __global__ __launch_bounds__(64 * SD_GROUPS) void k_sd_split(SdGemmArgs a) {
         qt_f32x4 v = part[0][c][lane];
 #pragma unroll
         for (int g = 1; g < SD_GROUPS; g++) v += part[g][c][lane];
-        if (serial) v = sd_serial(a, t, j0 + j, n);
+        v = sd_finite(a, v, t, j0 + j, n, t < a.T && n < a.N, lane);
         sd_epilogue(a, t, z, n, v);
     }
 }
@@ -609,17 +647,18 @@ extern "C" size_t qt_sd_pack_elems(int K, int N, int ntap, int phases) {
 }
 extern "C" hipError_t qt_launch_sd_pack(const float *src, long long sn, long long sk, long long sc, int cols, int stride,
                                         int ntap, int phases, int N, int n0, int nn, int k0, int kk, uint16_t *dst,
-                                        int *bad, hipStream_t st) {
-    if (!src || !dst || !bad || n0 % 16 || k0 % 32 || nn <= 0 || kk <= 0 || n0 + nn > N) return hipErrorInvalidValue;
-    const SdPackArgs a = {src, sn, sk, sc, cols, stride, ntap, phases, (N + 15) / 16, n0, nn, k0, kk, dst, bad};
+                                        hipStream_t st) {
+    if (!src || !dst || n0 % 16 || k0 % 32 || nn <= 0 || kk <= 0 || n0 + nn > N) return hipErrorInvalidValue;
+    const SdPackArgs a = {src, sn, sk, sc, cols, stride, ntap, phases, (N + 15) / 16, n0, nn, k0, kk, dst};
     const int t = (kk + 31) / 32 * ntap * ((nn + 15) / 16);
     hipLaunchKernelGGL(k_sd_pack, dim3((t + QT_WAVES - 1) / QT_WAVES, 1, phases), dim3(SD_WG), 0, st, a);
     return hipGetLastError();
 }
 
 // tile: 0 = by size, 16, 32, 64 or 128 = rows per workgroup.  Every tile sums each output's
-// products in the same order, so the choice never changes a result bit.
-extern "C" hipError_t qt_launch_sd_gemm(const float *X, int ldx, int Tx, int xlo, const uint16_t *W, int serial, int K, int N,
+// products in the same order, and takes an output again (sd_finite) for that output's own operands
+// alone, so the choice never changes a result bit.
+extern "C" hipError_t qt_launch_sd_gemm(const float *X, int ldx, int Tx, int xlo, const uint16_t *W, int K, int N,
                                         int ntap, const int *off, int phases, int T, float *Y, int ldy, const float *bias,
                                         const float *cscale, const float *R, const float *sa, const float *sib,
                                         float *Y2, int epi, int tile, hipStream_t st) {
@@ -630,7 +669,7 @@ extern "C" hipError_t qt_launch_sd_gemm(const float *X, int ldx, int Tx, int xlo
     if ((epi & (SD_EPI_SNAKE | SD_EPI_SNAKE2)) && (!sa || !sib)) return hipErrorInvalidValue;
     if ((epi & SD_EPI_SNAKE2) && (!Y2 || (epi & SD_EPI_SNAKE))) return hipErrorInvalidValue;
     SdGemmArgs a;
-    a.X = X; a.ldx = ldx; a.Tx = Tx; a.xlo = xlo; a.W = W; a.serial = serial; a.K = K; a.N = N; a.ntap = ntap;
+    a.X = X; a.ldx = ldx; a.Tx = Tx; a.xlo = xlo; a.W = W; a.K = K; a.N = N; a.ntap = ntap;
     a.slices = (K + 31) / 32; a.tiles = (N + 15) / 16; a.phases = phases;
     int omax = off[0];
     a.omin = off[0];

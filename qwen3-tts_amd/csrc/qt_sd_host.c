@@ -28,13 +28,10 @@
 
 enum { SD_BIAS = 1, SD_GELU = 2, SD_CSCALE = 4, SD_RESID = 8, SD_SNAKE = 16, SD_SNAKE2 = 32 };
 
-#define SD_MAXCONV 80
-
 typedef struct {
     uint16_t *w; float *b;
     int K, N, ntap, phases;
     int off[8];
-    int id;                       /* index into the state's serial[] */
 } sd_conv_t;
 
 typedef struct { float *a, *ib; } sd_snake_t;
@@ -59,7 +56,6 @@ typedef struct {
     int cap;
     float *E, *V, *P, *H, *XN, *QKV, *A, *GU, *M, *LAT, *big[3];
     int *dcodes; float *daudio;
-    int n_convs, serial[SD_MAXCONV];  /* layers with a weight that has no planes (infinite or NaN) */
     void **allocs; int n_allocs, cap_allocs;
 } sd_t;
 
@@ -99,7 +95,6 @@ typedef struct {
     void *user;
     sd_t *s;
     float *tmp; size_t tmp_n;     /* device: the tensor being packed */
-    int *serial;                  /* device: [SD_MAXCONV] */
     int bad;
 } sd_ld_t;
 
@@ -162,12 +157,10 @@ static sd_conv_t sd_layer(sd_ld_t *L, int K, int N, int ntap, int phases) {
     sd_conv_t c; memset(&c, 0, sizeof c);
     c.K = K; c.N = N; c.ntap = ntap; c.phases = phases;
     if (L->bad) return c;
-    c.id = L->s->n_convs++;
-    if (!L->serial && (hipMalloc((void **)&L->serial, SD_MAXCONV * sizeof(int)) != hipSuccess ||
-                       hipMemsetAsync(L->serial, 0, SD_MAXCONV * sizeof(int), L->s->st) != hipSuccess)) L->bad = 1;
-    if (c.id >= SD_MAXCONV || !(c.w = (uint16_t *)sd_dalloc(L->s, qt_sd_pack_elems(K, N, ntap, phases) * sizeof(uint16_t))))
+    if (!(c.w = (uint16_t *)sd_dalloc(L->s, qt_sd_pack_elems(K, N, ntap, phases) * sizeof(uint16_t)))) {
+        qt_seterr("sd_init: device allocation failed");
         L->bad = 1;
-    if (L->bad) qt_seterr("sd_init: device allocation failed");
+    }
     return c;
 }
 
@@ -177,21 +170,18 @@ static void sd_pack(sd_ld_t *L, sd_conv_t *c, const char *wn, long long sn, long
                     int n0, int nn, int k0, int kk) {
     const float *w = sd_stage(L, wn, (long long)nn * kk * cols);
     if (L->bad) return;
-    if (qt_launch_sd_pack(w, sn, sk, sc, cols, stride, c->ntap, c->phases, c->N, n0, nn, k0, kk, c->w, L->serial + c->id,
-                          L->s->st) != hipSuccess) {
+    if (qt_launch_sd_pack(w, sn, sk, sc, cols, stride, c->ntap, c->phases, c->N, n0, nn, k0, kk, c->w, L->s->st) !=
+        hipSuccess) {
         qt_seterr("sd_init: packing %s failed", wn);
         L->bad = 1;
     }
 }
 
-/* which layers' weights have no planes, once every layer is packed; frees the loader's buffers */
+/* once every layer is packed: waits for it and frees the loader's buffer */
 static int sd_loaded(sd_ld_t *L) {
-    if (!L->bad && L->serial &&
-        (hipMemcpyAsync(L->s->serial, L->serial, SD_MAXCONV * sizeof(int), hipMemcpyDeviceToHost, L->s->st) != hipSuccess ||
-         hipStreamSynchronize(L->s->st) != hipSuccess)) L->bad = 1;
+    if (hipStreamSynchronize(L->s->st) != hipSuccess) L->bad = 1;
     if (L->tmp) (void)hipFree(L->tmp);
-    if (L->serial) (void)hipFree(L->serial);
-    L->tmp = NULL; L->serial = NULL;
+    L->tmp = NULL;
     return L->bad;
 }
 
@@ -228,7 +218,7 @@ void *qwen_hip_sd_init(qwen_hip_sd_get_fn get, void *user) {
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) { qt_seterr("sd_init: no HIP device"); return NULL; }
     sd_t *s = (sd_t *)calloc(1, sizeof *s);
     if (!s) { qt_seterr("sd_init: out of host memory"); return NULL; }
-    sd_ld_t L = {get, user, s, NULL, 0, NULL, 0};
+    sd_ld_t L = {get, user, s, NULL, 0, 0};
     char nm[160], nb[160];
     if (hipStreamCreateWithFlags(&s->st, hipStreamNonBlocking) != hipSuccess) { qt_seterr("sd_init: stream"); goto fail; }
     /* codebooks: EMA sums over usage, on the device */
@@ -334,7 +324,7 @@ void *qwen_hip_sd_init(qwen_hip_sd_get_fn get, void *user) {
         s->rope_s = sd_put(&L, c + SD_ROPE_POS * 32, (size_t)SD_ROPE_POS * 32);
         free(c);
     }
-    if (sd_loaded(&L) || hipStreamSynchronize(s->st) != hipSuccess) goto fail;
+    if (sd_loaded(&L)) goto fail;
     return s;
 fail:
     L.bad = 1;
@@ -372,14 +362,14 @@ static int sd_reserve(sd_t *s, int n) {
 
 static hipError_t sd_run(const sd_t *s, const sd_conv_t *c, const float *X, int Tx, int T, float *Y, int epi,
                          const float *cscale, const float *R) {
-    return qt_launch_sd_gemm(X, c->K, Tx, 0, c->w, s->serial[c->id], c->K, c->N, c->ntap, c->off, c->phases, T, Y, c->N,
+    return qt_launch_sd_gemm(X, c->K, Tx, 0, c->w, c->K, c->N, c->ntap, c->off, c->phases, T, Y, c->N,
                              c->b, cscale, R, NULL, NULL, NULL, epi | (c->b ? SD_BIAS : 0), 0, s->st);
 }
 
 /* the same with a snake on the output: in place (Y2 == NULL) or into Y2 beside Y */
 static hipError_t sd_run_snake(const sd_t *s, const sd_conv_t *c, const float *X, int Tx, int T, float *Y, int epi,
                                const float *R, const sd_snake_t *sn, float *Y2) {
-    return qt_launch_sd_gemm(X, c->K, Tx, 0, c->w, s->serial[c->id], c->K, c->N, c->ntap, c->off, c->phases, T, Y, c->N, c->b, NULL, R,
+    return qt_launch_sd_gemm(X, c->K, Tx, 0, c->w, c->K, c->N, c->ntap, c->off, c->phases, T, Y, c->N, c->b, NULL, R,
                              sn->a, sn->ib, Y2, epi | (c->b ? SD_BIAS : 0) | (Y2 ? SD_SNAKE2 : SD_SNAKE), 0, s->st);
 }
 
@@ -509,7 +499,7 @@ static int sd_op(float *Y, const float *X, const float *W, const float *bias, in
         return -1;
     }
     sd_one_t one = {W, (long long)Cout * Cin * k};
-    sd_ld_t L = {sd_one_get, &one, &tmp, NULL, 0, NULL, 0};
+    sd_ld_t L = {sd_one_get, &one, &tmp, NULL, 0, 0};
     if (hipStreamCreateWithFlags(&tmp.st, hipStreamNonBlocking) != hipSuccess) { qt_seterr("op_sd_conv: stream"); return -1; }
     sd_conv_t c = stride ? sd_convt(&L, "w", NULL, Cin, Cout, k, stride) : sd_conv(&L, "w", NULL, Cout, Cin, k, d);
     if (!L.bad && bias) c.b = sd_put(&L, bias, (size_t)Cout);
@@ -519,7 +509,7 @@ static int sd_op(float *Y, const float *X, const float *W, const float *bias, in
     if (hipMalloc((void **)&dx, (size_t)Tin * Cin * sizeof(float)) != hipSuccess ||
         hipMalloc((void **)&dy, (size_t)Tout * Cout * sizeof(float)) != hipSuccess) { qt_seterr("op_sd_conv: alloc"); goto done; }
     if (hipMemcpy(dx, X, (size_t)Tin * Cin * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) goto done;
-    if (qt_launch_sd_gemm(dx, Cin, Tin, 0, c.w, tmp.serial[c.id], Cin, Cout, c.ntap, c.off, c.phases, Tin, dy, Cout, c.b, NULL, NULL, NULL,
+    if (qt_launch_sd_gemm(dx, Cin, Tin, 0, c.w, Cin, Cout, c.ntap, c.off, c.phases, Tin, dy, Cout, c.b, NULL, NULL, NULL,
                           NULL, NULL, c.b ? SD_BIAS : 0, tile, tmp.st) != hipSuccess ||
         hipMemcpyAsync(Y, dy, (size_t)Tout * Cout * sizeof(float), hipMemcpyDeviceToHost, tmp.st) != hipSuccess ||
         hipStreamSynchronize(tmp.st) != hipSuccess) { qt_seterr("op_sd_conv: launch failed"); goto done; }
@@ -657,7 +647,7 @@ static hipError_t sds_gemm(const sd_t *s, const sd_conv_t *c, const float *X, in
                            const float *cscale, const float *R, const sd_snake_t *sn, float *Y2) {
     int e = epi | (c->b ? SD_BIAS : 0);
     if (sn) e |= Y2 ? SD_SNAKE2 : SD_SNAKE;
-    return qt_launch_sd_gemm(X, c->K, T, xlo, c->w, s->serial[c->id], c->K, c->N, c->ntap, c->off, c->phases, T, Y, c->N, c->b, cscale, R,
+    return qt_launch_sd_gemm(X, c->K, T, xlo, c->w, c->K, c->N, c->ntap, c->off, c->phases, T, Y, c->N, c->b, cscale, R,
                              sn ? sn->a : NULL, sn ? sn->ib : NULL, Y2, e, 0, s->st);
 }
 

@@ -204,6 +204,41 @@ def test_op_sd_conv_non_finite(cin, tile, what):
     assert np.allclose(y[ok], want[ok], rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("cin", [96, 512])
+@pytest.mark.parametrize("what", ["x", "w"])
+def test_op_sd_conv_non_finite_leaves_other_bits(cin, what):
+    """An output is taken again from its f32 operands for those operands alone: what no infinity or NaN
+    reaches keeps the bits of the clean call, and every tile gives the same result."""
+    rng = np.random.default_rng(cin)
+    T, cout = 150, 148
+    x = rng.standard_normal((T, cin)).astype(np.float32)
+    w = (rng.standard_normal((cout, cin, 3)) / np.sqrt(cin * 3)).astype(np.float32)
+
+    def run(tile):
+        y = np.empty((T, cout), np.float32)
+        hip.check(hip.lib().qwen_hip_op_sd_conv(y.ctypes.data, x.ctypes.data, w.ctypes.data, None, T, cin, cout, 3, 2, tile),
+                  "op_sd_conv")
+        return y
+
+    clean = run(64)
+    reached = np.zeros((T, cout), bool)
+    if what == "x":
+        w[:, 1] = np.clip(w[:, 1], -0.1, 0.1)
+        clean = run(64)
+        x[7, 3], x[40, 0], x[41, 5], x[100, 1] = np.inf, -np.inf, np.nan, 3.40e38
+        for r in (7, 40, 41, 100):
+            reached[[r, r + 2, r + 4]] = True
+    else:
+        w[3, 2, 0], w[97, 5, 2] = np.inf, np.nan
+        reached[:, [3, 97]] = True
+    outs = [run(t) for t in (16, 32, 64, 128)]
+    for y in outs:
+        assert np.array_equal(y[~reached].view(np.uint32), clean[~reached].view(np.uint32))
+        assert np.array_equal(y, outs[0], equal_nan=True)
+    want = np.isnan(outs[0])
+    assert want.any() and not want[~reached].any() and (what == "w" or np.isfinite(outs[0][100:105]).all())
+
+
 @pytest.mark.parametrize("cin,tile", [(96, 16), (96, 128), (512, 16), (512, 32), (512, 64)])
 @pytest.mark.parametrize("beside", [0.0, np.inf])
 def test_op_sd_conv_weight_past_bf16_range(cin, tile, beside):
