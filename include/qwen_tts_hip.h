@@ -201,11 +201,12 @@ int   qwen_hip_talker_batch_download_slot(void *state, int b, uint16_t *kv_k, ui
 int   qwen_hip_talker_batch_step_async(void *state, int n_steps);
 int   qwen_hip_talker_batch_sync(void *state);
 void *qwen_hip_talker_batch_stream(void *state);
-/* Test/measurement switch (no reference counterpart): int8 projections make their
- * activation pieces inside the projection launch (on = 1, the default wherever every
- * projection shape allows it) or in a launch of their own (0); both give the same bytes.
- * Applies to Talker and CP batch states; one that runs on the bf16 planes (few streams) goes
- * over to the pieces with the first call.  Returns the mode in effect, -1 on error. */
+/* Test/measurement switch (no reference counterpart): int8 projections run on the activation
+ * pieces, made inside the projection launch (on = 1, wherever every projection shape allows
+ * it) or in a launch of their own (0), the same bytes both ways; or as the batch was created
+ * (2): few streams on the bf16 planes, whose bits differ from the pieces', more as with 1.
+ * Applies to Talker and CP batch states of int8 weights.  Returns the mode in effect, -1 on
+ * error. */
 int   qwen_hip_batch_fold_pieces(void *state, int on);
 
 /* ---- level 2: Code Predictor (qwen_tts_cuda_talker.cu:751-841; qwen_tts_metal.m:2246) ---- */

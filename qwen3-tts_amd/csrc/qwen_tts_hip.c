@@ -2315,23 +2315,22 @@ fail:
     bt->dead = 1;
     return -1;
 }
-/* int8 projections: make the activation pieces inside each projection launch (on = 1,
- * the default where every projection shape allows it) or in a launch of their own (0).
- * A batch that runs on the bf16 planes (qt_few.hip) goes over to the pieces either way.
- * The two give the same bytes; the switch is for tests and measurement.  Returns the
- * mode in effect, -1 on error. */
+/* int8 projections on the activation pieces, made inside each projection launch (on = 1, where
+ * every projection shape allows it) or in a launch of their own (0): the same bytes both ways; or
+ * as the batch was created (2): few streams on the bf16 planes (qt_few.hip), more as with 1.  The
+ * switch is for tests and measurement.  Returns the mode in effect, -1 on error. */
 int qwen_hip_batch_fold_pieces(void *state, int on) {
     batch_t *bt = (batch_t *)state;
     if (!bt || bt->dead) { SETERR("batch state is dead or NULL"); return -1; }
     const int want = on && batch_px_ok(bt);
-    const int pieces = bt->s->prec == QWEN_HIP_INT8;
+    const int i8 = bt->s->prec == QWEN_HIP_INT8, pieces = i8 && on != 2;
     if (want != bt->fold || pieces != bt->pieces) {
         HCK(hipStreamSynchronize(bt->st));
         if (bt->graph_ready) { (void)hipGraphExecDestroy(bt->exec); bt->graph_ready = 0; }
         bt->fold = want;
         bt->pieces = pieces;
     }
-    return bt->fold;
+    return i8 && bt->few.x && !bt->pieces ? 2 : bt->fold;
 fail:
     bt->dead = 1;
     return -1;

@@ -461,11 +461,12 @@ class TalkerBatch:
         return res, out
 
     def fold_pieces(self, on):
-        """int8: activation pieces inside the projection launches (True) or apart; returns the mode in effect."""
-        r = lib().qwen_hip_batch_fold_pieces(self.h, int(bool(on)))
+        """int8: activation pieces inside the projection launches (True) or apart, or the route that the
+        batch was created with (None); returns the mode in effect (for None 2 is the bf16 planes)."""
+        r = lib().qwen_hip_batch_fold_pieces(self.h, 2 if on is None else int(bool(on)))
         if r < 0:
             raise RuntimeError("qwen_hip_batch_fold_pieces failed: " + last_error())
-        return bool(r)
+        return r if on is None else bool(r)
 
     def upload_slot(self, b, kv_k, kv_v, n):
         """kv_k/kv_v: [B][n_layers][src_kv_max][kv_dim] bf16 (the batch engine layout)."""

@@ -326,6 +326,33 @@ def test_batch_fold_pieces_matches_separate_launch(B):
     g.free()
 
 
+@pytest.mark.parametrize("B,created", [(5, 2), (48, 2), (49, 1)])
+def test_batch_fold_pieces_and_back(B, created):
+    """int8: the pieces give the same bytes inside the launches and apart, and a batch comes back to the
+    route that it was created with, bit for bit (the bf16 planes up to 48 streams of the 0.6B shape)."""
+    print(f"[case] fold pieces and back B={B}", flush=True)
+    _, shape, t = model_dir("mini")
+    cos, sin = synth.rope_tables(shape.head_dim, shape.rope_theta, 64)
+    g = hip.Talker(shape, hip.layers_from_tensors(t, shape), synth.bf16_to_f32(t["talker.model.norm.weight"]), cos, sin,
+                   hip.BF16, 64, quantize_to=hip.INT8)
+    bt = hip.TalkerBatch(g, B)
+    rng = np.random.default_rng(B)
+    pos = np.zeros(B, np.int32)
+    E = rng.normal(0, 0.5, (B, shape.hidden)).astype(np.float32)
+    first = bt.step(E, pos)
+    assert bt.fold_pieces(True)
+    inside = bt.step(E, pos)
+    assert not bt.fold_pieces(False)
+    apart = bt.step(E, pos)
+    assert bt.fold_pieces(None) == created
+    again, (_, layers) = bt.step(E, pos), bt.step_layers(E, pos)
+    assert np.array_equal(inside, apart) and np.array_equal(again, first) and np.array_equal(layers, first)
+    assert np.array_equal(inside, first) == (created == 1)
+    assert max(rel_l2(inside[b], first[b]) for b in range(B)) <= 1e-3
+    bt.free()
+    g.free()
+
+
 def test_batch_rejects_bad_arguments():
     shape = synth.SHAPES["tiny"]
     t = synth.generate(shape, 0x5EED0009, 0.0, threads=4, only=lambda n: n.startswith("talker.model."))
