@@ -294,6 +294,16 @@ int qwen_hip_op_swiglu(float *out, const float *gate_up, int n);
  * (epi 0), Y += that (epi 1), or SwiGLU of the interleaved gate|up rows into Y[S][N/2]
  * (epi 2); W bf16, f32 host arrays, N and K multiples of 64. */
 int qwen_hip_op_prefill_gemm(float *Y, const uint16_t *W, const float *X, int S, int N, int K, int epi);
+/* One projection of a few rows alone, as a batched step of few streams and a short prompt run it
+ * (no reference counterpart as one call): host arrays, W [N][K] of the given precision (int8 with
+ * its row scales, q4_0 as blocks), X f32 [S][K], gain [K], S <= 64, N and K multiples of 64.
+ * epi 0: Y[S][N] = RMSNorm(X) . W^T;  epi 1: Y += (X gain) . W^T, and next_gain [N] gives planes
+ * [3][S][N], whose sum is Y next_gain, and sums [S][N/16], the sums of squares of 16 columns each
+ * (N <= 4096);
+ * epi 2: planes [3][S][N/2] of the SwiGLU of RMSNorm(X) . W^T (interleaved gate|up rows).  What an
+ * epilogue does not name may be NULL. */
+int qwen_hip_op_few_gemm(int prec, int epi, float *Y, const void *W, const float *scale, const float *X, int S, int N, int K,
+                         const float *gain, float eps, const float *next_gain, float *planes, float *sums);
 /* The prefill's causal attention alone (qwen_causal_attention, k.c:3454-3560, as
  * t.c:904-907 calls it): out f32[S][nh*128] from QKV f32[S][(nh + 2 nkv)*128] holding the
  * normed, rotated q | k | v rows of every position. */

@@ -2731,6 +2731,67 @@ fail:
     return -1;
 }
 
+/* One projection of a few rows (qt_few.hip) on its own, host pointers: the rows X[S][K] times gain
+ * as planes, and by epi (QT_PF_*) Y = RMSNorm(X) . W^T, Y += (X gain) . W^T with the planes of
+ * Y next_gain and the sums of squares of each 16 columns of Y, or the planes of the SwiGLU of
+ * RMSNorm(X) . W^T. */
+int qwen_hip_op_few_gemm(int prec, int epi, float *Y, const void *W, const float *scale, const float *X, int S, int N, int K,
+                         const float *gain, float eps, const float *next_gain, float *planes, float *sums) {
+    hipStream_t st = op_stream();
+    dmat_t m; memset(&m, 0, sizeof m);
+    float *dx = NULL, *dg = NULL, *dn = NULL, *dy = NULL, *ss = NULL, *so = NULL;
+    uint16_t *dp = NULL, *dpo = NULL, *hp = NULL;
+    void *tmp = NULL;
+    qwen_hip_mat_t src = {W, scale};
+    int rc = -1;
+    REQ(st, "no stream");
+    REQ(S >= 1 && S <= 64 && N >= 64 && K >= 64 && N % 64 == 0 && K % 64 == 0 && epi >= QT_PF_STORE && epi <= QT_PF_SWIGLU &&
+        prec >= QWEN_HIP_BF16 && prec <= QWEN_HIP_Q4_0, "bad shape/epi/precision");
+    REQ(W && X && gain && (epi == QT_PF_SWIGLU || Y) && (epi == QT_PF_STORE || planes) && (epi != QT_PF_RESID || (next_gain && sums)),
+        "null argument");
+    const int C = epi == QT_PF_SWIGLU ? N / 2 : N, rt = (S + 15) / 16;
+    const size_t ne = qt_few_planes_elems(S, C);
+    REQ(dmat_alloc(&m, prec, N, K) == 0, "alloc");
+    if (prec == QWEN_HIP_Q4_0) HCK(hipMalloc(&tmp, (size_t)N * (K / 32) * 18 + 16));
+    REQ(dmat_put(&m, 0, &src, prec, N, st, tmp) == 0, "upload");
+    REQ((dx = up_f32(X, (size_t)S * K, st)) && (dg = up_f32(gain, K, st)), "upload");
+    HCK(hipMalloc((void **)&dp, qt_few_planes_elems(S, K) * sizeof(uint16_t)));
+    HCK(hipMalloc((void **)&ss, (size_t)S * qt_few_first() * sizeof(float)));
+    HCK(qt_launch_few_planes(dx, K, S, K, dg, dp, ss, st));
+    if (epi == QT_PF_RESID) {
+        REQ((dy = up_f32(Y, (size_t)S * N, st)) && (dn = up_f32(next_gain, N, st)), "upload");
+        HCK(hipMalloc((void **)&so, (size_t)S * (N / 16) * sizeof(float)));
+    } else if (epi == QT_PF_STORE) {
+        HCK(hipMalloc((void **)&dy, (size_t)S * N * sizeof(float)));
+    }
+    if (epi != QT_PF_STORE) {
+        HCK(hipMalloc((void **)&dpo, ne * sizeof(uint16_t)));
+        REQ((hp = malloc(ne * sizeof(uint16_t))) != NULL, "host alloc");
+    }
+    HCK(few_proj(&m, epi, dp, S, ss, qt_few_first(), eps, dy, dn, dpo, so, st));
+    if (dy) HCK(hipMemcpyAsync(Y, dy, (size_t)S * N * sizeof(float), hipMemcpyDeviceToHost, st));
+    if (so) HCK(hipMemcpyAsync(sums, so, (size_t)S * (N / 16) * sizeof(float), hipMemcpyDeviceToHost, st));
+    if (dpo) HCK(hipMemcpyAsync(hp, dpo, ne * sizeof(uint16_t), hipMemcpyDeviceToHost, st));
+    HCK(hipStreamSynchronize(st));
+    if (dpo)
+        for (int p = 0; p < 3; p++)
+            for (int r = 0; r < S; r++)
+                for (int k = 0; k < C; k++) {           /* qt_frag_at's order */
+                    const size_t at = ((size_t)((k >> 5) * rt + (r >> 4)) * 3 + p) * 512 + ((r & 15) + 16 * ((k & 31) >> 3)) * 8 + (k & 7);
+                    const uint32_t u = (uint32_t)hp[at] << 16;
+                    memcpy(&planes[((size_t)p * S + r) * C + k], &u, sizeof u);
+                }
+    rc = 0;
+fail:
+    dmat_free(&m);
+    {
+        void *b[] = {dx, dg, dn, dy, ss, so, dp, dpo, tmp};
+        for (size_t i = 0; i < sizeof b / sizeof b[0]; i++) if (b[i]) (void)hipFree(b[i]);
+    }
+    free(hp);
+    return rc;
+}
+
 /* The prefill's causal attention alone: out[S][nh*128] from QKV host f32[S][(nh+2nkv)*128]
  * (q | k | v rows as the prefill holds them after norm and RoPE). */
 int qwen_hip_op_prefill_attention(float *out, const float *QKV, int S, int nh, int nkv, float scale) {

@@ -36,7 +36,7 @@ EXPORTS = [
     "qwen_hip_cp_batch_init", "qwen_hip_cp_batch_step", "qwen_hip_cp_batch_free", "qwen_hip_op_matmat_int8", "qwen_hip_op_matmat_q4_0",
     "qwen_hip_cp_set_prefill2", "qwen_hip_cp_prefill2",
     "qwen_hip_talker_prefill", "qwen_hip_talker_prefill_async", "qwen_hip_op_prefill_gemm",
-    "qwen_hip_op_prefill_attention", "qwen_hip_talker_step_layers", "qwen_hip_op_matmat_int8_noalloc",
+    "qwen_hip_op_few_gemm", "qwen_hip_op_prefill_attention", "qwen_hip_talker_step_layers", "qwen_hip_op_matmat_int8_noalloc",
     "qwen_hip_generate", "qwen_hip_talker_load_file",
     "qwen_hip_sd_init", "qwen_hip_sd_load_file", "qwen_hip_sd_decode", "qwen_hip_sd_decode_device",
     "qwen_hip_sd_latent", "qwen_hip_sd_stream", "qwen_hip_sd_free", "qwen_hip_op_sd_conv",
@@ -103,6 +103,8 @@ def lib():
         L.qwen_hip_talker_prefill.argtypes = [vp, vp, vp, i]; L.qwen_hip_talker_prefill.restype = i
         L.qwen_hip_talker_prefill_async.argtypes = [vp, i, i]; L.qwen_hip_talker_prefill_async.restype = i
         L.qwen_hip_op_prefill_gemm.argtypes = [vp, vp, vp, i, i, i, i]; L.qwen_hip_op_prefill_gemm.restype = i
+        L.qwen_hip_op_few_gemm.argtypes = [i, i, vp, vp, vp, vp, i, i, i, vp, f, vp, vp, vp]
+        L.qwen_hip_op_few_gemm.restype = i
         L.qwen_hip_op_prefill_attention.argtypes = [vp, vp, i, i, i, C.c_float]
         L.qwen_hip_op_prefill_attention.restype = i
         L.qwen_hip_talker_download_kv.argtypes = [vp, vp, vp, i, i]; L.qwen_hip_talker_download_kv.restype = i
