@@ -269,6 +269,62 @@ def test_batch_row_tiles_vs_oracle(oracle, name, B, prec):
     g.free()
 
 
+@pytest.mark.parametrize("prec,pieces", [("bf16", False), ("int8", False), ("int8", True), ("int4", False)])
+@pytest.mark.parametrize("name,at", [("mini", (383, 767, 1000)),
+                                     ("tiny", (382, 383, 384, 385, 0, 766, 767, 768, 769, 31, 1000, 1150, 1151, 1152, 400, 800, 1))])
+def test_batch_long_caches_vs_oracle(oracle, name, at, prec, pieces):
+    """Caches around the edges of the 384-key chunks that at most 128 (stream, kv head) pairs are split
+    into, so that the last chunk's workgroup merges up to four of them, into planes (three, or
+    seventeen rows: two row tiles) or, on the int8 pieces, into f32 rows; two steps, so that the second one's
+    chunks hold the first one's keys and the arrival counters are used again."""
+    print(f"[case] batch long caches {prec} {name} pieces={pieces}", flush=True)
+    from oracle.oracle import talker_from_tensors
+    _, shape, t = model_dir(name)
+    B, kv_max = len(at), 1200
+    cos, sin = synth.rope_tables(shape.head_dim, shape.rope_theta, kv_max)
+    g = hip.Talker(shape, hip.layers_from_tensors(t, shape), synth.bf16_to_f32(t["talker.model.norm.weight"]), cos, sin,
+                   hip.BF16, kv_max, quantize_to=-1 if prec == "bf16" else hip.PREC[prec])
+    ot, keep = talker_from_tensors(oracle, t, shape, prec, kv_max, cos, sin)
+    rng = np.random.default_rng(B)
+    kv = [synth.f32_to_bf16_rne(rng.standard_normal((B,) + keep["kv_k"].shape, dtype=np.float32)) for _ in range(2)]
+    bt = hip.TalkerBatch(g, B)
+    if pieces:
+        bt.fold_pieces(True)
+    for b in range(B):
+        bt.upload_slot(b, kv[0], kv[1], at[b])
+    pos = np.array(at, np.int32)
+    E = rng.normal(0, 0.5, (2, B, shape.hidden)).astype(np.float32)
+    got = [bt.step(E[i], pos + i) for i in range(2)]
+    for b in range(B):
+        keep["kv_k"][:], keep["kv_v"][:] = kv[0][b], kv[1][b]
+        for i in range(2):
+            want, _ = oracle.talker_step(ot, E[i, b], at[b] + i)
+            assert rel_l2(got[i][b], want) <= 1e-3 and np.abs(got[i][b] - want).max() <= 2e-2, (i, b, rel_l2(got[i][b], want))
+    bt.free()
+    g.free()
+
+
+@pytest.mark.parametrize("prec", ["bf16", "int8", "int4"])
+def test_batch_non_finite_stream_alone(prec):
+    """An input with an infinity, a NaN or squares that overflow ends in its own stream's row."""
+    print(f"[case] batch non-finite stream {prec}", flush=True)
+    _, shape, t = model_dir("tiny")
+    cos, sin = synth.rope_tables(shape.head_dim, shape.rope_theta, 64)
+    g = hip.Talker(shape, hip.layers_from_tensors(t, shape), synth.bf16_to_f32(t["talker.model.norm.weight"]), cos, sin,
+                   hip.BF16, 64, quantize_to=-1 if prec == "bf16" else hip.PREC[prec])
+    B, pos = 19, np.zeros(19, np.int32)
+    bt = hip.TalkerBatch(g, B)
+    E = np.random.default_rng(1).normal(0, 0.5, (B, shape.hidden)).astype(np.float32)
+    clean = bt.step(E, pos)
+    E[3, 7], E[17, 0] = np.inf, np.nan
+    E[11] *= 1e25
+    got = bt.step(E, pos)
+    rest = np.delete(np.arange(B), [3, 11, 17])
+    assert np.array_equal(got[rest], clean[rest]) and np.isnan(got[[3, 17]]).all() and not got[11].any()
+    bt.free()
+    g.free()
+
+
 @need_ref
 def test_batch_of_identical_streams_matches_single_step():
     """B copies of one stream (the reference's batch self-test, cu:657-730 /
@@ -392,6 +448,34 @@ def test_cp_batch_step_vs_oracle(oracle, prec):
             want = np.array(x[b], copy=True)
             assert oracle.lib.qo_cp_pass(C.byref(streams[b][0]), want.ctypes.data, p) == 0
             assert rel_l2(got[b], want) <= 1e-3, (p, b, rel_l2(got[b], want))
+    cp.free()
+
+
+@pytest.mark.parametrize("prec", ["bf16", "int8", "int4"])
+@pytest.mark.parametrize("name,B", [("tiny", 33), ("mini", 6), ("mini", 17), ("mini", 50)])
+def test_cp_batch_tiles_vs_oracle(oracle, name, B, prec):
+    """The batched Code Predictor pass over whole and partial row tiles, at ragged positions, up to and
+    past the stream counts of the few-rows projections (int8: 48): every stream's residual after each of
+    three passes, and at 0, against the oracle's pass on that stream's own cache."""
+    from oracle.oracle import talker_from_tensors
+    print(f"[case] CP batch {prec} {name} B={B}", flush=True)
+    _, shape, t = model_dir(name)
+    cp = hip.cp_from_tensors(t, shape, hip.PREC[prec])
+    cos, sin = synth.rope_tables(shape.cp_head_dim, shape.rope_theta, 64)
+    ot, keep = talker_from_tensors(oracle, t, shape, prec, 64, cos, sin, cp=True)
+    cache = [np.zeros((B,) + keep["kv_k"].shape, np.uint16) for _ in range(2)]
+    rng = np.random.default_rng(B)
+    pos = np.zeros(B, np.int32)
+    for it in range(3):
+        x = rng.standard_normal((B, shape.cp_hidden)).astype(np.float32)
+        got = cp.batch_step(x, pos)
+        for b in range(B):
+            keep["kv_k"][:], keep["kv_v"][:] = cache[0][b], cache[1][b]
+            want = np.array(x[b], copy=True)
+            assert oracle.lib.qo_cp_pass(C.byref(ot), want.ctypes.data, int(pos[b])) == 0
+            cache[0][b], cache[1][b] = keep["kv_k"], keep["kv_v"]
+            assert rel_l2(got[b], want) <= 1e-3, (it, b, rel_l2(got[b], want))
+        pos += np.arange(B, dtype=np.int32) % 2         # half of the streams take position 0 again
     cp.free()
 
 

@@ -182,10 +182,11 @@ def test_prefill_async_replays_reproduce_the_prefill():
 
 
 @pytest.mark.parametrize("name,seq", [("mini", 100), ("mini17", 40), ("mini", 240), ("tiny", 64), ("mini", 65), ("mini17", 49),
-                                      ("mini", 1)])
+                                      ("mini", 1), ("mini", 45), ("mini", 64), ("mini17", 17), ("mini17", 32), ("mini17", 33)])
 def test_prefill_matches_oracle_layer_shapes(oracle, name, seq):
     """The 0.6B / 1.7B layer shapes (2 layers) against the oracle prefill, then one decode
-    step from each side's KV.  240 positions leave 16 padding rows in the O projection's planes."""
+    step from each side's KV.  240 positions leave 16 padding rows in the O projection's planes; up to 64
+    (1.7B: 32) the projections are those of a few rows."""
     from oracle.oracle import talker_from_tensors
     print(f"[case] prefill oracle {name} seq={seq}", flush=True)
     d, shape, t = model_dir(name)
@@ -206,6 +207,25 @@ def test_prefill_matches_oracle_layer_shapes(oracle, name, seq):
     h = tk.step(x, seq)
     h_o, _ = oracle.talker_step(ot, x, seq)
     assert rel_l2(h, h_o) <= 1e-3
+    tk.free()
+
+
+@pytest.mark.parametrize("seq", [21, 64, 90])
+def test_prefill_non_finite_position(seq):
+    """A NaN input leaves the cache rows of the positions before it as they are, on the few-rows
+    projections (up to 64 positions) and past them."""
+    _, shape, t = model_dir("tiny")
+    cos, sin = synth.rope_tables(shape.head_dim, shape.rope_theta, 128)
+    tk = hip.Talker(shape, hip.layers_from_tensors(t, shape), synth.bf16_to_f32(t["talker.model.norm.weight"]), cos, sin,
+                    hip.BF16, 128)
+    e = np.random.default_rng(seq).normal(0, 0.5, (seq, shape.hidden)).astype(np.float32)
+    tk.prefill(e)
+    k, v = tk.download_kv(seq)
+    e[18, 3] = np.nan
+    assert np.isnan(tk.prefill(e)).all()
+    k2, v2 = tk.download_kv(seq)
+    assert _kv_close(k2[:, :18], k[:, :18]) and _kv_close(v2[:, :18], v[:, :18])
+    assert np.isnan(synth.bf16_to_f32(k2[:, 18])).all()
     tk.free()
 
 
