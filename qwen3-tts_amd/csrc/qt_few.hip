@@ -23,7 +23,8 @@
 //     sums start from zero, and its f16 scale multiplies them in f32;
 //   * RMSNorm is applied around the product: the planes are those of x * gain, each maker of
 //     16 columns of x leaves the sum of their squares (one float a row), and the consumer
-//     scales its sums by 1/rms: the row's statistic needs no launch of its own.
+//     scales its sums by 1/rms: the row's statistic needs no launch of its own.  (An x whose
+//     square overflows is cut, qf_cut.)
 #include "qt_planes.h"
 
 #define QF_W 8                   // waves of a workgroup, and parts of K
@@ -60,6 +61,12 @@ __device__ __forceinline__ void qf_put4(uint16_t *P, int RT, int row, int k, qt_
         *reinterpret_cast<uint2 *>(d + 512 * p) =
             make_uint2((uint32_t)pc[p][0] | ((uint32_t)pc[p][1] << 16), (uint32_t)pc[p][2] | ((uint32_t)pc[p][3] << 16));
 }
+
+// x as the planes of x * gain take it: past 2^64 its square alone is past f32's range, the row's 1/rms
+// is 0 and its result 0 (as x (1/rms) is), whatever finite value x has; cut there, the sums that the 0
+// multiplies stay finite.  An infinity or a NaN stays one.
+__device__ __forceinline__ float qf_cut(float x) { return fabsf(x) > 0x1p64f && fabsf(x) < INFINITY ? copysignf(0x1p64f, x) : x; }
+__device__ __forceinline__ qt_f32x4 qf_cut4(qt_f32x4 v) { return qt_f32x4{qf_cut(v[0]), qf_cut(v[1]), qf_cut(v[2]), qf_cut(v[3])}; }
 
 // 8 weights as a lane's operand: bf16 as they are, int8 converted (exact), q4_0 nibbles (element e in bits 4 e, + 8) unpacked
 template <int PREC> struct QfWord { using t = qt_u32x4; };
@@ -229,8 +236,10 @@ __global__ __launch_bounds__(QF_T) void k_few(QtFewArgs a) {
         v = old + v;
         *reinterpret_cast<qt_f32x4 *>(a.Y + (size_t)row * a.ldy + n) = v;
         if (a.Pout) {
-            qf_put4(a.Pout, a.RT, row, n, v * gn);
             float sq = fmaf(v[3], v[3], fmaf(v[2], v[2], fmaf(v[1], v[1], v[0] * v[0])));
+            qt_f32x4 c = v;
+            if (__any(!(sq < INFINITY))) c = qf_cut4(v);
+            qf_put4(a.Pout, a.RT, row, n, c * gn);
             sq += __shfl_xor(sq, 16);              // a row's four lanes are all in the tile or all past S
             sq += __shfl_xor(sq, 32);
             if (kg == 0) a.sspo[(size_t)row * (a.N / 16) + blockIdx.x * NT + wave] = sq;
@@ -251,7 +260,7 @@ __global__ __launch_bounds__(256) void k_few_planes(const float *X, int ldx, int
     for (int k = 4 * threadIdx.x; k < K; k += 1024) {
         qt_f32x4 v = *reinterpret_cast<const qt_f32x4 *>(x + k);
         ss = fmaf(v[3], v[3], fmaf(v[2], v[2], fmaf(v[1], v[1], fmaf(v[0], v[0], ss))));
-        qf_put4(P, RT, row, k, v * *reinterpret_cast<const qt_f32x4 *>(gain + k));
+        qf_put4(P, RT, row, k, qf_cut4(v) * *reinterpret_cast<const qt_f32x4 *>(gain + k));
     }
     ss = block_sum(ss, red);
     if (threadIdx.x < QF_FIRST) ssp[row * QF_FIRST + threadIdx.x] = threadIdx.x ? 0.f : ss;

@@ -117,22 +117,26 @@ def test_op_few_gemm_planes_are_exact(prec):
 @pytest.mark.parametrize("prec", ["bf16", "int8", "q4_0"])
 def test_op_few_gemm_non_finite_rows(oracle, prec):
     """An infinity or a NaN makes its row NaN (the norm's 0 times infinity), a row whose squares overflow
-    becomes 0 as x * (1 / rms) does, and no other row changes by a bit."""
+    becomes 0 as x * (1 / rms) does, up to the largest float, and no other row changes by a bit."""
     S, N, K = 37, 128, 512
     rng = np.random.default_rng(3)
     W, scale, _ = _weights(oracle, prec, synth.f32_to_bf16_rne((rng.standard_normal((N, K)) * 0.05).astype(np.float32)))
     X = rng.standard_normal((S, K)).astype(np.float32)
-    gain, ng = (1 + 0.1 * rng.standard_normal(K)).astype(np.float32), np.ones(N, np.float32)
-    clean = [_few(prec, e, W, scale, X, N, gain, None, ng) for e in (STORE, RESID, SWIGLU)]
+    gain, ng = (1 + 0.1 * rng.standard_normal(K)).astype(np.float32), (1 + 0.1 * rng.standard_normal(N)).astype(np.float32)
+    Y0 = rng.standard_normal((S, N)).astype(np.float32)
+    clean = [_few(prec, e, W, scale, X, N, gain, Y0, ng) for e in (STORE, RESID, SWIGLU)]
     X[2, 5], X[17, 511], X[36, 0] = np.inf, np.nan, -np.inf
     X[20] *= 1e25
-    nan, rest = [2, 17, 36], np.delete(np.arange(S), [2, 17, 20, 36])
-    got = [_few(prec, e, W, scale, X, N, gain, None, ng) for e in (STORE, RESID, SWIGLU)]
-    assert np.isnan(got[0][0][nan]).all() and not got[0][0][20].any()
-    assert np.array_equal(got[0][0][rest], clean[0][0][rest])
-    assert not np.isfinite(got[1][0][nan]).any() and np.isfinite(got[1][0][20]).all()
-    assert not np.isfinite(got[1][2][nan]).any() and np.isinf(got[1][2][20]).any()
-    assert np.array_equal(got[1][0][rest], clean[1][0][rest]) and np.array_equal(got[1][2][rest], clean[1][2][rest])
-    assert np.array_equal(got[1][1][:, rest], clean[1][1][:, rest])
-    assert np.isnan(got[2][1].sum(0)[nan]).all() and not got[2][1][:, 20].any()
-    assert np.array_equal(got[2][1][:, rest], clean[2][1][:, rest])
+    X[21] = np.sign(X[21]) * np.finfo(np.float32).max
+    Y0[20], Y0[21] = 1e25, np.finfo(np.float32).max
+    nan, big, rest = [2, 17, 36], [20, 21], np.delete(np.arange(S), [2, 17, 20, 21, 36])
+    y, _, _ = _few(prec, STORE, W, scale, X, N, gain)
+    assert np.isnan(y[nan]).all() and not y[big].any() and np.array_equal(y[rest], clean[0][0][rest])
+    _, h, _ = _few(prec, SWIGLU, W, scale, X, N, gain)
+    assert np.isnan(h.sum(0)[nan]).all() and not h[:, big].any() and np.array_equal(h[:, rest], clean[2][1][:, rest])
+    X[big] = 0.0
+    y, p, ss = _few(prec, RESID, W, scale, X, N, gain, Y0, ng)
+    assert not np.isfinite(y[nan]).any() and not np.isfinite(ss[nan]).any()
+    assert np.array_equal(y[big], Y0[big]) and np.isinf(ss[big]).all() and np.isfinite(p[:, big]).all()
+    for got, want in zip((y, p.swapaxes(0, 1), ss), (clean[1][0], clean[1][1].swapaxes(0, 1), clean[1][2])):
+        assert np.array_equal(got[rest], want[rest])
