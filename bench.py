@@ -425,8 +425,8 @@ def main():
 def bench_batch(args):
     """Config 5: B concurrent 1.7B streams on one GPU, each stream's KV length drawn
     uniform in [lo, hi] from a seed (ragged), weights read once per step for all streams
-    (int8 / q4_0: MFMA over exact int8 activation pieces; bf16: MFMA over exact bf16
-    planes), attention over every stream's own cache.  A step = one batched step
+    (MFMA over exact bf16 activation planes; int8 past 16 and q4_0 past 32 streams of the
+    1.7B shape over exact int8 pieces), attention over every stream's own cache.  A step = one batched step
     of all B streams; value = ms per batched step (device-resident inputs, positions
     advancing on the device), tokens_per_s = B / step time.  The KV contents are zeros
     beyond what the steps write (attention reads every byte regardless of value)."""
@@ -674,7 +674,7 @@ def bench_frames(args):
         "frames_per_s": round(1000.0 / ms, 1), "frames_generated": len(codes), "eos": eos is not None,
         "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None,
-                     "kernel": "frame loop (head + k_sample + CP frame graph + k_frame_embed + k_pstep), whole call",
+                     "kernel": "frame loop (head + k_sample + CP frame + k_frame_embed + fused step), whole call",
                      "bytes_per_launch": int(frame_bytes * K), "avg_us": round(dt * 1e6, 1), "steps_per_launch": K},
         "cpu_baseline": None,
     }
@@ -927,7 +927,7 @@ def bench_cp_batch(args):
         "stream_passes_per_s": round(B * 1000.0 / ms, 1),
         "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None,
-                     "kernel": "batched CP pass (pieces + MFMA projections + batched attention, one hipGraph)",
+                     "kernel": "batched CP pass (MFMA projections + batched attention, one hipGraph)",
                      "bytes_per_launch": int(step_bytes), "avg_us": round(ms * 1e3, 1), "steps_per_launch": 1},
         "cpu_baseline": None,
     }

@@ -170,9 +170,10 @@ int   qwen_hip_talker_launch_kernel(void *state, int kernel, int layer, int n);
  * streams: every precision runs each projection as one GEMM over the B streams on the
  * matrix cores -- on the bf16 MFMA with exact bf16 activation planes; int8 and q4_0 past
  * qt_few_ok's stream counts on the integer MFMA with exact int8 activation pieces); each
- * stream has its
- * own bf16 KV cache (single state's kv_max) and its own position (ragged).  Free the
- * batch before the single state. */
+ * stream has its own bf16 KV cache (single state's kv_max) and its own position (ragged).
+ * A stream's result does not depend on the other streams or on its slot, but its bits depend
+ * on B: the projections' kernels and the attention's chunk length are chosen by the stream
+ * count.  Free the batch before the single state. */
 
 /* replaces qwen_cuda_talker_batch_init(single, B)      (qwen_tts_cuda_talker.cu:595) */
 void *qwen_hip_talker_batch_init(void *single, int B);
